@@ -189,10 +189,10 @@ struct Batch {
   std::vector<double*> tA, tB;
   std::vector<GemmTable> tpre;
   TripMol* dtm = nullptr;
-  long* dtprefix = nullptr;
+  int2* dtrange = nullptr;   // each molecule's work items [x, y)
   int2* dtri = nullptr;
   int* dtsave = nullptr;
-  double *dtw = nullptr, *dtpart = nullptr, *dtout = nullptr;
+  double *dtpart = nullptr, *dtout = nullptr;
   // linear response: concatenated trial/sigma vectors, amplitude backups, and
   // the per-molecule pointers (r1, r2, s1, s2; nm each) the sigma kernels read
   double *dlr_r1 = nullptr, *dlr_r2 = nullptr, *dlr_s1 = nullptr, *dlr_s2 = nullptr;
@@ -227,9 +227,8 @@ struct Batch {
   long *dlr_len = nullptr, *dlr_base = nullptr;
   char* dlr_stage = nullptr;   // job lists and results of the space calls
   size_t lr_stage_cap = 0;
-  long ttotal = 0, twstride = 0;
-  int tgrid = 0, tgrid_mfma = 0;
-  bool tglobal = false;
+  int tcount[3] = {0, 0, 0};   // work items per size class
+  int tcus = 1;
 
   // device memory: hipMalloc per buffer, or -- when `arena` is set (the
   // no-allocation entry point) -- consecutive 256-byte aligned pieces of a
@@ -1618,12 +1617,12 @@ static void setup_triples(Batch& b, int device) {
   const int nm = b.nm;
   b.tA.assign(nm, nullptr);
   b.tB.assign(nm, nullptr);
-  std::vector<long> prefix(nm + 1, 0);
+  size_t total = 0;
   for (int k = 0; k < nm; ++k) {
     const long o = b.o[k], v = b.v[k];
     b.tA[k] = b.dalloc<double>(o * v * v * v);
     b.tB[k] = b.dalloc<double>(o * o * o * v);
-    prefix[k + 1] = prefix[k] + o * (o + 1) * (o + 2) / 6;
+    total += o * (o + 1) * (o + 2) / 6;
   }
   b.tpre.clear();
   // (xp|yd) at [p][x][y][d]: rows (p, x) of P, columns (y, d) of Q = gamma P (undressed)
@@ -1640,42 +1639,39 @@ static void setup_triples(Batch& b, int device) {
     return prob(cmp(M.P, o, N, 1, 1, N2, 0), cmp(M.Q + o, 1, N2, 0, v, N, 1), rm(b.tB[k], o * v), o * o, o * v, N,
                 1.0, 0.0);
   }));
-  // work items: molecule and occupied triple i >= j >= k (i ascending)
-  std::vector<int2> items;
-  items.reserve(prefix[nm]);
-  for (int m = 0; m < nm; ++m)
+  // work items: molecule and occupied triple i >= j >= k, by size class and
+  // within a class the larger molecules first, so that what runs last is short
+  std::vector<int> order(nm);
+  for (int k = 0; k < nm; ++k) order[k] = k;
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+    const int cx = trip_class(b.v[x]), cy = trip_class(b.v[y]);
+    return cx != cy ? cx < cy : b.v[x] > b.v[y];
+  });
+  std::vector<int2> items, range(nm);
+  items.reserve(total);
+  b.tcount[0] = b.tcount[1] = b.tcount[2] = 0;
+  for (int m : order) {
+    range[m].x = (int)items.size();
     for (int i = 0; i < b.o[m]; ++i)
       for (int j = 0; j <= i; ++j)
         for (int k = 0; k <= j; ++k) items.push_back(int2{m, i | (j << 8) | (k << 16)});
+    range[m].y = (int)items.size();
+    b.tcount[trip_class(b.v[m])] += range[m].y - range[m].x;
+  }
   std::vector<TripMol> tm(nm);
   for (int k = 0; k < nm; ++k) {
     const Mol& M = b.hm[k];
     tm[k] = TripMol{M.n, M.o, M.v, 0, b.tA[k], b.tB[k], M.Gklcd, M.t1, M.t2, M.F};
   }
-  b.ttotal = prefix[nm];
-  // molecules with v <= kTripLdsV go to the matrix-core kernel (W in LDS, one
-  // workgroup per CU); the others keep W in a global block per workgroup
-  int vglob = 0;
-  bool small = false;
-  for (int k = 0; k < nm; ++k) {
-    if (b.v[k] > kTripLdsV) vglob = std::max(vglob, b.v[k]);
-    else small = true;
-  }
-  b.tglobal = vglob > 0;
-  int cus = 0;
-  HCHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
-  b.tgrid_mfma = small ? std::max(1, cus) : 0;
-  b.twstride = ((long)vglob * vglob * vglob + 31) / 32 * 32;
-  b.tgrid = b.tglobal ? (int)std::max<long>(1, std::min<long>(b.ttotal, 1024)) : 1;
+  HCHECK(hipDeviceGetAttribute(&b.tcus, hipDeviceAttributeMultiprocessorCount, device));
   b.dtm = b.dalloc<TripMol>(nm);
-  b.dtprefix = b.dalloc<long>(nm + 1);
+  b.dtrange = b.dalloc<int2>(nm);
   b.dtri = b.dalloc<int2>(items.size());
-  b.dtw = b.dalloc<double>((size_t)b.tgrid * b.twstride);
-  b.dtpart = b.dalloc<double>(2 * std::max<long>(1, b.ttotal));
+  b.dtpart = b.dalloc<double>(2 * items.size());
   b.dtout = b.dalloc<double>(2 * (long)nm);
   b.dtsave = b.dalloc<int>(nm);
   HCHECK(hipMemcpy(b.dtm, tm.data(), nm * sizeof(TripMol), hipMemcpyHostToDevice));
-  HCHECK(hipMemcpy(b.dtprefix, prefix.data(), (nm + 1) * sizeof(long), hipMemcpyHostToDevice));
+  HCHECK(hipMemcpy(b.dtrange, range.data(), nm * sizeof(int2), hipMemcpyHostToDevice));
   HCHECK(hipMemcpy(b.dtri, items.data(), items.size() * sizeof(int2), hipMemcpyHostToDevice));
 }
 
@@ -1715,8 +1711,7 @@ int hcc_batch_triples(hcc_ctx* ctx, double* energies, double* e_t) {
   HCHECK(hipMemcpyAsync(first.t1, first.w1, span * sizeof(double), hipMemcpyDeviceToDevice, s));
   prof_close(ctx);
   prof_open(ctx, kProfTriples);
-  HCHECK(launch_triples(b.dtm, b.nm, b.dtprefix, b.ttotal, b.dtri, b.dtw, b.twstride, b.tgrid, b.tgrid_mfma, b.tglobal,
-                        b.dtpart, b.dtout, s));
+  HCHECK(launch_triples(b.dtm, b.nm, b.dtrange, b.dtri, b.tcount, b.tcus, b.dtpart, b.dtout, s));
   prof_close(ctx);
   prof_open(ctx, kProfTriplesEw);
   arm_all(b.dst, b.dact, b.dtsave, b.nm, true, s);

@@ -17,19 +17,14 @@ struct TripMol {
 };
 
 constexpr int kTripMaxOV = 32;   // o, v <= 32
-constexpr int kTripLdsV = 24;    // v <= 24: matrix-core kernel with W in LDS (else W in global memory)
 
-size_t triples_lds_bytes();
-size_t triples_mfma_lds_bytes();
-// prefix: nm + 1 item offsets; items: per work item (molecule, occupied
-// triple i >= j >= k packed as i | j << 8 | k << 16), a molecule's items
-// consecutive from prefix[m]; wscratch:
-// grid blocks of wstride >= v^3 doubles (v > kTripLdsV); grid_mfma: workgroups
-// of the matrix-core kernel (0: no molecule with v <= kTripLdsV); any_global:
-// some molecule has v > kTripLdsV; part: 2 per item; out: 2 per molecule
-// (E[T], E[ST])
-hipError_t launch_triples(const TripMol* mols, int nm, const long* prefix, long total, const int2* items,
-                          double* wscratch, long wstride, int grid, int grid_mfma, bool any_global, double* part,
-                          double* out, hipStream_t s);
+// Size classes of the work items, a kernel each: v <= 16, v <= 24 and v <= 32.
+int trip_class(int v);
+// items: per work item (molecule, occupied triple i >= j >= k packed as
+// i | j << 8 | k << 16), the items of class 0 first, then 1, then 2 (count[3]
+// of each), a molecule's items consecutive: [range.x, range.y); cus: compute
+// units of the device; part: 2 per item; out: 2 per molecule (E[T], E[ST])
+hipError_t launch_triples(const TripMol* mols, int nm, const int2* range, const int2* items, const int* count, int cus,
+                          double* part, double* out, hipStream_t s);
 
 }  // namespace hcc

@@ -4,8 +4,8 @@ import numpy as np
 import pytest
 
 from helios_amd import capi, molecules as M
-from oracle import ccsd
-from tests._molprep import prepare
+from oracle import ccsd, triples as T
+from tests._molprep import prepare, random_amplitudes
 
 pytestmark = pytest.mark.gpu
 
@@ -45,3 +45,26 @@ def test_diis_system_sizes(steps):
     assert st == 1
     assert abs(e[0] - ref["energy"][0]) < 1e-8
     assert np.abs(t2 - ref["t2"]).max() < 1e-7
+
+
+@pytest.mark.parametrize("o,v", [(3, 2), (5, 15), (2, 16), (9, 17), (17, 9), (4, 23), (3, 24), (5, 25), (25, 26),
+                                 (6, 31), (31, 32)])
+def test_triples_size_classes(o, v):
+    """(T) at given amplitudes on both sides of the size classes' limits (v = 16,
+    24, 32; ragged row tiles, a second virtual block of 9 to 16), with the
+    tolerance of the kernel parity test: 1e-11 of |E[T]|."""
+    p = prepare(M.random_fragment(o + v + (o + v) % 2, seed=11))
+    n = o + v
+    C, F, G = p["C"][:, :n], p["F"][:n, :n], p["G"]
+    if n < p["n"]:   # an odd count: leave the last site and orbital out
+        C, G = C[:n], G[:n, :n]
+    t1, t2 = random_amplitudes(o, v, 100 * o + v, 0.05, 0.05)
+    ctx = capi.Context(0, capi.HCC_FP64, 20)
+    ctx.set_molecule(C, F, G, o, p["eref"])
+    ctx.set_amplitudes(t1, t2)
+    _, et = ctx.batch_triples()
+    ctx.close()
+    ref = T.closed_shell_sliced(C, F, G, o, t1, t2)
+    print(o, v, et[0], ref, et[0] - ref)
+    assert abs(et[0, 0] - ref[0]) < 1e-11 * abs(ref[0])
+    assert abs(et[0, 1] - ref[1]) < 1e-11 * abs(ref[0])
