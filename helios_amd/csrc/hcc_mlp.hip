@@ -16,11 +16,11 @@
 // LDS round trip is needed between layers.  Weights and layer inputs are
 // BF16, accumulation FP32; biases, GELU and the output layer are FP32.
 //
-// Training (GPU, deterministic): a forward kernel (same device function)
-// stores the activations of a mini-batch, a per-sample backward kernel forms
-// dz2 and dz1 in FP32, a weight-gradient kernel sums per-parameter over
-// sample chunks, and one kernel reduces the chunks in a fixed order and
-// applies Adam.  No atomics anywhere: results are bitwise reproducible.
+// Training (GPU, deterministic): one kernel per mini-batch takes every wave's
+// samples forward (same device function), backward and into weight-gradient
+// sums on the matrix cores, 16 samples at a time; a second kernel reduces the
+// workgroups' sums in a fixed order and applies Adam.  No atomics anywhere:
+// results are bitwise reproducible.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -36,13 +36,13 @@ namespace hcc {
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
-constexpr int kAct = 272;   // stored activations per sample: z1, h1r, z2, h2 (64 each), x (16)
-constexpr int kActZ1 = 0, kActH1 = 64, kActZ2 = 128, kActH2 = 192, kActX = 256;
-
 __device__ __forceinline__ float bfr(float x) { return (float)(__bf16)x; }
 __device__ __forceinline__ float gelu(float z) { return 0.5f * z * (1.f + erff(z * 0.70710678118654752f)); }
-__device__ __forceinline__ float gelu_prime(float z) {
-  return 0.5f * (1.f + erff(z * 0.70710678118654752f)) + z * expf(-0.5f * z * z) * 0.39894228040143268f;
+// gelu(z) and its derivative, which share the error function
+__device__ __forceinline__ float gelu_both(float z, float& prime) {
+  const float e = 1.f + erff(z * 0.70710678118654752f);
+  prime = 0.5f * e + z * expf(-0.5f * z * z) * 0.39894228040143268f;
+  return 0.5f * z * e;
 }
 
 // ---------------------------------------------------------------------------
@@ -137,8 +137,10 @@ __device__ void net_load(Net& N, const float* __restrict__ w, int lane) {
   N.b3 = w[kOffB3];
 }
 
+// what the backward pass needs of this lane's units: gelu' at z1 and z2, the
+// rounded first hidden layer and the second
 struct Acts {
-  float z1[16], h1r[16], z2[16], h2[16];
+  float d1[16], h1r[16], d2[16], h2[16];
 };
 
 // Forward pass of the wave's 16 samples; x holds features 8g..8g+7 of sample
@@ -155,12 +157,9 @@ __device__ float net_forward(const Net& N, const bf8 x, Acts& A) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const float z = c1[mb][r] + N.b1[4 * mb + r];
-      const float h = gelu(z);
+      const float h = STORE ? gelu_both(z, A.d1[4 * mb + r]) : gelu(z);
       hb[mb >> 1][4 * (mb & 1) + r] = (__bf16)h;
-      if (STORE) {
-        A.z1[4 * mb + r] = z;
-        A.h1r[4 * mb + r] = bfr(h);
-      }
+      if (STORE) A.h1r[4 * mb + r] = bfr(h);
     }
   f4 c2[4];
 #pragma unroll
@@ -174,12 +173,9 @@ __device__ float net_forward(const Net& N, const bf8 x, Acts& A) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const float z = c2[mb][r] + N.b2[4 * mb + r];
-      const float h = gelu(z);
+      const float h = STORE ? gelu_both(z, A.d2[4 * mb + r]) : gelu(z);
       p += N.w3[4 * mb + r] * h;
-      if (STORE) {
-        A.z2[4 * mb + r] = z;
-        A.h2[4 * mb + r] = h;
-      }
+      if (STORE) A.h2[4 * mb + r] = h;
     }
   p += __shfl_xor(p, 16);
   p += __shfl_xor(p, 32);
@@ -396,15 +392,11 @@ __global__ __launch_bounds__(256) void k_mlp_collect(const Mol* __restrict__ mol
   r[kMlpF + 1] = 1.f;
 }
 
-// Forward over a mini-batch: sample sb of the batch is row (base + sb) * A + C
-// mod ns (a permutation of the rows for gcd(A, ns) = 1).  STORE: keep the
-// activations and dL/dy for the backward pass.  Per-workgroup loss sums
-// (fixed order) go to lossp[blockIdx.x].
-template <bool STORE>
+// Forward over rows base .. base + nb - 1: per-workgroup loss sums (fixed
+// order) to lossp[blockIdx.x], outputs to yout unless null.
 __global__ __launch_bounds__(256) void k_mlp_forward(const float* __restrict__ w, const float* __restrict__ rows,
-                                                     long ns, long pa, long pc, long base, int nb,
-                                                     float* __restrict__ act, float* __restrict__ dy,
-                                                     double* __restrict__ lossp, float* __restrict__ yout) {
+                                                     long base, int nb, double* __restrict__ lossp,
+                                                     float* __restrict__ yout) {
   __shared__ double sl[256];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
   Net net;
@@ -413,34 +405,16 @@ __global__ __launch_bounds__(256) void k_mlp_forward(const float* __restrict__ w
     const int loc = wave * 64 + grp * 16 + n;
     const int sb = blockIdx.x * 256 + loc;
     const bool ok = sb < nb;
-    const long row = ok ? ((base + sb) * pa + pc) % ns : 0;
-    const float* R = rows + row * kMlpRow;
+    const float* R = rows + (ok ? base + sb : 0) * kMlpRow;
     float f[kMlpF];
 #pragma unroll
     for (int q = 0; q < kMlpF; ++q) f[q] = ok ? R[q] : 0.f;
     Acts A;
-    const float y = net_forward<STORE>(net, pack_x(f, g), A);
+    const float y = net_forward<false>(net, pack_x(f, g), A);
     const float tg = ok ? R[kMlpF] : 0.f, wt = ok ? R[kMlpF + 1] : 0.f;
     const float d = y - tg;
     if (g == 0) sl[loc] = ok ? (double)(wt * d * d) : 0.0;
     if (yout != nullptr && ok && g == 0) yout[sb] = y;
-    if (STORE && ok) {
-      float* P = act + (long)sb * kAct;
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int u = 16 * mb + 4 * g + r;
-          P[kActZ1 + u] = A.z1[4 * mb + r];
-          P[kActH1 + u] = A.h1r[4 * mb + r];
-          P[kActZ2 + u] = A.z2[4 * mb + r];
-          P[kActH2 + u] = A.h2[4 * mb + r];
-        }
-      if (g < 2)
-#pragma unroll
-        for (int q = 0; q < 8; ++q) P[kActX + 8 * g + q] = bfr(g == 0 ? f[q] : f[8 + q]);
-      if (g == 0) dy[sb] = 2.f * wt * d / (float)nb;
-    }
   }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -450,71 +424,185 @@ __global__ __launch_bounds__(256) void k_mlp_forward(const float* __restrict__ w
   }
 }
 
-// per-sample backward: dz2 = dy w3 gelu'(z2), dz1 = (W2^T dz2) gelu'(z1)
-__global__ __launch_bounds__(256) void k_mlp_backward(const float* __restrict__ w, int nb,
-                                                      const float* __restrict__ act, const float* __restrict__ dy,
-                                                      float* __restrict__ gact) {
-  __shared__ float W2s[kMlpH * kMlpH];
-  __shared__ float w3s[kMlpH];
-  for (int q = threadIdx.x; q < kMlpH * kMlpH; q += 256) W2s[q] = bfr(w[kOffW2 + q]);
-  if (threadIdx.x < kMlpH) w3s[threadIdx.x] = bfr(w[kOffW3 + threadIdx.x]);
+// Loss and weight gradient of a mini-batch: sample sb is row
+// ((base + sb) pa + pc) mod ns (a permutation of the rows for gcd(pa, ns) = 1).
+// A workgroup takes `per_block` samples (64 or 256) and writes their loss and
+// its gradient sums, part[blockIdx.x][kMlpParams]; samples past nb add zero.
+//
+// Everything between the rows and the sums stays in registers and LDS, 16
+// samples of a wave at a time:
+//  * forward as in the guess (BF16 operands, FP32 accumulation);
+//  * dz2 = dy w3 gelu'(z2) on the lane that holds the unit, dz1 = (W2^T dz2)
+//    gelu'(z1) with V_MFMA_F32_16X16X4F32: the K step (mb, r) takes units
+//    16 mb + 4 g + r of the four lane groups, which is what they hold, so dz2
+//    is the B operand as it stands;
+//  * dW2 += dz2 h1^T and dW1 += dz1 x^T with the samples along K (FP32
+//    products and sums, 80 accumulators a lane), from an LDS transpose with a
+//    row pitch of 80 floats (reads and 16-byte writes without bank conflicts);
+//    the biases and dW3 are summed per lane.
+// Bound by the GELU arithmetic and this chain's latency: one wave per SIMD,
+// for the accumulators and the network's operands take over 256 registers.
+// The separate forward, backward and per-parameter gradient kernels, with 400
+// activations a sample through memory, took 420 us for 65000 rows; this one
+// takes 59 (477 -> 97 us for the whole call, 195 -> 63 us for a few thousand rows).
+constexpr int kGradThreads = 256;
+constexpr int kGradLd = 80;
+constexpr int kGradW2Ld = 68;
+constexpr int kGradWave = 16 * (3 * kGradLd + 16);   // floats of a wave: dz2, h1, dz1 [n][80], x [n][16]
+constexpr int kGradLds = 4 * kGradWave + kMlpH * kGradW2Ld > 4 * kOffB3 ? 4 * kGradWave + kMlpH * kGradW2Ld : 4 * kOffB3;
+__global__ __launch_bounds__(kGradThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_mlp_gradient(
+    const float* __restrict__ w, const float* __restrict__ rows, long ns, long pa, long pc, long base, int nb,
+    int per_block, double* __restrict__ lossp, float* __restrict__ part) {
+  __shared__ __attribute__((aligned(16))) float lds[kGradLds];
+  __shared__ double sl[kGradThreads];
+  __shared__ float sb3[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
+  float* const D2 = lds + wave * kGradWave;
+  float* const H1 = D2 + 16 * kGradLd;
+  float* const D1 = H1 + 16 * kGradLd;
+  float* const Xs = D1 + 16 * kGradLd;
+  float* const W2s = lds + 4 * kGradWave;   // W2[k][j], rounded
+  for (int q = threadIdx.x; q < kMlpH * kMlpH; q += kGradThreads) W2s[(q >> 6) * kGradW2Ld + (q & 63)] = bfr(w[kOffW2 + q]);
+  Net net;
+  net_load(net, w, lane);
+  f4 gw2[4][4], gw1[4];
+  float gb1[16], gb2[16], gw3[16], gb3 = 0.f;
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    gw1[a] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = 0; b < 4; ++b) gw2[a][b] = f4{0.f, 0.f, 0.f, 0.f};
+  }
+#pragma unroll
+  for (int u = 0; u < 16; ++u) gb1[u] = gb2[u] = gw3[u] = 0.f;
+  double loss = 0.0;
+  const int passes = per_block / 64;
+  for (int pass = 0; pass < passes; ++pass) {
+    const int sb = blockIdx.x * per_block + (wave * passes + pass) * 16 + n;
+    const bool ok = sb < nb;
+    const float* R = rows + (ok ? ((base + sb) * pa + pc) % ns : 0) * kMlpRow;
+    float f[kMlpF];
+#pragma unroll
+    for (int q = 0; q < kMlpF; ++q) f[q] = ok ? R[q] : 0.f;
+    const float tg = ok ? R[kMlpF] : 0.f, wt = ok ? R[kMlpF + 1] : 0.f;
+    Acts A;
+    const float y = net_forward<true>(net, pack_x(f, g), A);
+    const float d = y - tg, dy = ok ? 2.f * wt * d / (float)nb : 0.f;
+    if (g == 0) loss += ok ? (double)(wt * d * d) : 0.0;
+    float dz2[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      dz2[u] = dy * net.w3[u] * A.d2[u];
+      gb2[u] += dz2[u];
+      gw3[u] += dy * A.h2[u];
+    }
+    gb3 += dy;
+    __syncthreads();   // the previous pass has read the tiles (first pass: W2s is written)
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb) {
+      *reinterpret_cast<f4*>(&D2[n * kGradLd + 16 * mb + 4 * g]) = f4{dz2[4 * mb], dz2[4 * mb + 1], dz2[4 * mb + 2], dz2[4 * mb + 3]};
+      *reinterpret_cast<f4*>(&H1[n * kGradLd + 16 * mb + 4 * g]) = f4{A.h1r[4 * mb], A.h1r[4 * mb + 1], A.h1r[4 * mb + 2], A.h1r[4 * mb + 3]};
+    }
+    if (g < 2)
+#pragma unroll
+      for (int q = 0; q < 8; ++q) Xs[n * 16 + 8 * g + q] = bfr(g == 0 ? f[q] : f[8 + q]);
+    f4 c[4];
+#pragma unroll
+    for (int jb = 0; jb < 4; ++jb) c[jb] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int jb = 0; jb < 4; ++jb)
+          c[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(W2s[(16 * mb + 4 * g + r) * kGradW2Ld + 16 * jb + n],
+                                                       dz2[4 * mb + r], c[jb], 0, 0, 0);
+#pragma unroll
+    for (int jb = 0; jb < 4; ++jb) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        c[jb][r] *= A.d1[4 * jb + r];
+        gb1[4 * jb + r] += c[jb][r];
+      }
+      *reinterpret_cast<f4*>(&D1[n * kGradLd + 16 * jb + 4 * g]) = c[jb];
+    }
+    __syncthreads();
+    // samples 4 s + g along K: rows are the units of a block, columns those of the layer below
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const float* const d2 = D2 + (4 * s + g) * kGradLd + n;
+      const float* const h1 = H1 + (4 * s + g) * kGradLd + n;
+      const float* const d1 = D1 + (4 * s + g) * kGradLd + n;
+      const float x = Xs[(4 * s + g) * 16 + n];
+      float hk[4];
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) hk[kb] = h1[16 * kb];
+#pragma unroll
+      for (int mb = 0; mb < 4; ++mb) {
+        const float a = d2[16 * mb];
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) gw2[mb][kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, hk[kb], gw2[mb][kb], 0, 0, 0);
+        gw1[mb] = __builtin_amdgcn_mfma_f32_16x16x4f32(d1[16 * mb], x, gw1[mb], 0, 0, 0);
+      }
+    }
+  }
+  // the lanes of a group hold the same units: sums over their samples
+#pragma unroll
+  for (int off = 1; off < 16; off <<= 1) {
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      gb1[u] += __shfl_xor(gb1[u], off);
+      gb2[u] += __shfl_xor(gb2[u], off);
+      gw3[u] += __shfl_xor(gw3[u], off);
+    }
+    gb3 += __shfl_xor(gb3, off);
+  }
+  sl[threadIdx.x] = loss;
   __syncthreads();
-  const int sb = blockIdx.x * 256 + threadIdx.x;
-  if (sb >= nb) return;
-  const float* P = act + (long)sb * kAct;
-  float* G = gact + (long)sb * 2 * kMlpH;
-  const float d = dy[sb];
-  float dz2[kMlpH];
+  float* const S = lds + wave * kOffB3;   // this wave's sums in parameter order
 #pragma unroll
-  for (int k = 0; k < kMlpH; ++k) {
-    dz2[k] = d * w3s[k] * gelu_prime(P[kActZ2 + k]);
-    G[kMlpH + k] = dz2[k];
-  }
-  for (int j = 0; j < kMlpH; ++j) {
-    float s = 0.f;
+  for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
-    for (int k = 0; k < kMlpH; ++k) s += W2s[k * kMlpH + j] * dz2[k];
-    G[j] = s * gelu_prime(P[kActZ1 + j]);
+    for (int r = 0; r < 4; ++r) {
+      const int m = 16 * mb + 4 * g + r;
+      S[kOffW1 + m * kMlpF + n] = gw1[mb][r];
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) S[kOffW2 + m * kMlpH + 16 * kb + n] = gw2[mb][kb][r];
+      if (n == 0) {
+        S[kOffB1 + m] = gb1[4 * mb + r];
+        S[kOffB2 + m] = gb2[4 * mb + r];
+        S[kOffW3 + m] = gw3[4 * mb + r];
+      }
+    }
+  if (lane == 0) sb3[wave] = gb3;
+  __syncthreads();
+  float* const P = part + (long)blockIdx.x * kMlpParams;
+  for (int q = threadIdx.x; q < kOffB3; q += kGradThreads)
+    P[q] = lds[q] + lds[kOffB3 + q] + lds[2 * kOffB3 + q] + lds[3 * kOffB3 + q];
+  if (threadIdx.x == 0) {
+    P[kOffB3] = sb3[0] + sb3[1] + sb3[2] + sb3[3];
+    double s = 0.0;
+    for (int k = 0; k < 4; ++k)
+      for (int q = 0; q < 16; ++q) s += sl[64 * k + q];
+    lossp[blockIdx.x] = s;
   }
 }
 
-// per-parameter gradient sums over one chunk of the mini-batch
-__global__ __launch_bounds__(256) void k_mlp_wgrad(int nb, int chunk, const float* __restrict__ act,
-                                                   const float* __restrict__ gact, const float* __restrict__ dy,
-                                                   float* __restrict__ part) {
-  const int p = blockIdx.y * 256 + threadIdx.x;
-  if (p >= kMlpParams) return;
-  const int n0 = blockIdx.x * chunk, n1 = min(nb, n0 + chunk);
-  float s = 0.f;
-  if (p < kOffB1) {
-    const int m = p / kMlpF, f = p % kMlpF;
-    for (int n = n0; n < n1; ++n) s += gact[(long)n * 128 + m] * act[(long)n * kAct + kActX + f];
-  } else if (p < kOffW2) {
-    const int m = p - kOffB1;
-    for (int n = n0; n < n1; ++n) s += gact[(long)n * 128 + m];
-  } else if (p < kOffB2) {
-    const int m = (p - kOffW2) / kMlpH, k = (p - kOffW2) % kMlpH;
-    for (int n = n0; n < n1; ++n) s += gact[(long)n * 128 + kMlpH + m] * act[(long)n * kAct + kActH1 + k];
-  } else if (p < kOffW3) {
-    const int m = p - kOffB2;
-    for (int n = n0; n < n1; ++n) s += gact[(long)n * 128 + kMlpH + m];
-  } else if (p < kOffB3) {
-    const int k = p - kOffW3;
-    for (int n = n0; n < n1; ++n) s += dy[n] * act[(long)n * kAct + kActH2 + k];
-  } else {
-    for (int n = n0; n < n1; ++n) s += dy[n];
-  }
-  part[(long)blockIdx.x * kMlpParams + p] = s;
-}
-
-// fixed-order reduction of the chunk sums, then (update) one Adam step
+// fixed-order reduction of the workgroups' sums (8 threads per parameter, 32
+// consecutive parameters of a sum row per load), then (update) one Adam step
 __global__ __launch_bounds__(256) void k_mlp_adam(float* __restrict__ w, float* __restrict__ m1, float* __restrict__ m2,
                                                   float* __restrict__ grad, const float* __restrict__ part, int nchunk,
                                                   float lr, float bc1, float bc2, int update) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p >= kMlpParams) return;
+  __shared__ float red[8][32];
+  const int p = blockIdx.x * 32 + (threadIdx.x & 31), grp = threadIdx.x >> 5;
   float g = 0.f;
-  for (int c = 0; c < nchunk; ++c) g += part[(long)c * kMlpParams + p];
+  if (p < kMlpParams)
+#pragma unroll 8
+    for (int c = grp; c < nchunk; c += 8) g += part[(long)c * kMlpParams + p];
+  red[grp][threadIdx.x & 31] = g;
+  __syncthreads();
+  if (grp != 0 || p >= kMlpParams) return;
+  for (int c = 1; c < 8; ++c) g += red[c][threadIdx.x];
   grad[p] = g;
   if (!update) return;
   const float a = 0.9f * m1[p] + 0.1f * g;
@@ -538,9 +626,9 @@ struct hcc_mlp {
   float* rows = nullptr;
   int* where = nullptr;
   long cap = 0, count = 0;
-  // mini-batch buffers (grown on demand)
-  int bcap = 0;
-  float *act = nullptr, *gact = nullptr, *dy = nullptr, *part = nullptr, *yout = nullptr;
+  // mini-batch buffers (grown on demand): gradient sums per workgroup, loss sums
+  int pcap = 0;
+  float* part = nullptr;
   double* lossp = nullptr;
   long lcap = 0;
   long step = 0;
@@ -549,8 +637,6 @@ struct hcc_mlp {
 
 namespace {
 
-constexpr int kChunk = 256;   // samples per weight-gradient chunk
-
 template <class T>
 void dalloc(T** p, size_t count) {
   if (*p) HCHECK(hipFree(*p));
@@ -558,15 +644,15 @@ void dalloc(T** p, size_t count) {
   HCHECK(hipMalloc((void**)p, std::max<size_t>(1, count) * sizeof(T)));
 }
 
-void ensure_batch(hcc_mlp* net, int nb) {
-  if (nb <= net->bcap) return;
-  const int cap = std::max(nb, 256);
-  dalloc(&net->act, (size_t)cap * kAct);
-  dalloc(&net->gact, (size_t)cap * 2 * kMlpH);
-  dalloc(&net->dy, (size_t)cap);
-  dalloc(&net->yout, (size_t)cap);
-  dalloc(&net->part, (size_t)((cap + kChunk - 1) / kChunk) * kMlpParams);
-  net->bcap = cap;
+// Samples per workgroup of the gradient kernel: 64 (16 per wave) keep up to
+// 256 CUs busy on mini-batches; beyond 16384 samples 256 bound the number of
+// gradient sums to reduce (65000 samples: 1016 sums of 21 KB instead of 254).
+int samples_per_block(long nb) { return nb <= 16384 ? 64 : 256; }
+
+void ensure_part(hcc_mlp* net, int blocks) {
+  if (blocks <= net->pcap) return;
+  dalloc(&net->part, (size_t)blocks * kMlpParams);
+  net->pcap = blocks;
 }
 
 void ensure_loss(hcc_mlp* net, long blocks) {
@@ -575,24 +661,21 @@ void ensure_loss(hcc_mlp* net, long blocks) {
   net->lcap = blocks;
 }
 
-// one mini-batch: forward (stored), backward, gradient; update = Adam step
-void batch_step(hcc_mlp* net, long ns, long pa, long pc, long base, int nb, double* lossp, bool update, float lr) {
+// one mini-batch of nb samples on `blocks` workgroups (those past nb add
+// zero): loss and gradient; update = Adam step
+void batch_step(hcc_mlp* net, long ns, long pa, long pc, long base, int nb, int blocks, int per_block, double* lossp,
+                bool update, float lr) {
   hipStream_t s = net->stream;
-  const int blocks = (nb + 255) / 256;
-  hipLaunchKernelGGL(k_mlp_forward<true>, dim3(blocks), dim3(256), 0, s, net->w, net->rows, ns, pa, pc, base, nb,
-                     net->act, net->dy, lossp, (float*)nullptr);
-  hipLaunchKernelGGL(k_mlp_backward, dim3(blocks), dim3(256), 0, s, net->w, nb, net->act, net->dy, net->gact);
-  const int nchunk = (nb + kChunk - 1) / kChunk;
-  hipLaunchKernelGGL(k_mlp_wgrad, dim3(nchunk, (kMlpParams + 255) / 256), dim3(256), 0, s, nb, kChunk, net->act,
-                     net->gact, net->dy, net->part);
+  hipLaunchKernelGGL(k_mlp_gradient, dim3(blocks), dim3(kGradThreads), 0, s, net->w, net->rows, ns, pa, pc, base, nb,
+                     per_block, lossp, net->part);
   float bc1 = 1.f, bc2 = 1.f;
   if (update) {
     net->step += 1;
     bc1 = (float)(1.0 - std::pow(0.9, (double)net->step));
     bc2 = (float)(1.0 - std::pow(0.999, (double)net->step));
   }
-  hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 255) / 256), dim3(256), 0, s, net->w, net->m1, net->m2,
-                     net->grad, net->part, nchunk, lr, bc1, bc2, update ? 1 : 0);
+  hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 31) / 32), dim3(256), 0, s, net->w, net->m1, net->m2,
+                     net->grad, net->part, blocks, lr, bc1, bc2, update ? 1 : 0);
   HCHECK(hipGetLastError());
 }
 
@@ -661,8 +744,7 @@ void hcc_mlp_destroy(hcc_mlp* net) {
   if (net == nullptr) return;
   (void)hipSetDevice(net->device);
   for (void* p : {(void*)net->w, (void*)net->m1, (void*)net->m2, (void*)net->grad, (void*)net->rows,
-                  (void*)net->where, (void*)net->act, (void*)net->gact, (void*)net->dy, (void*)net->part,
-                  (void*)net->yout, (void*)net->lossp})
+                  (void*)net->where, (void*)net->part, (void*)net->lossp})
     if (p) (void)hipFree(p);
   if (net->stream) (void)hipStreamDestroy(net->stream);
   delete net;
@@ -757,10 +839,10 @@ int hcc_mlp_write_samples(hcc_mlp* net, const float* rows, long count) {
 int hcc_mlp_gradient(hcc_mlp* net, long first, int count, double* loss, float* grad) {
   if (net == nullptr || first < 0 || count < 1 || first + count > net->count) return HCC_E_ARG;
   MLP_BEGIN
-  ensure_batch(net, count);
-  const int blocks = (count + 255) / 256;
+  const int per = samples_per_block(count), blocks = (count + per - 1) / per;
+  ensure_part(net, blocks);
   ensure_loss(net, blocks);
-  batch_step(net, net->count, 1, 0, first, count, net->lossp, false, 0.f);
+  batch_step(net, net->count, 1, 0, first, count, blocks, per, net->lossp, false, 0.f);
   std::vector<double> lp(blocks);
   HCHECK(hipMemcpyAsync(lp.data(), net->lossp, blocks * sizeof(double), hipMemcpyDeviceToHost, net->stream));
   if (grad) HCHECK(hipMemcpyAsync(grad, net->grad, kMlpParams * sizeof(float), hipMemcpyDeviceToHost, net->stream));
@@ -779,8 +861,8 @@ int hcc_mlp_train(hcc_mlp* net, int epochs, int batch, float lr, float lr_final,
   const long ns = net->count;
   const int nb = (int)std::min<long>(batch, ns);
   const long steps = (ns + nb - 1) / nb;
-  const int bpb = (nb + 255) / 256;
-  ensure_batch(net, nb);
+  const int per = samples_per_block(nb), bpb = (nb + per - 1) / per;
+  ensure_part(net, bpb);
   ensure_loss(net, steps * bpb);
   const long total = steps * (long)epochs;
   std::vector<double> lp((size_t)steps * bpb);
@@ -797,7 +879,7 @@ int hcc_mlp_train(hcc_mlp* net, int epochs, int batch, float lr, float lr_final,
       const int cnt = (int)std::min<long>(nb, ns - base);
       const double frac = (double)(ep * steps + k) / (double)std::max<long>(1, total - 1);
       const float lrk = (float)(lr_final + 0.5 * (lr - lr_final) * (1.0 + std::cos(3.14159265358979 * frac)));
-      batch_step(net, ns, pa, pc, base, cnt, net->lossp + k * bpb, true, lrk);
+      batch_step(net, ns, pa, pc, base, cnt, bpb, per, net->lossp + k * bpb, true, lrk);
     }
     HCHECK(hipMemcpyAsync(lp.data(), net->lossp, lp.size() * sizeof(double), hipMemcpyDeviceToHost, net->stream));
     HCHECK(hipStreamSynchronize(net->stream));
@@ -816,8 +898,8 @@ int hcc_mlp_evaluate(hcc_mlp* net, double* loss) {
   const long ns = net->count;
   const long blocks = (ns + 255) / 256;
   ensure_loss(net, blocks);
-  hipLaunchKernelGGL(k_mlp_forward<false>, dim3((unsigned)blocks), dim3(256), 0, net->stream, net->w, net->rows, ns,
-                     1L, 0L, 0L, (int)ns, (float*)nullptr, (float*)nullptr, net->lossp, (float*)nullptr);
+  hipLaunchKernelGGL(k_mlp_forward, dim3((unsigned)blocks), dim3(256), 0, net->stream, net->w, net->rows, 0L, (int)ns,
+                     net->lossp, (float*)nullptr);
   HCHECK(hipGetLastError());
   std::vector<double> lp(blocks);
   HCHECK(hipMemcpyAsync(lp.data(), net->lossp, blocks * sizeof(double), hipMemcpyDeviceToHost, net->stream));
@@ -840,8 +922,8 @@ int hcc_mlp_predict(hcc_mlp* net, const float* features, long count, float* y) {
   const long blocks = (count + 255) / 256;
   double* lp = nullptr;
   dalloc(&lp, (size_t)blocks);
-  hipLaunchKernelGGL(k_mlp_forward<false>, dim3((unsigned)blocks), dim3(256), 0, net->stream, net->w, rows, count,
-                     1L, 0L, 0L, (int)count, (float*)nullptr, (float*)nullptr, lp, yd);
+  hipLaunchKernelGGL(k_mlp_forward, dim3((unsigned)blocks), dim3(256), 0, net->stream, net->w, rows, 0L, (int)count,
+                     lp, yd);
   HCHECK(hipGetLastError());
   HCHECK(hipStreamSynchronize(net->stream));
   HCHECK(hipMemcpy(y, yd, count * sizeof(float), hipMemcpyDeviceToHost));

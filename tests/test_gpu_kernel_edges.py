@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from helios_amd import capi, molecules as M
-from oracle import ccsd, triples as T
+from oracle import ccsd, mlp, triples as T
 from tests._molprep import prepare, random_amplitudes
 
 pytestmark = pytest.mark.gpu
@@ -68,3 +68,51 @@ def test_triples_size_classes(o, v):
     print(o, v, et[0], ref, et[0] - ref)
     assert abs(et[0, 0] - ref[0]) < 1e-11 * abs(ref[0])
     assert abs(et[0, 1] - ref[1]) < 1e-11 * abs(ref[0])
+
+
+def _rows(count, seed):
+    rng = np.random.default_rng(seed)
+    rows = np.zeros((count, mlp.NF + 2), dtype=np.float32)
+    rows[:, :mlp.NF] = rng.normal(0, 1, (count, mlp.NF))
+    rows[:, mlp.NF] = rng.normal(0, 0.5, count)
+    rows[:, mlp.NF + 1] = rng.uniform(0.2, 1.0, count)
+    p = mlp.init(7).astype(np.float64)
+    p[mlp.OFF_W3:mlp.OFF_B3] *= 20.0
+    p[mlp.OFF_B1:mlp.OFF_W2] = rng.normal(0, 0.3, 64)
+    p[mlp.OFF_B2:mlp.OFF_W3] = rng.normal(0, 0.3, 64)
+    return rows, p.astype(np.float32)
+
+
+@pytest.mark.parametrize("count", [1, 17, 64, 65, 16384, 16385])
+def test_mlp_gradient_sizes(count):
+    """Loss and gradient where a wave's 16 samples, a workgroup's 64 and the
+    switch to 256 samples per workgroup begin and end, against the oracle with
+    the tolerances of test_gradient_matches_oracle, parameter block by block."""
+    rows, p = _rows(count, count)
+    tr = capi.Trainer(count)
+    tr.set_params(p)
+    tr.write_samples(rows)
+    loss, g = tr.gradient()
+    tr.close()
+    lo, go = mlp.backward(p, rows[:, :mlp.NF], rows[:, mlp.NF].astype(np.float64),
+                          rows[:, mlp.NF + 1].astype(np.float64))
+    assert abs(loss - lo) <= 1e-4 * lo
+    for a, b in [(mlp.OFF_W1, mlp.OFF_B1), (mlp.OFF_B1, mlp.OFF_W2), (mlp.OFF_W2, mlp.OFF_B2),
+                 (mlp.OFF_B2, mlp.OFF_W3), (mlp.OFF_W3, mlp.OFF_B3), (mlp.OFF_B3, mlp.NPARAM)]:
+        assert np.abs(g[a:b] - go[a:b]).max() <= 1e-2 * np.abs(go[a:b]).max() + 1e-7
+
+
+def test_epoch_loss_with_a_short_last_batch():
+    """The last mini-batch of an epoch (44 of 300 rows in batches of 128) fills
+    fewer workgroups than the others; with steps of 1e-30 the epoch's mean loss
+    is the plain loss, up to FP32 rounding of each row's."""
+    rows, p = _rows(300, 5)
+    tr = capi.Trainer(300)
+    tr.set_params(p)
+    tr.write_samples(rows)
+    loss, _ = tr.gradient()
+    hist = tr.train(epochs=2, batch=128, lr=1e-30, lr_final=1e-30)
+    moved = np.abs(tr.params().astype(np.float64) - p).max()   # six Adam steps of at most about 1e-30
+    tr.close()
+    assert moved < 1e-29
+    assert np.abs(hist - loss).max() <= 1e-6 * loss
