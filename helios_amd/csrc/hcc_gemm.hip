@@ -11,11 +11,14 @@
 // round-robin over the 8 XCDs by the dispatcher, so logical tile
 // (b % 8) * ceil(T/8) + b / 8 gives each XCD one contiguous run of tiles and
 // keeps a molecule's tiles (which share operands) in one L2.
+#include <type_traits>
+
 #include "hcc_internal.h"
 
 namespace hcc {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
+typedef double d2 __attribute__((ext_vector_type(2)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
@@ -34,12 +37,16 @@ __device__ __forceinline__ gdouble* gptr(double* p) { return (gdouble*)p; }
 // slab's store to LDS.  Valid offsets stay below 2 GiB (the largest operand is
 // far smaller).
 constexpr int kRsrcBytes = 0x7ffffff0;
-constexpr int kOobOffset = 0x7ffffff8;
+constexpr unsigned kPadByte = 0x80000000u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const double* p) {
   return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, kRsrcBytes, 0x00020000);
 }
 __device__ __forceinline__ double bload(__amdgpu_buffer_rsrc_t r, int byte_off) {
   return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, byte_off, 0, 0));
+}
+// 16 bytes at an 8-byte aligned offset
+__device__ __forceinline__ d2 bload2(__amdgpu_buffer_rsrc_t r, int byte_off) {
+  return __builtin_bit_cast(d2, __builtin_amdgcn_raw_buffer_load_b128(r, byte_off, 0, 0));
 }
 // r / radix for 0 <= r < kMaxIndex, 1 <= radix < kMaxRadix (exact, see Operand)
 __device__ __forceinline__ int quot(int r, double inv) { return (int)(((double)r + 0.5) * inv); }
@@ -64,34 +71,43 @@ __device__ __forceinline__ int logical_tile(int total) {
 }
 
 // ---------------------------------------------------------------------------
-// FP64 kernel.  Template on the output tile (BM x BN, 32x32 per wave, 4 or 1
-// waves).  LDS layouts follow the operand's unit stride so that both the
-// staging stores and the MFMA fragment reads are free of bank conflicts:
-//   K-contiguous operands are staged [row][k] with a 17-double pitch,
-//   row-contiguous operands [k][row] with a (BM+2)-double pitch.
-// The composite-index offsets along K are precomputed once per work item into
-// LDS tables (chunks up to kKTab), so the slab loop does no integer division.
+// FP64 kernel: output tile BM x BN, 32x32 per wave (4 waves or 1), 16-deep K
+// slabs staged through LDS.
+//
+// What bounds it: the matrix cores, and next to them the return path of the
+// vector loads -- a 64-lane 8-byte load occupies it for 32 cycles (4 lanes at
+// a time), which at 64x64 tiles is as long as the slab's matrix work.  So an
+// operand is staged in 16-byte pairs along its unit-stride dimension wherever
+// pairs exist (GemmProb::modes):
+//   mode 0  pairs along K, staged [row][k];
+//   mode 1  pairs along the rows (columns of B), staged [k][row];
+//   mode 2  single elements, staged [k][row]: any strides.
+// Pairs along K never straddle a run of an odd composite radix: K is
+// enumerated with one padding element behind each such run (GemmProb::krun),
+// and a pair whose second element is padding (bit 0 of its K-table entry)
+// drops it.  Measured with single loads and with pairs, TF/s of 2 M N K: one
+// 100-site molecule's 2500^3 contractions 42-50 and 45-53, its solve 313 and
+// 287 ms; 512 ragged molecules of 10 to 48 sites 37-41 and 38-43, 316 and
+// 305 ms (64 at 4096^3, where the last wave of tiles weighs little).  The
+// register bound keeps the accumulators in VGPRs: with a larger budget the
+// compiler moves them to AGPRs and back every slab.
+//
+// Fragments are read from LDS 16 bytes at a time too: mode 0 gives a lane two
+// consecutive K, used by the two halves of an 8-deep step (the K order within
+// a step is free), modes 1 and 2 two consecutive rows, one for each of the
+// wave's two 16-row blocks.  Both layouts are free of bank conflicts.
 // ---------------------------------------------------------------------------
-constexpr int kKTab = 2048;
-constexpr int kPk = kBK + 1;   // pitch of the [row][k] staging layout (16-deep slabs)
+constexpr int kPk = kBK + 2;   // pitch of the [row][k] staging layout (16-byte aligned rows)
 
-// K-contiguous operands are staged [k / 16][row][k % 16] with a 17-double
-// row pitch (16-deep panels), whatever the slab depth BK.
-template <int BM, int BN, int BK>
+template <int BM, int BN>
 struct F64Tile {
-  static constexpr int kWaves = (BM / 32) * (BN / 32);
-  static constexpr int kT = 64 * kWaves;
-  // pitch of the [k][m] layout: == 16 (mod 32) doubles, so the fragment reads
-  // of rows k and k+1 (lanes 0-15 and 16-31) fall in disjoint bank halves
+  static constexpr int kT = 64 * (BM / 32) * (BN / 32);
+  // pitch of the [k][row] layout: == 16 (mod 32) doubles, so that the
+  // fragment reads of neighbouring K fall in disjoint bank halves
   static constexpr int kPa = BM + 16;
   static constexpr int kPb = BN + 16;
-  static constexpr int kLdsA = ((BK / 16) * BM * kPk > BK * kPa) ? (BK / 16) * BM * kPk : BK * kPa;
-  static constexpr int kLdsB = ((BK / 16) * BN * kPk > BK * kPb) ? (BK / 16) * BN * kPk : BK * kPb;
-  // offset of (row, k) in the K-contiguous layout of an R-row operand
-  template <int R>
-  static __device__ __forceinline__ int rk(int row, int k) { return (k >> 4) * (R * kPk) + row * kPk + (k & 15); }
-  static constexpr int kNA = BM * BK / kT;    // A elements per thread per slab
-  static constexpr int kNB = BN * BK / kT;
+  static constexpr int kLdsA = BM * kPk > kBK * kPa ? BM * kPk : kBK * kPa;
+  static constexpr int kLdsB = BN * kPk > kBK * kPb ? BN * kPk : kBK * kPb;
   // K-offset table length (LDS) per chunk: small enough that the table does
   // not limit the workgroups per CU
   static constexpr int kKT = BM >= 64 ? 1024 : 512;
@@ -99,56 +115,61 @@ struct F64Tile {
 
 #define HCC_F64_THREADS(BM_, BN_) (64 * ((BM_) / 32) * ((BN_) / 32))
 
-// AKF: A's unit stride runs along K; BNF: B's unit stride runs along N.  Both
-// are template parameters so the slab loop is straight-line code and the
-// accumulators stay in AGPRs across iterations.  BK: slab depth (16 or 32;
-// 32 halves the barriers per K for long contractions).
-template <int BM, int BN, int BK, bool AKF, bool BNF>
-__global__ __launch_bounds__(HCC_F64_THREADS(BM, BN)) void gemm_f64_kernel(const GemmProb* __restrict__ probs,
-                                                                           const int* __restrict__ tile_prob,
-                                                                           int total_tiles,
-                                                                           const int* __restrict__ active) {
-  using TL = F64Tile<BM, BN, BK>;
+// staged pieces of thread t (of T) in an R-row x 16 slab: piece i is the pair
+// or element at (row(t, i), k(t, i))
+template <int MODE, int R, int T>
+struct F64Stage {
+  static constexpr int kN = (MODE == 2 ? R * kBK : R * kBK / 2) / T;   // pieces per thread
+  static constexpr int kNK = MODE == 0 ? 1 : kN;                        // distinct K per thread
+  static_assert(kN * T == (MODE == 2 ? R * kBK : R * kBK / 2) && T % 8 == 0, "staging covers the slab");
+  static __device__ __forceinline__ int row(int t, int i) {
+    return MODE == 0 ? t / 8 + (T / 8) * i : (MODE == 1 ? 2 * (t % (R / 2)) : t % R);
+  }
+  static __device__ __forceinline__ int k(int t, int i) {
+    return MODE == 0 ? 2 * (t % 8) : (MODE == 1 ? t / (R / 2) + (2 * T / R) * i : t / R + (T / R) * i);
+  }
+};
+
+// one tile of problem P: staging modes MA of A, MB of B
+template <int BM, int BN, int MA, int MB>
+__device__ __forceinline__ void gemm_f64_tile(const GemmProb& P, int lt, double* As, double* Bs, unsigned* koffA,
+                                              unsigned* koffB) {
+  using TL = F64Tile<BM, BN>;
   constexpr int T = TL::kT;
-  __shared__ double As[TL::kLdsA];
-  __shared__ double Bs[TL::kLdsB];
-  __shared__ int koffA[TL::kKT];
-  __shared__ int koffB[TL::kKT];
-  const int tile = logical_tile(total_tiles);
-  if (tile >= total_tiles) return;
-  const GemmProb P = probs[find_problem(tile_prob, tile)];
-  if (active != nullptr && active[P.mol] == 0) return;
+  using SA = F64Stage<MA, BM, T>;
+  using SB = F64Stage<MB, BN, T>;
   const int tiles_n = (P.N + BN - 1) / BN;
   const int tiles_mn = ((P.M + BM - 1) / BM) * tiles_n;
-  int lt = tile - P.tile_begin;
   const int ks = lt / tiles_mn;
   lt -= ks * tiles_mn;
   const int m0 = (lt / tiles_n) * BM;
   const int n0 = (lt % tiles_n) * BN;
   const int kbeg = ks * P.kchunk;
-  const int kend = min(P.K, kbeg + P.kchunk);
+  const int kend = min(P.kpad, kbeg + P.kchunk);
   const int t = threadIdx.x;
-  const int lane = t & 63, wave = t >> 6;
+  const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int wm = (wave / (BN / 32)) * 32, wn = (wave % (BN / 32)) * 32;
 
-  // fixed (non-K) offsets of this thread's staged elements; -1 marks padding
-  int fa[TL::kNA], fb[TL::kNB], kqa[TL::kNA], kqb[TL::kNB];
+  // fixed (non-K) byte offsets of this thread's staged pieces; kPadByte
+  // marks padding, as it does in the K tables: every sum with one sentinel
+  // lies past the resources (reads 0), a sum of two wraps to the operand's
+  // first elements, whose products only reach padding rows or columns.  The
+  // second element of a pair at an odd problem's last row is the next one in
+  // memory (the arenas end in padding) and reaches a padding row only.
+  unsigned fa[SA::kN], fb[SB::kN];
 #pragma unroll
-  for (int i = 0; i < TL::kNA; ++i) {
-    const int q = t + i * T;
-    const int m = m0 + (AKF ? q / BK : q % BM);
-    kqa[i] = AKF ? q % BK : q / BM;
-    fa[i] = m < P.M ? row_off(P.A, m) : -1;
+  for (int i = 0; i < SA::kN; ++i) {
+    const int m = m0 + SA::row(t, i);
+    fa[i] = m < P.M ? 8u * (unsigned)row_off(P.A, m) : kPadByte;
   }
 #pragma unroll
-  for (int i = 0; i < TL::kNB; ++i) {
-    const int q = t + i * T;
-    const int n = n0 + (BNF ? q % BN : q / BK);
-    kqb[i] = BNF ? q / BN : q % BK;
-    fb[i] = n < P.N ? col_off(P.B, n) : -1;
+  for (int i = 0; i < SB::kN; ++i) {
+    const int n = n0 + SB::row(t, i);
+    fb[i] = n < P.N ? 8u * (unsigned)col_off(P.B, n) : kPadByte;
   }
   const __amdgpu_buffer_rsrc_t rA = rsrc(P.A.p), rB = rsrc(P.B.p);
-  double ra[TL::kNA], rb[TL::kNB];
+  d2 ra[SA::kN], rb[SB::kN];   // mode 2 uses the first element
+  unsigned ca = 0, cb = 0;     // mode 0: bit 0 = the pair's second element is padding
 
   d4 acc[2][2];
 #pragma unroll
@@ -157,102 +178,147 @@ __global__ __launch_bounds__(HCC_F64_THREADS(BM, BN)) void gemm_f64_kernel(const
     for (int j = 0; j < 2; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
 
   for (int c0 = kbeg; c0 < kend; c0 += TL::kKT) {
-    const int cend = min(kend, c0 + TL::kKT);
+    const int clen = min(kend - c0, TL::kKT);
     __syncthreads();
-    for (int q = t; q < cend - c0; q += T) {
-      koffA[q] = col_off(P.A, c0 + q);
-      koffB[q] = row_off(P.B, c0 + q);
+    // K offsets of the chunk, with a slab of padding behind it for the last,
+    // partial slab and the final prefetch
+    for (int q = t; q < clen + 2 * kBK; q += T) {
+      const int kp = c0 + q;
+      const int hi = P.krun > 0 ? quot(kp, P.irun) : 0, lo = kp - hi * (P.krun + 1);
+      const int k = kp - hi, run = P.krun > 0 ? P.krun : P.K;   // krun = 0: one run of K
+      const bool in = q < clen && lo < run && k < P.K;
+      const unsigned last = lo + 1 >= run ? 1u : 0u;
+      koffA[q] = in ? 8u * (unsigned)col_off(P.A, k) | last : kPadByte;
+      koffB[q] = in ? 8u * (unsigned)row_off(P.B, k) | last : kPadByte;
     }
     __syncthreads();
-    // staging loads: padded elements read 0 through the out-of-range offset
-    const int klast = cend - c0 - 1;
-    auto load = [&](int k0) {
+    auto load = [&](int kl0) {
+      unsigned ka[SA::kNK], kb[SB::kNK];
 #pragma unroll
-      for (int i = 0; i < TL::kNA; ++i) {
-        const int kl = k0 - c0 + kqa[i];
-        const int kv = koffA[min(kl, klast)];
-        ra[i] = bload(rA, fa[i] >= 0 && kl <= klast ? (fa[i] + kv) * 8 : kOobOffset);
+      for (int i = 0; i < SA::kNK; ++i) ka[i] = koffA[kl0 + SA::k(t, i)];
+#pragma unroll
+      for (int i = 0; i < SB::kNK; ++i) kb[i] = koffB[kl0 + SB::k(t, i)];
+      if (MA == 0) ca = ka[0];
+      if (MB == 0) cb = kb[0];
+#pragma unroll
+      for (int i = 0; i < SA::kN; ++i) {
+        const int off = (int)(fa[i] + (ka[MA == 0 ? 0 : i] & ~1u));
+        if (MA == 2) ra[i][0] = bload(rA, off);
+        else ra[i] = bload2(rA, off);
       }
 #pragma unroll
-      for (int i = 0; i < TL::kNB; ++i) {
-        const int kl = k0 - c0 + kqb[i];
-        const int kv = koffB[min(kl, klast)];
-        rb[i] = bload(rB, fb[i] >= 0 && kl <= klast ? (fb[i] + kv) * 8 : kOobOffset);
+      for (int i = 0; i < SB::kN; ++i) {
+        const int off = (int)(fb[i] + (kb[MB == 0 ? 0 : i] & ~1u));
+        if (MB == 2) rb[i][0] = bload(rB, off);
+        else rb[i] = bload2(rB, off);
       }
     };
-    load(c0);
-    for (int k0 = c0; k0 < cend; k0 += BK) {
+    load(0);
+    for (int k0 = 0; k0 < clen; k0 += kBK) {
 #pragma unroll
-      for (int i = 0; i < TL::kNA; ++i) {
-        const int q = t + i * T;
-        if (AKF) As[TL::template rk<BM>(q / BK, q % BK)] = ra[i];
-        else As[(q / BM) * TL::kPa + q % BM] = ra[i];
+      for (int i = 0; i < SA::kN; ++i) {
+        if (MA == 0) {
+          if (ca & 1u) ra[i][1] = 0.0;
+          *(d2*)&As[SA::row(t, i) * kPk + SA::k(t, i)] = ra[i];
+        } else if (MA == 1) {
+          *(d2*)&As[SA::k(t, i) * TL::kPa + SA::row(t, i)] = ra[i];
+        } else {
+          As[SA::k(t, i) * TL::kPa + SA::row(t, i)] = ra[i][0];
+        }
       }
 #pragma unroll
-      for (int i = 0; i < TL::kNB; ++i) {
-        const int q = t + i * T;
-        if (BNF) Bs[(q / BN) * TL::kPb + q % BN] = rb[i];
-        else Bs[TL::template rk<BN>(q / BK, q % BK)] = rb[i];
+      for (int i = 0; i < SB::kN; ++i) {
+        if (MB == 0) {
+          if (cb & 1u) rb[i][1] = 0.0;
+          *(d2*)&Bs[SB::row(t, i) * kPk + SB::k(t, i)] = rb[i];
+        } else if (MB == 1) {
+          *(d2*)&Bs[SB::k(t, i) * TL::kPb + SB::row(t, i)] = rb[i];
+        } else {
+          Bs[SB::k(t, i) * TL::kPb + SB::row(t, i)] = rb[i][0];
+        }
       }
       __syncthreads();
-      load(min(k0 + BK, cend));   // the last prefetch is fully masked
+      load(k0 + kBK);   // the last prefetch reads only padding
 #pragma unroll
-      for (int kk = 0; kk < BK; kk += 4) {
-        const int kr = kk + (lane >> 4);
-        const int ma = wm + (lane & 15), nb = wn + (lane & 15);
-        const double a0 = AKF ? As[TL::template rk<BM>(ma, kr)] : As[kr * TL::kPa + ma];
-        const double a1 = AKF ? As[TL::template rk<BM>(ma + 16, kr)] : As[kr * TL::kPa + ma + 16];
-        const double b0 = BNF ? Bs[kr * TL::kPb + nb] : Bs[TL::template rk<BN>(nb, kr)];
-        const double b1 = BNF ? Bs[kr * TL::kPb + nb + 16] : Bs[TL::template rk<BN>(nb + 16, kr)];
-        acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
-        acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
-        acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
-        acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
+      for (int kk = 0; kk < kBK; kk += 8) {
+        const int kg = kk + 2 * (lane >> 4), l = lane & 15;
+        d2 a[2], b[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          a[i] = MA == 0 ? *(const d2*)&As[(wm + 16 * i + l) * kPk + kg] : *(const d2*)&As[(kg + i) * TL::kPa + wm + 2 * l];
+          b[i] = MB == 0 ? *(const d2*)&Bs[(wn + 16 * i + l) * kPk + kg] : *(const d2*)&Bs[(kg + i) * TL::kPb + wn + 2 * l];
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(MA == 0 ? a[i][h] : a[h][i], MB == 0 ? b[j][h] : b[h][j],
+                                                               acc[i][j], 0, 0, 0);
       }
       __syncthreads();
     }
   }
 
   // epilogue: for the FP64 MFMA, D[row][col] of a 16x16 block sits in lane
-  // (col + 16*(row%4)), element row/4
-  if (P.ksplit > 1) {
-    gdouble* __restrict__ W = gptr(P.ws + (long)ks * P.M * P.N);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int col = n0 + wn + 16 * j + (lane & 15);
-      if (col >= P.N) continue;
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = m0 + wm + 16 * i + (lane >> 4) + 4 * r;
-          if (row < P.M) W[(long)row * P.N + col] = acc[i][j][r];
-        }
-    }
-    return;
-  }
-  gdouble* __restrict__ Cp = gptr(P.C.p);
+  // (col + 16*(row%4)), element row/4; modes 1 and 2 interleave the rows
+  // (columns) of the two blocks
+  gdouble* __restrict__ W = gptr(P.ksplit > 1 ? P.ws + (long)ks * P.M * P.N : P.C.p);
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    const int col = n0 + wn + 16 * j + (lane & 15);
+    const int col = n0 + wn + (MB == 0 ? 16 * j + (lane & 15) : 2 * (lane & 15) + j);
     if (col >= P.N) continue;
-    const int co = col_off(P.C, col);
+    const int co = P.ksplit > 1 ? col : col_off(P.C, col);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = m0 + wm + 16 * i + (lane >> 4) + 4 * r;
+        const int br = (lane >> 4) + 4 * r, row = m0 + wm + (MA == 0 ? 16 * i + br : 2 * br + i);
         if (row >= P.M) continue;
+        if (P.ksplit > 1) {
+          W[(long)row * P.N + co] = acc[i][j][r];
+          continue;
+        }
         const int o = row_off(P.C, row) + co;
         double v = P.alpha * acc[i][j][r];
-        if (P.beta != 0.0) v += P.beta * Cp[o];
-        Cp[o] = v;
+        if (P.beta != 0.0) v += P.beta * W[o];
+        W[o] = v;
       }
     }
   }
 }
 
-
+template <int BM, int BN>
+__global__ __launch_bounds__(HCC_F64_THREADS(BM, BN)) __attribute__((amdgpu_waves_per_eu(BM == 64 ? 5 : 3))) void gemm_f64_kernel(const GemmProb* __restrict__ probs,
+                                                                           const int* __restrict__ tile_prob,
+                                                                           int total_tiles,
+                                                                           const int* __restrict__ active) {
+  using TL = F64Tile<BM, BN>;
+  __shared__ __attribute__((aligned(16))) double As[TL::kLdsA];
+  __shared__ __attribute__((aligned(16))) double Bs[TL::kLdsB];
+  __shared__ unsigned koffA[TL::kKT + 2 * kBK];
+  __shared__ unsigned koffB[TL::kKT + 2 * kBK];
+  const int tile = logical_tile(total_tiles);
+  if (tile >= total_tiles) return;
+  const GemmProb P = probs[find_problem(tile_prob, tile)];
+  if (active != nullptr && active[P.mol] == 0) return;
+  const int lt = tile - P.tile_begin;
+#define HCC_F64_TILE(MA, MB) \
+  case 3 * MA + MB: gemm_f64_tile<BM, BN, MA, MB>(P, lt, As, Bs, koffA, koffB); break;
+  switch (P.modes) {   // uniform over the workgroup
+    HCC_F64_TILE(0, 0)
+    HCC_F64_TILE(0, 1)
+    HCC_F64_TILE(0, 2)
+    HCC_F64_TILE(1, 0)
+    HCC_F64_TILE(1, 1)
+    HCC_F64_TILE(1, 2)
+    HCC_F64_TILE(2, 0)
+    HCC_F64_TILE(2, 1)
+    HCC_F64_TILE(2, 2)
+  }
+#undef HCC_F64_TILE
+}
 
 // ---------------------------------------------------------------------------
 // Correction-form ("dual") GEMM of the mixed-precision inner iterations:
@@ -721,25 +787,36 @@ hipError_t launch_compact_table(const GemmProb* src, const int* idx, const int* 
   return hipGetLastError();
 }
 
-template <int BM, int BN, int BK>
-static void launch_f64(const GemmProb* probs, const int* tp, int total_tiles, const int* active, hipStream_t s,
-                       int grid, int flags) {
-  constexpr int T = HCC_F64_THREADS(BM, BN);
-  switch (flags & 3) {
-    case 0: hipLaunchKernelGGL((gemm_f64_kernel<BM, BN, BK, false, false>), dim3(grid), dim3(T), 0, s, probs, tp, total_tiles, active); break;
-    case 1: hipLaunchKernelGGL((gemm_f64_kernel<BM, BN, BK, true, false>), dim3(grid), dim3(T), 0, s, probs, tp, total_tiles, active); break;
-    case 2: hipLaunchKernelGGL((gemm_f64_kernel<BM, BN, BK, false, true>), dim3(grid), dim3(T), 0, s, probs, tp, total_tiles, active); break;
-    default: hipLaunchKernelGGL((gemm_f64_kernel<BM, BN, BK, true, true>), dim3(grid), dim3(T), 0, s, probs, tp, total_tiles, active); break;
+void set_f64_modes(GemmProb& p) {
+  const int ra = one_run_cols(p.A) ? 0 : p.A.rc, rb = one_run_rows(p.B) ? 0 : p.B.rr;   // runs along K
+  int ma = unit_cols(p.A) ? 0 : (unit_rows(p.A) && (one_run_rows(p.A) || p.A.rr % 2 == 0) ? 1 : 2);
+  int mb = unit_cols(p.B) ? (one_run_cols(p.B) || p.B.rc % 2 == 0 ? 1 : 2) : (unit_rows(p.B) ? 0 : 2);
+  // a padded enumeration for one operand's odd runs shifts the other's pairs
+  // against its own runs unless they are the same
+  p.krun = 0;
+  if (ma == 0 && ra % 2 == 1) p.krun = ra;
+  if (mb == 0 && rb > 0 && p.krun > 0 && rb != p.krun) mb = 2;
+  if (mb == 0 && rb % 2 == 1 && p.krun == 0) {
+    p.krun = rb;
+    if (ma == 0 && ra > 0) ma = 2;
   }
+  p.modes = 3 * ma + mb;
+  p.kpad = p.krun > 0 ? p.K + p.K / p.krun : p.K;
+  p.irun = 1.0 / (p.krun + 1);
+}
+
+template <int BM, int BN>
+static void launch_f64(const GemmProb* probs, const int* tp, int total_tiles, const int* active, hipStream_t s) {
+  hipLaunchKernelGGL((gemm_f64_kernel<BM, BN>), dim3((total_tiles + 7) / 8 * 8), dim3(HCC_F64_THREADS(BM, BN)), 0, s, probs,
+                     tp, total_tiles, active);
 }
 
 hipError_t launch_gemm_f64(const GemmProb* probs, const int* tile_prob, int total_tiles, const int* active,
-                           hipStream_t s, int tile, int flags) {
+                           hipStream_t s, int tile) {
   if (total_tiles <= 0) return hipSuccess;
-  int grid = ((total_tiles + 7) / 8) * 8;
-  if (tile == 32) launch_f64<32, 32, 16>(probs, tile_prob, total_tiles, active, s, grid, flags);
-  else if (tile == 128) launch_f64<128, 32, 16>(probs, tile_prob, total_tiles, active, s, grid, flags);
-  else launch_f64<64, 64, 16>(probs, tile_prob, total_tiles, active, s, grid, flags);
+  if (tile == 32) launch_f64<32, 32>(probs, tile_prob, total_tiles, active, s);
+  else if (tile == 128) launch_f64<128, 32>(probs, tile_prob, total_tiles, active, s);
+  else launch_f64<64, 64>(probs, tile_prob, total_tiles, active, s);
   return hipGetLastError();
 }
 

@@ -45,6 +45,13 @@ inline Operand make_operand(double* p, int rr, int rc, int srh, int srl, int sch
   return Operand{p, rr, rc, srh, srl, sch, scl, 1.0 / rr, 1.0 / rc};
 }
 
+// the unit stride of an operand's columns or rows, and whether that dimension
+// is one contiguous run (else it comes in runs of its radix)
+inline bool unit_cols(const Operand& o) { return (o.rc == 1 ? o.sch : o.scl) == 1; }
+inline bool unit_rows(const Operand& o) { return (o.rr == 1 ? o.srh : o.srl) == 1; }
+inline bool one_run_cols(const Operand& o) { return o.rc == 1 || o.sch == o.rc; }
+inline bool one_run_rows(const Operand& o) { return o.rr == 1 || o.srh == o.rr; }
+
 struct GemmProb {
   Operand A, B, C;  // A: M x K, B: K x N, C: M x N
   int M, N, K;
@@ -55,7 +62,13 @@ struct GemmProb {
   int a_kfast;      // 1: A's unit stride runs along K, 0: along M
   int b_nfast;      // 1: B's unit stride runs along N, 0: along K
   int ksplit;       // number of K chunks (1: no split)
-  int kchunk;       // K range of one chunk (multiple of the K tile)
+  int kchunk;       // K range of one chunk (multiple of the K tile), in kpad's enumeration
+  // FP64 kernel: staging modes of A and B (3 MA + MB, see gemm_f64_kernel), and
+  // the enumeration of K with one padding element behind every run of krun
+  // (0: no such runs), kpad elements long; irun = 1 / (krun + 1)
+  int modes;
+  int krun, kpad;
+  double irun;
   double* ws;       // split-K partials: ksplit x M x N, row-major (ksplit > 1)
   // correction ("delta") form, used by the mixed-precision inner iterations:
   // Cd += alpha * (A0 dB + dA (B0 + dB)) with A0 = A.p, B0 = B.p and the FP32
@@ -76,11 +89,11 @@ constexpr int kBM = 64, kBN = 64, kBK = 16, kThreads = 256;
 // launches one grouped GEMM over all problems of a table (device memory)
 // tile: 64 (64x64 tiles, 256 threads), 32 (32x32 tiles, 64 threads) or 128
 // (128x32 tiles, 256 threads, for outputs at most 32 columns wide);
-// flags: bit 0 = A's unit stride along K, bit 1 = B's unit stride along N
-// (the same for every problem of a table)
 // tile_prob: problem index of every global tile of the table
 hipError_t launch_gemm_f64(const GemmProb* probs, const int* tile_prob, int total_tiles,
-                           const int* active, hipStream_t s, int tile = 64, int flags = 3);
+                           const int* active, hipStream_t s, int tile = 64);
+// staging modes and K enumeration of a problem for the FP64 kernel
+void set_f64_modes(GemmProb& p);
 // correction-form GEMM (see GemmProb::dA/dB); bf16 = 1 rounds the operands to
 // BF16 for V_MFMA_F32_16X16X32_BF16 (FP32 accumulation; tile kinds 32, 64 and
 // 256 = 128x128 output tiles), 0 keeps FP64 (tile kind 64 only)

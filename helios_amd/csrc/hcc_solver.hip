@@ -52,8 +52,6 @@ static Operand cmp(double* p, int rr, int srh, int srl, int rc, int sch, int scl
   return make_operand(p, rr, rc, srh, srl, sch, scl);
 }
 
-static bool unit_cols(const Operand& o) { return (o.rc == 1 ? o.sch : o.scl) == 1; }
-static bool unit_rows(const Operand& o) { return (o.rr == 1 ? o.srh : o.srl) == 1; }
 
 struct GemmTable {
   GemmProb* d = nullptr;
@@ -117,20 +115,20 @@ static int choose_tile_dual(const GemmProb& p) {
 static void choose_split(GemmProb& p, int ts) {
   const int tmn = ((p.M + tile_m(ts) - 1) / tile_m(ts)) * ((p.N + tile_n(ts) - 1) / tile_n(ts));
   p.ksplit = 1;
-  p.kchunk = p.K;
+  p.kchunk = p.kpad;
   if (tmn >= 16 || p.K < 512) return;
   int want = (16 + tmn - 1) / tmn;
   int maxs = p.K / 128;
   int ks = std::min(want, std::max(1, maxs));
   ks = std::min(ks, 64);
   if (ks <= 1) return;
-  int chunk = (p.K + ks - 1) / ks;
+  int chunk = (p.kpad + ks - 1) / ks;
   chunk = (chunk + 31) / 32 * 32;      // multiple of both K tiles (16 for FP64, 32 for BF16)
   p.kchunk = chunk;
-  p.ksplit = (p.K + chunk - 1) / chunk;
+  p.ksplit = (p.kpad + chunk - 1) / chunk;
   if (p.ksplit <= 1) {
     p.ksplit = 1;
-    p.kchunk = p.K;
+    p.kchunk = p.kpad;
   }
 }
 
@@ -311,15 +309,15 @@ static int choose_tile(const GemmProb& p) {
 // K split of a problem into `ks` chunks (multiples of 32, both K tiles)
 static void force_split(GemmProb& p, int ks) {
   p.ksplit = 1;
-  p.kchunk = p.K;
+  p.kchunk = p.kpad;
   if (ks <= 1) return;
-  int chunk = (p.K + ks - 1) / ks;
+  int chunk = (p.kpad + ks - 1) / ks;
   chunk = (chunk + 31) / 32 * 32;
   p.kchunk = chunk;
-  p.ksplit = (p.K + chunk - 1) / chunk;
+  p.ksplit = (p.kpad + chunk - 1) / chunk;
   if (p.ksplit <= 1) {
     p.ksplit = 1;
-    p.kchunk = p.K;
+    p.kchunk = p.kpad;
   }
 }
 
@@ -413,6 +411,7 @@ static GemmTable make_table(Batch& b, const std::function<GemmProb(int)>& build,
     if (p.M <= 0 || p.N <= 0) continue;
     if (p.M >= kMaxIndex || p.N >= kMaxIndex || p.K >= kMaxIndex) throw std::string("GEMM dimension out of range");
     p.mol = k;
+    if (p.Cd == nullptr) set_f64_modes(p);
     int ts = 0, ks = -1;
     if (force_tile) {
       ts = force_tile;
@@ -463,7 +462,7 @@ static GemmProb prob(Operand A, Operand B, Operand C, int M, int N, int K, doubl
   p.C = C;
   p.M = M;
   p.N = N;
-  p.K = K;
+  p.K = p.kpad = K;
   p.alpha = alpha;
   p.beta = beta;
   return p;
@@ -538,7 +537,8 @@ static void allocate(Batch& b, bool keep_mp2) {
       off[k] = total;
       total += (size(b.n[k], b.o[k], b.v[k]) + 31) / 32 * 32;   // 256-byte aligned blocks
     }
-    double* base = b.dalloc<double>(total);
+    // a 16-byte load of the last element's pair reads one element more
+    double* base = b.dalloc<double>(total + 2);
     std::vector<double*> ptr(b.nm);
     for (int k = 0; k < b.nm; ++k) ptr[k] = base + off[k];
     return ptr;
@@ -985,7 +985,7 @@ namespace hcc {
 
 static void launch_table(hcc_ctx* c, const GemmTable& t) {
   const TableView v = view(t);
-  HCHECK(launch_gemm_f64(v.d, v.tp, v.tiles, c->batch->dact, c->stream, t.tile, t.flags));
+  HCHECK(launch_gemm_f64(v.d, v.tp, v.tiles, c->batch->dact, c->stream, t.tile));
   if (v.red > 0) HCHECK(launch_splitk_reduce(v.d, v.rp, v.rb, v.red, c->batch->dact, c->stream));
   if (t.alt >= 0) launch_table(c, c->batch->alt[t.alt]);
 }
@@ -3080,8 +3080,8 @@ int hcc_selftest_gemm(int m, int n, int k, const double* A, const double* B, dou
   int* dtp = nullptr;
   int rc = HCC_OK;
   try {
-    HCHECK(hipMalloc(&dA, sizeof(double) * m * k));
-    HCHECK(hipMalloc(&dB, sizeof(double) * k * n));
+    HCHECK(hipMalloc(&dA, sizeof(double) * ((size_t)m * k + 2)));
+    HCHECK(hipMalloc(&dB, sizeof(double) * ((size_t)k * n + 2)));
     HCHECK(hipMalloc(&dC, sizeof(double) * m * n));
     HCHECK(hipMalloc(&dp, sizeof(GemmProb)));
     HCHECK(hipMemcpy(dA, A, sizeof(double) * m * k, hipMemcpyHostToDevice));
@@ -3090,15 +3090,14 @@ int hcc_selftest_gemm(int m, int n, int k, const double* A, const double* B, dou
     GemmProb p = prob(rm(dA, k), rm(dB, n), rm(dC, n), m, n, k, alpha, beta);
     p.tiles_n = (n + kBN - 1) / kBN;
     p.tile_begin = 0;
-    p.a_kfast = 1;
-    p.b_nfast = 1;
     p.ksplit = 1;
-    p.kchunk = k;
+    set_f64_modes(p);
+    p.kchunk = p.kpad;
     const int tiles = ((m + kBM - 1) / kBM) * p.tiles_n;
     HCHECK(hipMemcpy(dp, &p, sizeof(p), hipMemcpyHostToDevice));
     HCHECK(hipMalloc(&dtp, sizeof(int) * tiles));
     HCHECK(hipMemset(dtp, 0, sizeof(int) * tiles));
-    HCHECK(launch_gemm_f64(dp, dtp, tiles, nullptr, nullptr, 64, 3));
+    HCHECK(launch_gemm_f64(dp, dtp, tiles, nullptr, nullptr, 64));
     HCHECK(hipDeviceSynchronize());
     HCHECK(hipMemcpy(C, dC, sizeof(double) * m * n, hipMemcpyDeviceToHost));
   } catch (const HipError&) {
