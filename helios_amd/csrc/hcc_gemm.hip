@@ -8,9 +8,9 @@
 // registers while the current one feeds the matrix cores.
 //
 // Tile -> workgroup mapping is XCD-aware: consecutive workgroups are spread
-// round-robin over the 8 XCDs by the dispatcher, so logical tile
-// (b % 8) * ceil(T/8) + b / 8 gives each XCD one contiguous run of tiles and
-// keeps a molecule's tiles (which share operands) in one L2.
+// round-robin over the 8 XCDs by the dispatcher, so workgroup b takes tile
+// b / 8 of XCD b % 8's contiguous run (XcdMap; equal runs in the correction
+// GEMM), which keeps a molecule's tiles (which share operands) in one L2.
 #include <type_traits>
 
 #include "hcc_internal.h"
@@ -292,15 +292,15 @@ __device__ __forceinline__ void gemm_f64_tile(const GemmProb& P, int lt, double*
 template <int BM, int BN>
 __global__ __launch_bounds__(HCC_F64_THREADS(BM, BN)) __attribute__((amdgpu_waves_per_eu(BM == 64 ? 5 : 3))) void gemm_f64_kernel(const GemmProb* __restrict__ probs,
                                                                            const int* __restrict__ tile_prob,
-                                                                           int total_tiles,
+                                                                           XcdMap xcd,
                                                                            const int* __restrict__ active) {
   using TL = F64Tile<BM, BN>;
   __shared__ __attribute__((aligned(16))) double As[TL::kLdsA];
   __shared__ __attribute__((aligned(16))) double Bs[TL::kLdsB];
   __shared__ unsigned koffA[TL::kKT + 2 * kBK];
   __shared__ unsigned koffB[TL::kKT + 2 * kBK];
-  const int tile = logical_tile(total_tiles);
-  if (tile >= total_tiles) return;
+  const int x = blockIdx.x & 7, tile = xcd.begin[x] + (int)(blockIdx.x >> 3);
+  if (tile >= xcd.begin[x + 1]) return;
   const GemmProb P = probs[find_problem(tile_prob, tile)];
   if (active != nullptr && active[P.mol] == 0) return;
   const int lt = tile - P.tile_begin;
@@ -806,17 +806,20 @@ void set_f64_modes(GemmProb& p) {
 }
 
 template <int BM, int BN>
-static void launch_f64(const GemmProb* probs, const int* tp, int total_tiles, const int* active, hipStream_t s) {
-  hipLaunchKernelGGL((gemm_f64_kernel<BM, BN>), dim3((total_tiles + 7) / 8 * 8), dim3(HCC_F64_THREADS(BM, BN)), 0, s, probs,
-                     tp, total_tiles, active);
+static void launch_f64(const GemmProb* probs, const int* tp, const XcdMap& xcd, int longest, const int* active,
+                       hipStream_t s) {
+  hipLaunchKernelGGL((gemm_f64_kernel<BM, BN>), dim3(8 * longest), dim3(HCC_F64_THREADS(BM, BN)), 0, s, probs, tp, xcd,
+                     active);
 }
 
-hipError_t launch_gemm_f64(const GemmProb* probs, const int* tile_prob, int total_tiles, const int* active,
+hipError_t launch_gemm_f64(const GemmProb* probs, const int* tile_prob, const XcdMap& xcd, const int* active,
                            hipStream_t s, int tile) {
-  if (total_tiles <= 0) return hipSuccess;
-  if (tile == 32) launch_f64<32, 32>(probs, tile_prob, total_tiles, active, s);
-  else if (tile == 128) launch_f64<128, 32>(probs, tile_prob, total_tiles, active, s);
-  else launch_f64<64, 64>(probs, tile_prob, total_tiles, active, s);
+  int longest = 0;
+  for (int x = 0; x < 8; ++x) longest = longest > xcd.begin[x + 1] - xcd.begin[x] ? longest : xcd.begin[x + 1] - xcd.begin[x];
+  if (longest <= 0) return hipSuccess;
+  if (tile == 32) launch_f64<32, 32>(probs, tile_prob, xcd, longest, active, s);
+  else if (tile == 128) launch_f64<128, 32>(probs, tile_prob, xcd, longest, active, s);
+  else launch_f64<64, 64>(probs, tile_prob, xcd, longest, active, s);
   return hipGetLastError();
 }
 

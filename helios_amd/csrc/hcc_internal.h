@@ -86,11 +86,16 @@ struct GemmProb {
 // Tile shape of the FP64 MFMA GEMM.
 constexpr int kBM = 64, kBN = 64, kBK = 16, kThreads = 256;
 
+// tiles [begin[x], begin[x + 1]) of a table run on XCD x
+struct XcdMap {
+  int begin[9];
+};
+
 // launches one grouped GEMM over all problems of a table (device memory)
 // tile: 64 (64x64 tiles, 256 threads), 32 (32x32 tiles, 64 threads) or 128
 // (128x32 tiles, 256 threads, for outputs at most 32 columns wide);
 // tile_prob: problem index of every global tile of the table
-hipError_t launch_gemm_f64(const GemmProb* probs, const int* tile_prob, int total_tiles,
+hipError_t launch_gemm_f64(const GemmProb* probs, const int* tile_prob, const XcdMap& xcd,
                            const int* active, hipStream_t s, int tile = 64);
 // staging modes and K enumeration of a problem for the FP64 kernel
 void set_f64_modes(GemmProb& p);

@@ -15,10 +15,9 @@ constexpr int kMaxDiis = 32;
 void ew_dress(const Mol* mols, const State* st, Ragged rgNN, int nm, hipStream_t s);
 void ew_fock_m(const Mol* mols, const State* st, Ragged rgN, Ragged rgNN, int nm, hipStream_t s);
 void ew_pouter(const Mol* mols, const State* st, Ragged rgN3, int nm, hipStream_t s);
-void ew_u(const Mol* mols, const State* st, Ragged rgT2, int nm, hipStream_t s);
-void ew_u(const MolD* mols, const State* st, Ragged rgT2, int nm, hipStream_t s);
-void ew_init_xx(const Mol* mols, const State* st, Ragged rgXX, int nm, hipStream_t s);
-void ew_init_xx(const MolD* mols, const State* st, Ragged rgXX, int nm, hipStream_t s);
+// u = 2 t2 - t2(a<->b) and the Fock parts of the E2 intermediates
+void ew_u_xx(const Mol* mols, const State* st, Ragged rgT2, Ragged rgXX, hipStream_t s);
+void ew_u_xx(const MolD* mols, const State* st, Ragged rgT2, Ragged rgXX, hipStream_t s);
 void ew_assemble(const Mol* mols, const State* st, Ragged rgT2, int nm, hipStream_t s);
 // x += t2 Xvv^T - Xoo^T t2 (the E2 terms, both index placements) for molecules
 // with o, v <= kE2Max (the others take the GEMM path); rgOcc: kE2Split blocks

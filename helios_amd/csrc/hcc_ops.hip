@@ -26,9 +26,10 @@ __device__ __forceinline__ int block_mol(const int* __restrict__ prefix, int nm,
   return lo;
 }
 
-#define RAGGED_PROLOGUE(SIZE)                                         \
-  const int mol = rg.bmol[blockIdx.x];                               \
-  const int lb = blockIdx.x - rg.prefix[mol];                        \
+#define RAGGED_PROLOGUE(SIZE) RAGGED_PROLOGUE_OF(blockIdx.x, SIZE)
+#define RAGGED_PROLOGUE_OF(BLOCK, SIZE)                              \
+  const int mol = rg.bmol[BLOCK];                                    \
+  const int lb = (BLOCK) - rg.prefix[mol];                           \
   const auto& M = mols[mol];                                         \
   const long e = (long)lb * kEwThreads + threadIdx.x;                \
   const long size_ = (SIZE);                                         \
@@ -165,9 +166,8 @@ __global__ __launch_bounds__(kEwThreads) void k_pouter(const Mol* __restrict__ m
 
 // u = 2 t2 - t2(a<->b); kEwItems elements per thread, loads before stores
 template <class MT>
-__global__ __launch_bounds__(kEwThreads) void k_u(const MT* __restrict__ mols, const State* __restrict__ st,
-                                                 Ragged rg, int nm) {
-  RAGGED_PROLOGUE((long)mols[mol].o * mols[mol].o * mols[mol].v * mols[mol].v);
+__device__ __forceinline__ void u_block(const MT* __restrict__ mols, const State* __restrict__ st, const Ragged& rg, int block) {
+  RAGGED_PROLOGUE_OF(block, (long)mols[mol].o * mols[mol].o * mols[mol].v * mols[mol].v);
   if (!st[mol].active) return;
   using V = std::remove_pointer_t<decltype(M.t2)>;
   const int v = M.v, vv = v * v;
@@ -194,9 +194,9 @@ __global__ __launch_bounds__(kEwThreads) void k_u(const MT* __restrict__ mols, c
 
 // Xvv = Ft_vv, Xoo = Ft_oo (the Fock parts of the E2 intermediates)
 template <class MT>
-__global__ __launch_bounds__(kEwThreads) void k_init_xx(const MT* __restrict__ mols, const State* __restrict__ st,
-                                                       Ragged rg, int nm) {
-  RAGGED_PROLOGUE((long)mols[mol].v * mols[mol].v + (long)mols[mol].o * mols[mol].o);
+__device__ __forceinline__ void init_xx_block(const MT* __restrict__ mols, const State* __restrict__ st, const Ragged& rg,
+                                              int block) {
+  RAGGED_PROLOGUE_OF(block, (long)mols[mol].v * mols[mol].v + (long)mols[mol].o * mols[mol].o);
   if (e >= size_ || !st[mol].active) return;
   const int N = M.n, o = M.o, v = M.v;
   if (e < (long)v * v) {
@@ -207,6 +207,15 @@ __global__ __launch_bounds__(kEwThreads) void k_init_xx(const MT* __restrict__ m
     const int k = f / o, j = f % o;
     M.Xoo[f] = M.Ft[(long)k * N + j];
   }
+}
+
+// k_u and k_init_xx in one launch (both precede the contractions that read u,
+// Xvv and Xoo): workgroups past the first table's are the second's
+template <class MT>
+__global__ __launch_bounds__(kEwThreads) void k_u_xx(const MT* __restrict__ mols, const State* __restrict__ st, Ragged rgT2,
+                                                    Ragged rgXX) {
+  if ((int)blockIdx.x < rgT2.nblocks) u_block(mols, st, rgT2, blockIdx.x);
+  else init_xx_block(mols, st, rgXX, blockIdx.x - rgT2.nblocks);
 }
 
 // w2 += x + x^T - 1/2 (Z[ai,bj] + Z[bj,ai]) - (Z[aj,bi] + Z[bi,aj]), with
@@ -902,24 +911,19 @@ void ew_pouter(const Mol* mols, const State* st, Ragged rgN3, int nm, hipStream_
   RAGGED_LAUNCH(k_pouter, rgN3, mols, st, rgN3, nm);
 }
 template <class MT>
-static void ew_u_t(const MT* mols, const State* st, Ragged rgT2, int nm, hipStream_t s) {
-  RAGGED_LAUNCH(k_u<MT>, rgT2, mols, st, rgT2, nm);
-}
-template <class MT>
-static void ew_init_xx_t(const MT* mols, const State* st, Ragged rgXX, int nm, hipStream_t s) {
-  RAGGED_LAUNCH(k_init_xx<MT>, rgXX, mols, st, rgXX, nm);
+static void ew_u_xx_t(const MT* mols, const State* st, Ragged rgT2, Ragged rgXX, hipStream_t s) {
+  const int blocks = rgT2.nblocks + rgXX.nblocks;
+  if (blocks > 0) hipLaunchKernelGGL(k_u_xx<MT>, dim3(blocks), dim3(kEwThreads), 0, s, mols, st, rgT2, rgXX);
 }
 template <class MT>
 static void ew_assemble_t(const MT* mols, const State* st, Ragged rgT2, int nm, hipStream_t s) {
   RAGGED_LAUNCH(k_assemble<MT>, rgT2, mols, st, rgT2, nm);
 }
-void ew_u(const Mol* mols, const State* st, Ragged rgT2, int nm, hipStream_t s) { ew_u_t(mols, st, rgT2, nm, s); }
-void ew_u(const MolD* mols, const State* st, Ragged rgT2, int nm, hipStream_t s) { ew_u_t(mols, st, rgT2, nm, s); }
-void ew_init_xx(const Mol* mols, const State* st, Ragged rgXX, int nm, hipStream_t s) {
-  ew_init_xx_t(mols, st, rgXX, nm, s);
+void ew_u_xx(const Mol* mols, const State* st, Ragged rgT2, Ragged rgXX, hipStream_t s) {
+  ew_u_xx_t(mols, st, rgT2, rgXX, s);
 }
-void ew_init_xx(const MolD* mols, const State* st, Ragged rgXX, int nm, hipStream_t s) {
-  ew_init_xx_t(mols, st, rgXX, nm, s);
+void ew_u_xx(const MolD* mols, const State* st, Ragged rgT2, Ragged rgXX, hipStream_t s) {
+  ew_u_xx_t(mols, st, rgT2, rgXX, s);
 }
 void ew_assemble(const Mol* mols, const State* st, Ragged rgT2, int nm, hipStream_t s) {
   ew_assemble_t(mols, st, rgT2, nm, s);

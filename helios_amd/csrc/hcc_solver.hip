@@ -68,6 +68,8 @@ struct GemmTable {
   // its molecule, tiles and split-K reduction blocks; the compacted copies of
   // the problems, the tile and reduction-block maps, and the uploaded lists
   std::vector<int> hmol, htiles, hred, hbuf;
+  std::vector<float> hcost;    // cost of one tile of each problem
+  XcdMap xcd{}, cxcd{};        // tiles of each XCD, full and compacted
   GemmProb* cd = nullptr;
   int *ctp = nullptr, *cbp = nullptr, *cbuf = nullptr;
   int ctiles = -1;             // tiles of the compacted copy; -1: not compacted
@@ -82,10 +84,32 @@ struct TableView {
   const int* rp;
   const int* rb;
   int red;
+  const XcdMap* xcd;
 };
 static TableView view(const GemmTable& t) {
-  if (t.ctiles < 0) return {t.d, t.tile_prob, t.tiles, t.red_prefix, t.red_bprob, t.red_blocks};
-  return {t.cd, t.ctp, t.ctiles, t.cbuf + 2 * t.nprob + 1, t.cbp, t.cred};
+  if (t.ctiles < 0) return {t.d, t.tile_prob, t.tiles, t.red_prefix, t.red_bprob, t.red_blocks, &t.xcd};
+  return {t.cd, t.ctp, t.ctiles, t.cbuf + 2 * t.nprob + 1, t.cbp, t.cred, &t.cxcd};
+}
+
+// Contiguous runs of a table's tiles for the 8 XCDs, of equal cost: the tiles
+// of one launch differ in K, so equal counts would leave XCDs idle.
+static XcdMap xcd_runs(const std::vector<int>& tiles, const std::vector<float>& cost) {
+  double total = 0.0;
+  for (size_t q = 0; q < tiles.size(); ++q) total += (double)tiles[q] * cost[q];
+  XcdMap m{};
+  double done = 0.0;
+  int at = 0, x = 1;
+  for (size_t q = 0; q < tiles.size(); ++q) {
+    const double c = (double)tiles[q] * cost[q];
+    while (x < 8 && done + c >= total * x / 8.0) {
+      m.begin[x] = std::max(m.begin[x - 1], at + (int)((total * x / 8.0 - done) / cost[q] + 0.5));
+      ++x;
+    }
+    done += c;
+    at += tiles[q];
+  }
+  for (; x < 9; ++x) m.begin[x] = at;
+  return m;
 }
 
 // Tile kinds of the FP64 GEMM: 64 (64x64, 4 waves), 32 (32x32, 1 wave) and
@@ -156,7 +180,10 @@ struct Batch {
   bool guess_large = false;   // some molecule has v > 32 (pairwise learned-guess kernel)
   Ragged rgT2x, rgT2Sx;   // rgT2, rgT2S with kEwItems elements per thread
   double *part1 = nullptr, *part2 = nullptr, *partE = nullptr, *partD = nullptr;
-  std::vector<GemmTable> pre, it;
+  std::vector<GemmTable> pre;
+  GemmTable g1;                  // Q = gamma P alone (set-up, (T))
+  std::vector<GemmTable> lv;     // the iteration's GEMMs, one table per dependency level
+  std::vector<GemmTable> it;     // one table per contraction (profiling and tuning; built on first use)
   std::vector<GemmTable> alt;   // second (other tile edge) parts of split contraction tables
   // mixed precision: BF16 copies of the outer-point operands (one per arena)
   struct Shadow {
@@ -343,7 +370,10 @@ static GemmTable build_group(Batch& b, std::vector<GemmProb> probs, int ts) {
     t.hmol.push_back(p.mol);
     t.htiles.push_back(((p.M + tile_m(ts) - 1) / tile_m(ts)) * p.tiles_n * p.ksplit);
     t.hred.push_back(p.ksplit > 1 ? (int)(((long)p.M * p.N + 255) / 256) : 0);
+    // matrix work of a tile plus the equivalent of its set-up, first loads and stores
+    t.hcost.push_back((float)(p.kchunk + 96));
   }
+  t.xcd = xcd_runs(t.htiles, t.hcost);
   if (!probs.empty()) {
     // the staging layout is a performance choice only (addressing is general):
     // take the largest problem's unit-stride flags for the whole table
@@ -397,49 +427,53 @@ static GemmTable build_group(Batch& b, std::vector<GemmProb> probs, int ts) {
   return t;
 }
 
-// Table of one contraction over every molecule.  Each problem gets its tile
-// edge and K split from the measured tuning of its (op, n_occ, n_virt) when
-// there is one, else from the cost heuristic (choose_tile / choose_split);
-// problems with 32x32 tiles go to a second launch (Batch::alt).
-// force_tile / force_ks (> 0) override both for every problem.
-static GemmTable make_table(Batch& b, const std::function<GemmProb(int)>& build, bool allow_split = true,
-                            int force_tile = 0, int op = -1, int force_ks = 0, bool dual = false) {
-  const int kinds[4] = {64, 32, 128, 256};
-  std::vector<GemmProb> groups[4];
-  for (int k = 0; k < b.nm; ++k) {
-    GemmProb p = build(k);
-    if (p.M <= 0 || p.N <= 0) continue;
-    if (p.M >= kMaxIndex || p.N >= kMaxIndex || p.K >= kMaxIndex) throw std::string("GEMM dimension out of range");
-    p.mol = k;
-    if (p.Cd == nullptr) set_f64_modes(p);
-    int ts = 0, ks = -1;
-    if (force_tile) {
-      ts = force_tile;
-      if (force_ks > 0) ks = force_ks;
-    } else if (b.tuning && op >= 0) {
-      auto it = b.tuning->find({op, b.o[k], b.v[k]});
-      if (it != b.tuning->end()) {
-        ts = it->second[0];
-        ks = it->second[1];
-      }
+// Tile kind and K split of problem p of molecule k: the measured tuning of its
+// (op, n_occ, n_virt) when there is one, else the cost heuristic (choose_tile /
+// choose_split); force_tile / force_ks (> 0) override both.  Returns the tile
+// kind, 0 for an empty problem.
+static int plan_problem(Batch& b, GemmProb& p, int k, bool allow_split, int force_tile, int op, int force_ks, bool dual) {
+  if (p.M <= 0 || p.N <= 0) return 0;
+  if (p.M >= kMaxIndex || p.N >= kMaxIndex || p.K >= kMaxIndex) throw std::string("GEMM dimension out of range");
+  p.mol = k;
+  if (p.Cd == nullptr) set_f64_modes(p);
+  int ts = 0, ks = -1;
+  if (force_tile) {
+    ts = force_tile;
+    if (force_ks > 0) ks = force_ks;
+  } else if (b.tuning && op >= 0) {
+    auto it = b.tuning->find({op, b.o[k], b.v[k]});
+    if (it != b.tuning->end()) {
+      ts = it->second[0];
+      ks = it->second[1];
     }
-    if (dual) {
-      if (ts != 32 && ts != 64 && ts != 256) ts = choose_tile_dual(p);
-    } else if (ts != 32 && ts != 64 && ts != 128) {
-      ts = choose_tile(p);
-    }
-    if (!allow_split) force_split(p, 1);
-    else if (ks >= 1) force_split(p, ks);
-    else choose_split(p, ts);
-    groups[ts == 64 ? 0 : (ts == 32 ? 1 : (ts == 128 ? 2 : 3))].push_back(p);
   }
-  // the first non-empty group is the table; the others hang off it through alt links
+  if (dual) {
+    if (ts != 32 && ts != 64 && ts != 256) ts = choose_tile_dual(p);
+  } else if (ts != 32 && ts != 64 && ts != 128) {
+    ts = choose_tile(p);
+  }
+  if (!allow_split) force_split(p, 1);
+  else if (ks >= 1) force_split(p, ks);
+  else choose_split(p, ts);
+  return ts;
+}
+
+// One launch per tile kind over the planned problems: the first non-empty group
+// is the table, the others hang off it through alt links.
+struct ProbGroups {
+  std::vector<GemmProb> of[4];
+  void add(const GemmProb& p, int ts) {
+    if (ts != 0) of[ts == 64 ? 0 : (ts == 32 ? 1 : (ts == 128 ? 2 : 3))].push_back(p);
+  }
+};
+static GemmTable link_groups(Batch& b, const ProbGroups& groups) {
+  const int kinds[4] = {64, 32, 128, 256};
   GemmTable head;
   bool have = false;
   int last = -1;   // index in b.alt of the last linked part, -1: the head
   for (int g = 0; g < 4; ++g) {
-    if (groups[g].empty()) continue;
-    GemmTable t = build_group(b, groups[g], kinds[g]);
+    if (groups.of[g].empty()) continue;
+    GemmTable t = build_group(b, groups.of[g], kinds[g]);
     if (!have) {
       head = t;
       have = true;
@@ -453,6 +487,18 @@ static GemmTable make_table(Batch& b, const std::function<GemmProb(int)>& build,
   }
   if (!have) head = build_group(b, {}, 64);
   return head;
+}
+
+// Table of one contraction over every molecule
+static GemmTable make_table(Batch& b, const std::function<GemmProb(int)>& build, bool allow_split = true,
+                            int force_tile = 0, int op = -1, int force_ks = 0, bool dual = false) {
+  ProbGroups groups;
+  for (int k = 0; k < b.nm; ++k) {
+    GemmProb p = build(k);
+    const int ts = plan_problem(b, p, k, allow_split, force_tile, op, force_ks, dual);
+    groups.add(p, ts);
+  }
+  return link_groups(b, groups);
 }
 
 static GemmProb prob(Operand A, Operand B, Operand C, int M, int N, int K, double alpha, double beta) {
@@ -714,10 +760,7 @@ static void build_tables(Batch& b) {
   // --- one iteration
   b.it.clear();
   b.ops.clear();
-  auto add = [&](const std::function<GemmProb(const Mol&)>& f) {
-    b.ops.push_back(f);
-    b.it.push_back(make_table(b, [&](int k) { return f(H[k]); }, true, 0, (int)b.it.size()));
-  };
+  auto add = [&](const std::function<GemmProb(const Mol&)>& f) { b.ops.push_back(f); };
   // g1: Q = gamma P
   add([](const Mol& M) {
     const int N = M.n, N2 = N * N;
@@ -868,6 +911,75 @@ static void build_tables(Batch& b) {
   });
 }
 
+enum ItOp {
+  G1_Q = 0, G2A, G2B, G3, G4_, G5, G6, G7, G8, G9, G10, G11, G12, G13, G14, G15, G16, G17, G18, G19, G20,
+  G21, G22, G23, G24, N_IT_OPS
+};
+
+// Dependency levels of the iteration's GEMMs: those of a level read only what
+// the levels before them (and the elementwise kernels between) have written
+// and write different arrays, so one launch per tile kind runs them all.  The
+// order of the contributions to an accumulated array (w1: G4, G6, G7; w2: G8,
+// G10, G13; WD: G17, G18, G19; x: G20, G23, G24) is that of the contractions,
+// so results do not depend on the grouping.
+//
+// Why: a launch costs 4.4 us inside a graph, more than the work of a
+// contraction of a small molecule, and the last wave of workgroups of each
+// launch leaves most of the chip idle (2500^3 contractions of one 100-site
+// molecule: 1600 tiles on 256 CUs, 45-53 TF/s alone).  Solves with one launch
+// per contraction and with levels: octatetraene 6.7 and 4.1 ms, 25 x 14 sites
+// 13.0 and 7.5 ms, 100 sites 287 and 223 ms, 512 ragged molecules 305 and
+// 285 ms.
+static const std::vector<std::vector<int>>& gemm_levels() {
+  static const std::vector<std::vector<int>> l = {
+      {G1_Q, G2A},
+      {G2B, G9, G8, G14, G17, G3, G5, G11},
+      {G10, G15, G12, G4_, G21, G22, G18},
+      {G16, G19, G13, G6},
+      {G20, G7},
+      {G23},
+      {G24},
+  };
+  return l;
+}
+constexpr int kLevelXX = 2;   // Xvv, Xoo and u must be set before this level
+
+// The molecules of a batch in the order of the level tables: dealt out to the
+// 8 XCDs from the largest down, each XCD's share (a contiguous run of the
+// table) largest first, so that the shares cost alike and end in short tiles.
+static std::vector<int> level_order(const Batch& b) {
+  std::vector<int> by(b.nm), out;
+  for (int k = 0; k < b.nm; ++k) by[k] = k;
+  auto work = [&](int k) { return (double)b.o[k] * b.o[k] * b.v[k] * b.v[k] * b.n[k] * b.n[k]; };
+  std::stable_sort(by.begin(), by.end(), [&](int x, int y) { return work(x) > work(y); });
+  for (int x = 0; x < 8; ++x)
+    for (int r = x; r < b.nm; r += 8) out.push_back(by[r]);
+  return out;
+}
+
+static void build_levels(Batch& b) {
+  const std::vector<int> order = level_order(b);
+  b.g1 = make_table(b, [&](int k) { return b.ops[G1_Q](b.hm[k]); }, true, 0, G1_Q);
+  b.lv.clear();
+  for (const auto& level : gemm_levels()) {
+    ProbGroups groups;
+    for (int k : order)
+      for (int op : level) {
+        GemmProb p = b.ops[op](b.hm[k]);
+        const int ts = plan_problem(b, p, k, true, 0, op, 0, false);
+        groups.add(p, ts);
+      }
+    b.lv.push_back(link_groups(b, groups));
+  }
+}
+
+// one table per contraction, for profiled solves and tuning
+static void need_op_tables(Batch& b) {
+  if (!b.it.empty()) return;
+  for (int q = 0; q < (int)b.ops.size(); ++q)
+    b.it.push_back(make_table(b, [&](int k) { return b.ops[q](b.hm[k]); }, true, 0, q));
+}
+
 // Correction-form twin of iteration GEMM `op` for molecule k: the FP64
 // problem plus its correction operands and BF16 operand copies.
 static GemmProb delta_prob(Batch& b, int op, int k) {
@@ -895,11 +1007,6 @@ static void build_delta_tables(Batch& b) {
     b.dit.push_back(make_table(b, [&](int k) { return delta_prob(b, q, k); }, true, b.mixed_bf16 ? 0 : 64,
                                b.mixed_bf16 ? kDualTuneOp + q : -1, 0, b.mixed_bf16));
 }
-
-enum ItOp {
-  G1_Q = 0, G2A, G2B, G3, G4_, G5, G6, G7, G8, G9, G10, G11, G12, G13, G14, G15, G16, G17, G18, G19, G20,
-  G21, G22, G23, G24, N_IT_OPS
-};
 
 }  // namespace hcc
 
@@ -985,7 +1092,7 @@ namespace hcc {
 
 static void launch_table(hcc_ctx* c, const GemmTable& t) {
   const TableView v = view(t);
-  HCHECK(launch_gemm_f64(v.d, v.tp, v.tiles, c->batch->dact, c->stream, t.tile));
+  HCHECK(launch_gemm_f64(v.d, v.tp, *v.xcd, c->batch->dact, c->stream, t.tile));
   if (v.red > 0) HCHECK(launch_splitk_reduce(v.d, v.rp, v.rb, v.red, c->batch->dact, c->stream));
   if (t.alt >= 0) launch_table(c, c->batch->alt[t.alt]);
 }
@@ -1009,8 +1116,12 @@ static void compact_table(Batch& b, GemmTable& t, const std::vector<int>& act, h
   int* tbeg = idx + np;
   int* rpre = tbeg + np + 1;
   int n = 0, tiles = 0, red = 0;
+  std::vector<int> ctiles;
+  std::vector<float> ccost;
   for (int q = 0; q < np; ++q) {
     if (act[t.hmol[q]] == 0) continue;
+    ctiles.push_back(t.htiles[q]);
+    ccost.push_back(t.hcost[q]);
     idx[n] = q;
     tbeg[n] = tiles;
     rpre[n] = red;
@@ -1024,6 +1135,7 @@ static void compact_table(Batch& b, GemmTable& t, const std::vector<int>& act, h
   HCHECK(launch_compact_table(t.d, t.cbuf, t.cbuf + np, t.cbuf + 2 * np + 1, n, tiles, red, t.cd, t.ctp, t.cbp, s));
   t.ctiles = tiles;
   t.cred = red;
+  t.cxcd = xcd_runs(ctiles, ccost);
 }
 
 // The FP64 residual's tables (dual = false) or the correction residual's
@@ -1039,7 +1151,7 @@ static bool compact_tables(hcc_ctx* c, bool dual, const std::vector<int>& act, i
   Batch& b = *c->batch;
   if (b.arena != nullptr || alive <= 0) return false;   // no-allocation contexts keep full tables
   int& last = dual ? b.dit_live : b.it_live;
-  std::vector<GemmTable>& tabs = dual ? b.dit : b.it;
+  std::vector<GemmTable>& tabs = dual ? b.dit : (c->prof ? b.it : b.lv);
   auto each = [&](const std::function<void(GemmTable&)>& f) {
     for (GemmTable& t : tabs)
       for (GemmTable* p = &t; p != nullptr; p = p->alt >= 0 ? &b.alt[p->alt] : nullptr) f(*p);
@@ -1090,7 +1202,7 @@ static bool compact_raggeds(hcc_ctx* c, const std::vector<int>& act, int alive) 
 // full tables and grids again (end of a solve: the energies and other callers
 // run every molecule)
 static void uncompact_tables(Batch& b) {
-  for (auto* v : {&b.it, &b.dit, &b.alt})
+  for (auto* v : {&b.it, &b.lv, &b.dit, &b.alt})
     for (GemmTable& t : *v) t.ctiles = -1;
   b.it_live = b.dit_live = 0;
   for (Batch::RgComp& r : b.rgc) *r.rg = r.full;
@@ -1181,7 +1293,8 @@ static bool take_stop(hcc_ctx* c) {
   return true;
 }
 
-// Omega1 -> w1 (without the F~_ai term), Omega2 -> w2
+// Omega1 -> w1 (without the F~_ai term), Omega2 -> w2.  While profiling every
+// contraction is launched (and timed) by itself.
 static void residual(hcc_ctx* c) {
   Batch& b = *c->batch;
   hipStream_t s = c->stream;
@@ -1190,17 +1303,19 @@ static void residual(hcc_ctx* c) {
   ew_fock_m(b.dm, b.dst, b.rgN, b.rgNN, b.nm, s);
   ew_pouter(b.dm, b.dst, b.rgN3, b.nm, s);
   prof_close(c);
-  gemm(c, b.it[G1_Q], G1_Q);
-  gemm(c, b.it[G2A], G2A);
-  gemm(c, b.it[G2B], G2B);
-  prof_open(c, kProfResidualEw);
-  ew_u(b.dm, b.dst, b.rgT2x, b.nm, s);
-  prof_close(c);
-  for (int g = G3; g <= G20; ++g) gemm(c, b.it[g], g);
-  prof_open(c, kProfResidualEw);
-  ew_init_xx(b.dm, b.dst, b.rgXX, b.nm, s);
-  prof_close(c);
-  for (int g = G21; g <= G24; ++g) gemm(c, b.it[g], g);
+  if (c->prof) need_op_tables(b);
+  for (int l = 0; l < (int)b.lv.size(); ++l) {
+    if (l == kLevelXX) {
+      prof_open(c, kProfResidualEw);
+      ew_u_xx(b.dm, b.dst, b.rgT2x, b.rgXX, s);
+      prof_close(c);
+    }
+    if (!c->prof) {
+      if (b.lv[l].nprob > 0) launch_table(c, b.lv[l]);
+      continue;
+    }
+    for (int op : gemm_levels()[l]) gemm(c, b.it[op], op);
+  }
   prof_open(c, kProfE2);
   ew_e2(b.dm, b.dst, b.rgOcc, b.nm, s);
   prof_close(c);
@@ -1257,13 +1372,9 @@ static void residual_delta(hcc_ctx* c) {
   dgemm(c, b.dit[G2A], 32 + G2A);
   dgemm(c, b.dit[G2B], 32 + G2B);
   prof_open(c, kProfResidualEwMixed);
-  ew_u(b.ddm, b.dst, b.rgT2x, b.nm, s);
+  ew_u_xx(b.ddm, b.dst, b.rgT2x, b.rgXX, s);
   prof_close(c);
-  for (int g = G3; g <= G20; ++g) dgemm(c, b.dit[g], 32 + g);
-  prof_open(c, kProfResidualEwMixed);
-  ew_init_xx(b.ddm, b.dst, b.rgXX, b.nm, s);
-  prof_close(c);
-  for (int g = G21; g <= G24; ++g) dgemm(c, b.dit[g], 32 + g);
+  for (int g = G3; g <= G24; ++g) dgemm(c, b.dit[g], 32 + g);
   prof_open(c, kProfE2Mixed);
   mixed_e2(b.dm, b.ddm, b.dst, b.rgOcc, b.nm, s);
   prof_close(c);
@@ -1288,7 +1399,7 @@ static void precompute(hcc_ctx* c) {
   ew_dress(b.dm, b.dst, b.rgNN, b.nm, s);
   ew_pouter(b.dm, b.dst, b.rgN3, b.nm, s);
   prof_close(c);
-  gemm(c, b.it[G1_Q], 62);
+  gemm(c, b.g1, 62);
   gemm(c, b.pre[2], 63);
   prof_open(c, kProfPrecomputeEw);
   make_L(b.dm, b.rgT2, b.nm, s);
@@ -1364,6 +1475,7 @@ static void load(hcc_ctx* c, int nmol, const int* n, const int* nocc, const doub
   }
   allocate(*b, keep_mp2);
   build_tables(*b);
+  build_levels(*b);
   if (b->mixed) build_delta_tables(*b);
   // upload, transposing the column-major inputs to row-major: one staging
   // image per arena (molecule blocks at their arena offsets), one copy each;
@@ -1704,7 +1816,7 @@ int hcc_batch_triples(hcc_ctx* ctx, double* energies, double* e_t) {
   ew_dress(b.dm, b.dst, b.rgNN, b.nm, s);
   ew_pouter(b.dm, b.dst, b.rgN3, b.nm, s);
   prof_close(ctx);
-  gemm(ctx, b.it[G1_Q], 62);
+  gemm(ctx, b.g1, 62);
   gemm(ctx, b.tpre[0], 58);
   gemm(ctx, b.tpre[1], 59);
   prof_open(ctx, kProfTriplesEw);
@@ -2882,15 +2994,19 @@ int hcc_tune_gemm(hcc_ctx* ctx, int op, int tile, int ksplit, int reps, double* 
   }
   API_BEGIN
   HCHECK(hipSetDevice(ctx->device));
-  const size_t nalloc = b.allocs.size(), nalt = b.alt.size();
+  size_t nalloc = b.allocs.size(), nalt = b.alt.size();
   GemmTable t;
   if (dual)
     t = tile == 0 ? b.dit[q]
                   : make_table(b, [&](int k) { return delta_prob(b, q, k); }, true, tile, -1, ksplit > 0 ? ksplit : 1,
                                true);
-  else
-    t = tile == 0 ? b.it[q]
-                  : make_table(b, [&](int k) { return b.ops[q](b.hm[k]); }, true, tile, -1, ksplit > 0 ? ksplit : 1);
+  else if (tile == 0) {
+    need_op_tables(b);
+    nalloc = b.allocs.size();
+    nalt = b.alt.size();
+    t = b.it[q];
+  } else
+    t = make_table(b, [&](int k) { return b.ops[q](b.hm[k]); }, true, tile, -1, ksplit > 0 ? ksplit : 1);
   auto run = [&]() {
     if (!dual) {
       launch_table(ctx, t);
@@ -2939,9 +3055,9 @@ int hcc_gemm_flops(hcc_ctx* ctx, double* per_iteration, double* per_solve_setup)
     if (t.alt >= 0) table_flops(b.alt[t.alt], acc);
   };
   std::vector<double> it(b.nm, 0.0), pre(b.nm, 0.0);
-  for (const auto& t : b.it) table_flops(t, it);
+  for (const auto& t : b.lv) table_flops(t, it);
   for (const auto& t : b.pre) table_flops(t, pre);
-  table_flops(b.it[G1_Q], pre);
+  table_flops(b.g1, pre);
   for (int k = 0; k < b.nm; ++k) {
     if (per_iteration) per_iteration[k] = it[k];
     if (per_solve_setup) per_solve_setup[k] = pre[k];
@@ -3097,7 +3213,7 @@ int hcc_selftest_gemm(int m, int n, int k, const double* A, const double* B, dou
     HCHECK(hipMemcpy(dp, &p, sizeof(p), hipMemcpyHostToDevice));
     HCHECK(hipMalloc(&dtp, sizeof(int) * tiles));
     HCHECK(hipMemset(dtp, 0, sizeof(int) * tiles));
-    HCHECK(launch_gemm_f64(dp, dtp, tiles, nullptr, nullptr, 64));
+    HCHECK(launch_gemm_f64(dp, dtp, xcd_runs({tiles}, {1.f}), nullptr, nullptr, 64));
     HCHECK(hipDeviceSynchronize());
     HCHECK(hipMemcpy(C, dC, sizeof(double) * m * n, hipMemcpyDeviceToHost));
   } catch (const HipError&) {

@@ -3,7 +3,7 @@ just short of full or nearly empty, against the oracle or plain FP64 numpy."""
 import numpy as np
 import pytest
 
-from helios_amd import capi, molecules as M
+from helios_amd import capi, molecules as M, ppp
 from oracle import ccsd, mlp, triples as T
 from tests._molprep import prepare, random_amplitudes
 
@@ -116,3 +116,25 @@ def test_epoch_loss_with_a_short_last_batch():
     tr.close()
     assert moved < 1e-29
     assert np.abs(hist - loss).max() <= 1e-6 * loss
+
+
+@pytest.mark.parametrize("o,v", [(1, 1), (1, 4), (3, 4), (4, 3), (5, 9), (8, 8), (7, 17), (16, 17), (33, 5), (5, 33)])
+def test_residual_at_ragged_sizes(o, v):
+    """Residuals at random amplitudes where n_occ and n_virt differ in parity and
+    size (runs of odd radix along K, single rows and columns, tiles of 16, 32,
+    33 and 64), with the tolerance of the residual parity test: 1e-11."""
+    m = M.polyene(o + v)
+    G, _, hk = ppp.model(m.coords, m.bonds)
+    e, C = np.linalg.eigh(hk)   # any orthonormal orbitals with a diagonal Fock matrix will do
+    F = np.diag(e)
+    t1, t2 = random_amplitudes(o, v, 10 * o + v)
+    B = ccsd.Blocks(ccsd.rint(C, G), o)
+    r1, r2 = ccsd.singles(F, B, t1, t2), ccsd.doubles(F, B, t1, t2)
+    ctx = capi.Context(0, capi.HCC_FP64, 20)
+    ctx.set_molecule(C, F, G, o, 0.0)
+    ctx.set_amplitudes(t1, t2)
+    d1, d2 = ctx.residual()
+    ctx.close()
+    print(o, v, np.abs(d1 - r1).max(), np.abs(d2 - r2).max())
+    assert np.abs(d1 - r1).max() < 1e-11 * max(1.0, np.abs(r1).max())
+    assert np.abs(d2 - r2).max() < 1e-11 * max(1.0, np.abs(r2).max())
