@@ -163,6 +163,50 @@ struct DevBuf {
 };
 
 // ---------------------------------------------------------------------------
+// device memory of a context
+// ---------------------------------------------------------------------------
+// Blocks that a replaced batch leaves for the next one: a load of the same
+// shapes then allocates nothing.  (hipMalloc and hipFree of the arenas of a
+// 1024-molecule batch took up to 370 ms of a 437 ms device-SCF load.)  The
+// blocks not taken by the time a load ends are freed, so a context never holds
+// more than its batch between calls, and running out of memory during a load
+// frees them first.
+struct DevBlock {
+  void* p;
+  size_t bytes;
+};
+struct DevPool {
+  std::vector<DevBlock> spare;
+  ~DevPool() { trim(); }
+  void trim() {
+    for (const DevBlock& b : spare) (void)hipFree(b.p);
+    spare.clear();
+  }
+  DevBlock take(size_t bytes) {
+    size_t best = spare.size();
+    for (size_t q = 0; q < spare.size(); ++q)
+      if (spare[q].bytes >= bytes && spare[q].bytes - bytes <= bytes / 8 + 65536 &&
+          (best == spare.size() || spare[q].bytes < spare[best].bytes))
+        best = q;
+    if (best < spare.size()) {
+      const DevBlock b = spare[best];
+      spare[best] = spare.back();
+      spare.pop_back();
+      return b;
+    }
+    void* p = nullptr;
+    hipError_t e = hipMalloc(&p, bytes);
+    if (e == hipErrorOutOfMemory && !spare.empty()) {
+      (void)hipGetLastError();
+      trim();
+      e = hipMalloc(&p, bytes);
+    }
+    if (e != hipSuccess) throw HipError{e, "hipMalloc"};
+    return {p, bytes};
+  }
+};
+
+// ---------------------------------------------------------------------------
 // batch
 // ---------------------------------------------------------------------------
 struct Batch {
@@ -175,7 +219,8 @@ struct Batch {
   Mol* dm = nullptr;
   State* dst = nullptr;
   int* dact = nullptr;
-  std::vector<void*> allocs;
+  DevPool* pool = nullptr;          // the context's (null with `arena`)
+  std::vector<DevBlock> allocs;
   Ragged rgNN, rgN3, rgT2, rgT2S, rgOV, rgXX, rgND, rgN, rgP2, rgPairL, rgPairBlk, rgOcc;
   bool guess_large = false;   // some molecule has v > 32 (pairwise learned-guess kernel)
   Ragged rgT2x, rgT2Sx;   // rgT2, rgT2S with kEwItems elements per thread
@@ -255,17 +300,31 @@ struct Batch {
   int tcount[3] = {0, 0, 0};   // work items per size class
   int tcus = 1;
 
-  // device memory: hipMalloc per buffer, or -- when `arena` is set (the
+  // device memory: blocks of the context's pool, or -- when `arena` is set (the
   // no-allocation entry point) -- consecutive 256-byte aligned pieces of a
   // caller-owned region of arena_cap bytes, never freed here
   char* arena = nullptr;
   size_t arena_cap = 0, arena_used = 0;
+  // requests of up to kSmall bytes come from chunks; while a load runs, what is
+  // uploaded into them is collected in a host image, copied once per chunk by
+  // flush_uploads (a load makes about a hundred small tables)
+  static constexpr size_t kSmall = 1 << 20, kChunk = 8 << 20;
+  struct Chunk {
+    char* dev;
+    size_t used;
+    std::vector<char> image;
+  };
+  std::vector<Chunk> chunks;
+  bool collecting = false;
+  // host copies of the elementwise grids' block prefixes
+  std::map<const int*, std::vector<int>> rg_pre;
 
   ~Batch() { release(); }
   void release() {
-    if (arena == nullptr)
-      for (void* p : allocs) (void)hipFree(p);
+    if (arena == nullptr && pool != nullptr)
+      for (const DevBlock& b : allocs) pool->spare.push_back(b);
     allocs.clear();
+    chunks.clear();
     if (dlr_space) (void)hipFree(dlr_space);
     if (dlr_stage) (void)hipFree(dlr_stage);
     dlr_space = nullptr;
@@ -279,21 +338,55 @@ struct Batch {
   }
   template <class T>
   T* dalloc(size_t count) {
-    void* p = nullptr;
     if (count == 0) count = 1;
+    const size_t bytes = (count * sizeof(T) + 255) / 256 * 256;
     if (arena != nullptr) {
-      const size_t bytes = (count * sizeof(T) + 255) / 256 * 256;
       if (bytes > arena_cap - arena_used)
         throw std::string("molecule too large for the no-allocation scratch region (") +
             std::to_string(arena_cap >> 20) + " MiB): needs more than " + std::to_string((arena_used + bytes) >> 20) +
             " MiB";
-      p = arena + arena_used;
+      void* p = arena + arena_used;
       arena_used += bytes;
       return static_cast<T*>(p);
     }
-    HCHECK(hipMalloc(&p, count * sizeof(T)));
-    allocs.push_back(p);
-    return static_cast<T*>(p);
+    if (bytes <= kSmall) {
+      if (chunks.empty() || chunks.back().used + bytes > kChunk) {
+        const DevBlock c = pool->take(kChunk);
+        allocs.push_back(c);
+        chunks.push_back(Chunk{static_cast<char*>(c.p), 0, {}});
+      }
+      Chunk& c = chunks.back();
+      void* p = c.dev + c.used;
+      c.used += bytes;
+      return static_cast<T*>(p);
+    }
+    allocs.push_back(pool->take(bytes));
+    return static_cast<T*>(allocs.back().p);
+  }
+  template <class T>
+  T* upload(const T* src, size_t count) {
+    T* p = dalloc<T>(count);
+    if (count == 0) return p;
+    if (collecting && count * sizeof(T) <= kSmall) {   // its piece ends the last chunk
+      Chunk& c = chunks.back();
+      const size_t at = (size_t)(reinterpret_cast<char*>(p) - c.dev);
+      c.image.resize(c.used);
+      memcpy(c.image.data() + at, src, count * sizeof(T));
+    } else {
+      HCHECK(hipMemcpy(p, src, count * sizeof(T), hipMemcpyHostToDevice));
+    }
+    return p;
+  }
+  template <class T>
+  T* upload(const std::vector<T>& v) {
+    return upload(v.data(), v.size());
+  }
+  void flush_uploads() {
+    for (Chunk& c : chunks) {
+      if (!c.image.empty()) HCHECK(hipMemcpy(c.dev, c.image.data(), c.image.size(), hipMemcpyHostToDevice));
+      std::vector<char>().swap(c.image);
+    }
+    collecting = false;
   }
 };
 
@@ -311,14 +404,13 @@ static Ragged make_ragged(Batch& b, const std::function<long(int, int, int)>& si
     pre[k + 1] = pre[k] + (int)blocks;
   }
   Ragged r;
-  r.prefix = b.dalloc<int>(pre.size());
-  HCHECK(hipMemcpy(r.prefix, pre.data(), pre.size() * sizeof(int), hipMemcpyHostToDevice));
+  r.prefix = b.upload(pre);
   r.nblocks = pre.back();
   std::vector<int> bm(r.nblocks);
   for (int k = 0; k < b.nm; ++k)
     for (int q = pre[k]; q < pre[k + 1]; ++q) bm[q] = k;
-  r.bmol = b.dalloc<int>(bm.size());
-  HCHECK(hipMemcpy(r.bmol, bm.data(), bm.size() * sizeof(int), hipMemcpyHostToDevice));
+  r.bmol = b.upload(bm);
+  b.rg_pre[r.prefix] = std::move(pre);
   return r;
 }
 
@@ -401,15 +493,12 @@ static GemmTable build_group(Batch& b, std::vector<GemmProb> probs, int ts) {
       }
       pre[q + 1] = pre[q] + blocks;
     }
-    t.red_prefix = b.dalloc<int>(pre.size());
-    HCHECK(hipMemcpy(t.red_prefix, pre.data(), pre.size() * sizeof(int), hipMemcpyHostToDevice));
+    t.red_prefix = b.upload(pre);
     t.red_blocks = pre.back();
     std::vector<int> bp(t.red_blocks);
     for (size_t q = 0; q < probs.size(); ++q)
       for (int x = pre[q]; x < pre[q + 1]; ++x) bp[x] = (int)q;
-    t.red_bprob = b.dalloc<int>(std::max<size_t>(1, bp.size()));
-    if (!bp.empty())
-      HCHECK(hipMemcpy(t.red_bprob, bp.data(), bp.size() * sizeof(int), hipMemcpyHostToDevice));
+    t.red_bprob = b.upload(bp);
   }
   if (tiles > 0) {
     std::vector<int> tp(tiles);
@@ -417,13 +506,9 @@ static GemmTable build_group(Batch& b, std::vector<GemmProb> probs, int ts) {
       const int end = q + 1 < probs.size() ? probs[q + 1].tile_begin : tiles;
       for (int x = probs[q].tile_begin; x < end; ++x) tp[x] = (int)q;
     }
-    t.tile_prob = b.dalloc<int>(tp.size());
-    HCHECK(hipMemcpy(t.tile_prob, tp.data(), tp.size() * sizeof(int), hipMemcpyHostToDevice));
+    t.tile_prob = b.upload(tp);
   }
-  if (t.nprob) {
-    t.d = b.dalloc<GemmProb>(probs.size());
-    HCHECK(hipMemcpy(t.d, probs.data(), probs.size() * sizeof(GemmProb), hipMemcpyHostToDevice));
-  }
+  if (t.nprob) t.d = b.upload(probs);
   return t;
 }
 
@@ -633,8 +718,7 @@ static void allocate(Batch& b, bool keep_mp2) {
     M.Ov = Ov[k];
     M.t2mp2 = mp2[k];
   }
-  b.dm = b.dalloc<Mol>(b.nm);
-  HCHECK(hipMemcpy(b.dm, b.hm.data(), b.nm * sizeof(Mol), hipMemcpyHostToDevice));
+  b.dm = b.upload(b.hm);
   if (b.mixed) {
     // corrections: FP32 twins of the variable buffers; inputs, constants and the
     // DIIS storage are shared with the outer point
@@ -661,8 +745,7 @@ static void allocate(Batch& b, bool keep_mp2) {
       float* base = b.dalloc<float>(total);
       for (int k = 0; k < b.nm; ++k) b.hd[k].*(f.dmember) = base + off[k];
     }
-    b.ddm = b.dalloc<MolD>(b.nm);
-    HCHECK(hipMemcpy(b.ddm, b.hd.data(), b.nm * sizeof(MolD), hipMemcpyHostToDevice));
+    b.ddm = b.upload(b.hd);
     auto add_shadow = [&](const FieldDef& f, bool variable) {
       const Mol& first = b.hm[0];
       const Mol& last = b.hm[b.nm - 1];
@@ -673,20 +756,16 @@ static void allocate(Batch& b, bool keep_mp2) {
         sh.hoff.push_back(b.hm[k].*(f.member) - base);
         sh.hlen.push_back(f.size(b.n[k], b.o[k], b.v[k]));
       }
-      sh.doff = b.dalloc<long>(b.nm);
-      sh.dlen = b.dalloc<long>(b.nm);
+      sh.doff = b.upload(sh.hoff);
+      sh.dlen = b.upload(sh.hlen);
       sh.dpre = b.dalloc<int>(b.nm + 1);
-      HCHECK(hipMemcpy(sh.doff, sh.hoff.data(), b.nm * sizeof(long), hipMemcpyHostToDevice));
-      HCHECK(hipMemcpy(sh.dlen, sh.hlen.data(), b.nm * sizeof(long), hipMemcpyHostToDevice));
       b.shadows.push_back(std::move(sh));
     };
     for (const auto& f : variable_fields()) add_shadow(f, true);
     for (const auto& f : constant_fields()) add_shadow(f, false);
   }
-  b.dst = b.dalloc<State>(b.nm);
-  HCHECK(hipMemset(b.dst, 0, b.nm * sizeof(State)));
-  b.dact = b.dalloc<int>(b.nm);
-  HCHECK(hipMemset(b.dact, 0, b.nm * sizeof(int)));
+  b.dst = b.upload(std::vector<State>(b.nm));   // all zero
+  b.dact = b.upload(std::vector<int>(b.nm, 0));
 
   b.rgNN = make_ragged(b, sz_nn);
   b.rgN3 = make_ragged(b, sz_n3, kPItems);
@@ -727,8 +806,7 @@ static void allocate(Batch& b, bool keep_mp2) {
     Batch::RgComp c;
     c.rg = r;
     c.full = *r;
-    c.pre.resize(b.nm + 1);
-    HCHECK(hipMemcpy(c.pre.data(), r->prefix, (b.nm + 1) * sizeof(int), hipMemcpyDeviceToHost));
+    c.pre = b.rg_pre[r->prefix];
     b.rgc.push_back(std::move(c));
   }
 }
@@ -1043,6 +1121,7 @@ struct hcc_ctx {
   int projtype = 2;
   int diis = 1;
   hipStream_t stream = nullptr;
+  DevPool pool;              // device blocks between two batches (declared before what returns blocks to it)
   Batch* batch = nullptr;
   std::string err;
   bool have_guess = false;
@@ -1445,11 +1524,18 @@ bool batch_view(hcc_ctx* c, BatchView* v) {
 // never with a half-built one.
 static void load(hcc_ctx* c, int nmol, const int* n, const int* nocc, const double* C, const double* F,
                  const double* G, const double* eref, bool keep_mp2) {
+  if (c->batch != nullptr && c->arena == nullptr) HCHECK(hipStreamSynchronize(c->stream));   // its blocks may be reused
   delete c->batch;
   c->batch = nullptr;
   c->have_guess = false;
+  struct Trim {
+    DevPool& pool;
+    ~Trim() { pool.trim(); }
+  } trim{c->pool};   // after the batch is built, or has failed and returned its blocks
   std::unique_ptr<Batch> owner(new Batch());
   Batch* b = owner.get();
+  b->pool = &c->pool;
+  b->collecting = c->arena == nullptr;
   b->arena = c->arena;
   b->arena_cap = c->arena_cap;
   b->nm = nmol;
@@ -1477,6 +1563,7 @@ static void load(hcc_ctx* c, int nmol, const int* n, const int* nocc, const doub
   build_tables(*b);
   build_levels(*b);
   if (b->mixed) build_delta_tables(*b);
+  b->flush_uploads();
   // upload, transposing the column-major inputs to row-major: one staging
   // image per arena (molecule blocks at their arena offsets), one copy each;
   // a null C or F is computed on the device afterwards (hcc_batch_load_scf)
@@ -1691,8 +1778,6 @@ int hcc_batch_load_scf(hcc_ctx* ctx, int nmol, const int* n, const int* n_occ, c
     off[k] = total;
     total += (long)n[k] * n[k];
   }
-  double* dcore = b.dalloc<double>(total);
-  double* dhk = b.dalloc<double>(total);
   double* dwork = b.dalloc<double>(total);
   std::vector<double> hc(total), hh(total);
   for (int k = 0; k < nmol; ++k)
@@ -1701,13 +1786,12 @@ int hcc_batch_load_scf(hcc_ctx* ctx, int nmol, const int* n, const int* n_occ, c
         hc[off[k] + (long)r * n[k] + c] = core[off[k] + r + (long)c * n[k]];
         hh[off[k] + (long)r * n[k] + c] = huckel[off[k] + r + (long)c * n[k]];
       }
-  HCHECK(hipMemcpy(dcore, hc.data(), total * sizeof(double), hipMemcpyHostToDevice));
-  HCHECK(hipMemcpy(dhk, hh.data(), total * sizeof(double), hipMemcpyHostToDevice));
+  double* dcore = b.upload(hc);
+  double* dhk = b.upload(hh);
   std::vector<ScfInput> in(nmol);
   for (int k = 0; k < nmol; ++k) in[k] = ScfInput{dcore + off[k], dhk + off[k], dwork + off[k]};
-  ScfInput* din = b.dalloc<ScfInput>(nmol);
+  ScfInput* din = b.upload(in);
   ScfResult* dres = b.dalloc<ScfResult>(nmol);
-  HCHECK(hipMemcpy(din, in.data(), nmol * sizeof(ScfInput), hipMemcpyHostToDevice));
   HCHECK(launch_rhf(b.dm, din, nmol, nmax, scf_accuracy, scf_maxiter, 0.05, dres, ctx->stream));
   std::vector<ScfResult> res(nmol);
   HCHECK(hipMemcpyAsync(res.data(), dres, nmol * sizeof(ScfResult), hipMemcpyDeviceToHost, ctx->stream));
@@ -1776,15 +1860,12 @@ static void setup_triples(Batch& b, int device) {
     tm[k] = TripMol{M.n, M.o, M.v, 0, b.tA[k], b.tB[k], M.Gklcd, M.t1, M.t2, M.F};
   }
   HCHECK(hipDeviceGetAttribute(&b.tcus, hipDeviceAttributeMultiprocessorCount, device));
-  b.dtm = b.dalloc<TripMol>(nm);
-  b.dtrange = b.dalloc<int2>(nm);
-  b.dtri = b.dalloc<int2>(items.size());
+  b.dtm = b.upload(tm);
+  b.dtrange = b.upload(range);
+  b.dtri = b.upload(items);
   b.dtpart = b.dalloc<double>(2 * items.size());
   b.dtout = b.dalloc<double>(2 * (long)nm);
   b.dtsave = b.dalloc<int>(nm);
-  HCHECK(hipMemcpy(b.dtm, tm.data(), nm * sizeof(TripMol), hipMemcpyHostToDevice));
-  HCHECK(hipMemcpy(b.dtrange, range.data(), nm * sizeof(int2), hipMemcpyHostToDevice));
-  HCHECK(hipMemcpy(b.dtri, items.data(), items.size() * sizeof(int2), hipMemcpyHostToDevice));
 }
 
 int hcc_batch_triples(hcc_ctx* ctx, double* energies, double* e_t) {
@@ -2994,7 +3075,8 @@ int hcc_tune_gemm(hcc_ctx* ctx, int op, int tile, int ksplit, int reps, double* 
   }
   API_BEGIN
   HCHECK(hipSetDevice(ctx->device));
-  size_t nalloc = b.allocs.size(), nalt = b.alt.size();
+  // the table built below is dropped at the end of the call
+  size_t nalloc = b.allocs.size(), nalt = b.alt.size(), nchunk = b.chunks.size(), used = nchunk ? b.chunks.back().used : 0;
   GemmTable t;
   if (dual)
     t = tile == 0 ? b.dit[q]
@@ -3004,6 +3086,8 @@ int hcc_tune_gemm(hcc_ctx* ctx, int op, int tile, int ksplit, int reps, double* 
     need_op_tables(b);
     nalloc = b.allocs.size();
     nalt = b.alt.size();
+    nchunk = b.chunks.size();
+    used = nchunk ? b.chunks.back().used : 0;
     t = b.it[q];
   } else
     t = make_table(b, [&](int k) { return b.ops[q](b.hm[k]); }, true, tile, -1, ksplit > 0 ? ksplit : 1);
@@ -3033,8 +3117,10 @@ int hcc_tune_gemm(hcc_ctx* ctx, int op, int tile, int ksplit, int reps, double* 
   *ms = el / reps;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  for (size_t q = nalloc; q < b.allocs.size(); ++q) HCHECK(hipFree(b.allocs[q]));
+  for (size_t q = nalloc; q < b.allocs.size(); ++q) HCHECK(hipFree(b.allocs[q].p));
   b.allocs.resize(nalloc);
+  b.chunks.resize(nchunk);
+  if (nchunk) b.chunks.back().used = used;
   b.alt.resize(nalt);
   ctx->have_guess = false;
   API_END
