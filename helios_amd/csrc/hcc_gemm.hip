@@ -9,8 +9,8 @@
 //
 // Tile -> workgroup mapping is XCD-aware: consecutive workgroups are spread
 // round-robin over the 8 XCDs by the dispatcher, so workgroup b takes tile
-// b / 8 of XCD b % 8's contiguous run (XcdMap; equal runs in the correction
-// GEMM), which keeps a molecule's tiles (which share operands) in one L2.
+// b / 8 of XCD b % 8's contiguous run (XcdMap), which keeps a molecule's tiles
+// (which share operands) in one L2.
 #include <type_traits>
 
 #include "hcc_internal.h"
@@ -65,18 +65,30 @@ __device__ __forceinline__ int find_problem(const int* __restrict__ tile_prob, i
   return tile_prob[tile];
 }
 
-__device__ __forceinline__ int logical_tile(int total) {
-  int t8 = (total + 7) >> 3;
-  return (int)(blockIdx.x & 7) * t8 + (int)(blockIdx.x >> 3);
+// Position of tile lt of a problem of tiles_m x tiles_n tiles: bands of H tile
+// rows, column by column within a band.  An XCD runs a contiguous range of lt,
+// so the tiles it has in flight cover a block of about H x (in flight / H)
+// and share that block's operand panels in its L2; row by row they would cover
+// one or two full rows and stream all of B once per row.  Solves with rows
+// and with bands: 100 sites (40 x 40 tiles of 64) 223 and 207 ms; 120 sites in
+// mixed precision (29 x 29 tiles of 128 in the correction forms, where B's
+// panels came from memory at 2.5 TB/s) 544 and 446 ms, correction levels included.
+template <int H>
+__device__ __forceinline__ void tile_pos(int lt, int tiles_m, int tiles_n, int& tm, int& tn) {
+  const int band = lt / (H * tiles_n), r = lt - band * H * tiles_n, h = min(H, tiles_m - band * H);
+  tn = r / h;
+  tm = band * H + r - tn * h;
 }
+// band heights: the square root of the tiles an XCD's 32 CUs hold
+constexpr int kBand64 = 12, kBand128 = 8;
 
 // ---------------------------------------------------------------------------
 // FP64 kernel: output tile BM x BN, 32x32 per wave (4 waves or 1), 16-deep K
 // slabs staged through LDS.
 //
 // What bounds it: the matrix cores, and next to them the return path of the
-// vector loads -- a 64-lane 8-byte load occupies it for 32 cycles (4 lanes at
-// a time), which at 64x64 tiles is as long as the slab's matrix work.  So an
+// vector loads -- a 64-lane 8-byte load occupies it for 16 cycles, as long as
+// a 16-byte one (31 and 62 bytes a cycle).  So an
 // operand is staged in 16-byte pairs along its unit-stride dimension wherever
 // pairs exist (GemmProb::modes):
 //   mode 0  pairs along K, staged [row][k];
@@ -138,12 +150,12 @@ __device__ __forceinline__ void gemm_f64_tile(const GemmProb& P, int lt, double*
   constexpr int T = TL::kT;
   using SA = F64Stage<MA, BM, T>;
   using SB = F64Stage<MB, BN, T>;
-  const int tiles_n = (P.N + BN - 1) / BN;
-  const int tiles_mn = ((P.M + BM - 1) / BM) * tiles_n;
-  const int ks = lt / tiles_mn;
-  lt -= ks * tiles_mn;
-  const int m0 = (lt / tiles_n) * BM;
-  const int n0 = (lt % tiles_n) * BN;
+  const int tiles_n = (P.N + BN - 1) / BN, tiles_m = (P.M + BM - 1) / BM;
+  const int ks = lt / (tiles_m * tiles_n);
+  lt -= ks * tiles_m * tiles_n;
+  int tm, tn;
+  tile_pos<kBand64>(lt, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
   const int kbeg = ks * P.kchunk;
   const int kend = min(P.kpad, kbeg + P.kchunk);
   const int t = threadIdx.x;
@@ -330,33 +342,19 @@ __global__ __launch_bounds__(HCC_F64_THREADS(BM, BN)) __attribute__((amdgpu_wave
 // threads; FP64 path: BK 16 and 16x16x4 MFMA; BF16 path: BK 32 and
 // 16x16x32 MFMA with [row][k] LDS staging.
 // ---------------------------------------------------------------------------
-template <bool AKF, bool BNF, bool BF>
-struct DualCfg {
-  static constexpr int BK = BF ? 32 : 16;
-  static constexpr int T = 256;
-  static constexpr int NE = 64 * BK / T;     // elements per operand per thread per slab
-};
-
+constexpr int kDualLds64 = 64 * kPk;   // [row][k] staging; [k][row] takes less
 template <bool AKF, bool BNF>
-__global__ __launch_bounds__(256) void gemm_dual_f64(const GemmProb* __restrict__ probs,
-                                                     const int* __restrict__ tile_prob, int total_tiles,
-                                                     const int* __restrict__ active) {
+__device__ __forceinline__ void gemm_dual_f64_tile(const GemmProb& P, int lt, double* A0s, double* dAs, double* dBs,
+                                                   double* Bfs) {
   constexpr int BM = 64, BN = 64, T = 256, BK = 16, NE = 4;
   constexpr int kPa = BM + 2, kPb = BN + 2;
-  __shared__ double A0s[BM * kPk > BK * kPa ? BM * kPk : BK * kPa];
-  __shared__ double dAs[BM * kPk > BK * kPa ? BM * kPk : BK * kPa];
-  __shared__ double dBs[BN * kPk > BK * kPb ? BN * kPk : BK * kPb];
-  __shared__ double Bfs[BN * kPk > BK * kPb ? BN * kPk : BK * kPb];
-  const int tile = logical_tile(total_tiles);
-  if (tile >= total_tiles) return;
-  const GemmProb P = probs[find_problem(tile_prob, tile)];
-  if (active != nullptr && active[P.mol] == 0) return;
-  const int tiles_n = (P.N + BN - 1) / BN;
-  const int tiles_mn = ((P.M + BM - 1) / BM) * tiles_n;
-  int lt = tile - P.tile_begin;
-  const int ks = lt / tiles_mn;
-  lt -= ks * tiles_mn;
-  const int m0 = (lt / tiles_n) * BM, n0 = (lt % tiles_n) * BN;
+  static_assert(BK * kPa <= kDualLds64 && BK * kPb <= kDualLds64, "staging fits");
+  const int tiles_n = (P.N + BN - 1) / BN, tiles_m = (P.M + BM - 1) / BM;
+  const int ks = lt / (tiles_m * tiles_n);
+  lt -= ks * tiles_m * tiles_n;
+  int tm, tn;
+  tile_pos<kBand64>(lt, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
   const int kbeg = ks * P.kchunk, kend = min(P.K, kbeg + P.kchunk);
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
@@ -470,6 +468,23 @@ __global__ __launch_bounds__(256) void gemm_dual_f64(const GemmProb* __restrict_
   }
 }
 
+__global__ __launch_bounds__(256) void gemm_dual_f64(const GemmProb* __restrict__ probs,
+                                                     const int* __restrict__ tile_prob, XcdMap xcd,
+                                                     const int* __restrict__ active) {
+  __shared__ double A0s[kDualLds64], dAs[kDualLds64], dBs[kDualLds64], Bfs[kDualLds64];
+  const int x = blockIdx.x & 7, tile = xcd.begin[x] + (int)(blockIdx.x >> 3);
+  if (tile >= xcd.begin[x + 1]) return;
+  const GemmProb P = probs[find_problem(tile_prob, tile)];
+  if (active != nullptr && active[P.mol] == 0) return;
+  const int lt = tile - P.tile_begin;
+  switch (P.modes & 3) {   // uniform over the workgroup
+    case 0: gemm_dual_f64_tile<false, false>(P, lt, A0s, dAs, dBs, Bfs); break;
+    case 1: gemm_dual_f64_tile<true, false>(P, lt, A0s, dAs, dBs, Bfs); break;
+    case 2: gemm_dual_f64_tile<false, true>(P, lt, A0s, dAs, dBs, Bfs); break;
+    default: gemm_dual_f64_tile<true, true>(P, lt, A0s, dAs, dBs, Bfs); break;
+  }
+}
+
 // HA / HB: the operand has a correction (dA / dB non-null for every problem
 // of the table).  A constant A needs only A0 dB, a constant B only dA B0.
 //
@@ -506,35 +521,26 @@ constexpr int kDualBK = 32;   // 64-deep slabs measured slower (K padding of the
 // after the current one's matrix-core work instead of during it; the staging
 // registers are then dead during that work, which lets six waves share a SIMD
 // (a one- or two-slab tile is mostly fixed latency, hidden by more tiles per CU)
+constexpr int kDualLD = kDualBK + 8;   // LDS pitch of a staged row
+constexpr int kDualKT = 512;           // K-table chunk
 template <bool AKF, bool BNF, bool HA, bool HB, int TS, bool SK>
-__global__ __launch_bounds__(TS * 4) __attribute__((amdgpu_waves_per_eu(SK ? 6 : 4, 8))) void gemm_dual_bf16(
-    const GemmProb* __restrict__ probs, const int* __restrict__ tile_prob, int total_tiles,
-    const int* __restrict__ active) {
-  constexpr int BK = kDualBK, BM = TS, BN = TS, T = TS * 4, LD = BK + 8, NE = 8;
+__device__ __forceinline__ void gemm_dual_tile(const GemmProb& P, int lt, __bf16* A0s, __bf16* dAs, __bf16* dBs,
+                                               __bf16* Bfs, int* koffA, int* koffB) {
+  constexpr int BK = kDualBK, BM = TS, BN = TS, T = TS * 4, LD = kDualLD, NE = 8;
   constexpr int FM = 2, FN = TS / 32;   // 16x16 blocks per wave along M and N
-  constexpr int KT = 512;               // K-table chunk
+  constexpr int KT = kDualKT;
   constexpr bool KA = AKF, KB = !BNF;   // operand K-contiguous in memory
   static_assert(BM * BK == NE * T, "staging covers the slab");
   using SA = Stage<KA, BK, BM, T>;
   using SB = Stage<KB, BK, BN, T>;
   typedef float f2 __attribute__((ext_vector_type(2)));
   typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-  __shared__ __attribute__((aligned(16))) __bf16 A0s[BM * LD];
-  __shared__ __attribute__((aligned(16))) __bf16 dAs[BM * LD];
-  __shared__ __attribute__((aligned(16))) __bf16 dBs[BN * LD];
-  __shared__ __attribute__((aligned(16))) __bf16 Bfs[BN * LD];
-  __shared__ int koffA[KT + BK];
-  __shared__ int koffB[KT + BK];
-  const int tile = logical_tile(total_tiles);
-  if (tile >= total_tiles) return;
-  const GemmProb P = probs[find_problem(tile_prob, tile)];
-  if (active != nullptr && active[P.mol] == 0) return;
-  const int tiles_n = (P.N + BN - 1) / BN;
-  const int tiles_mn = ((P.M + BM - 1) / BM) * tiles_n;
-  int lt = tile - P.tile_begin;
-  const int ks = lt / tiles_mn;
-  lt -= ks * tiles_mn;
-  const int m0 = (lt / tiles_n) * BM, n0 = (lt % tiles_n) * BN;
+  const int tiles_n = (P.N + BN - 1) / BN, tiles_m = (P.M + BM - 1) / BM;
+  const int ks = lt / (tiles_m * tiles_n);
+  lt -= ks * tiles_m * tiles_n;
+  int tm, tn;
+  tile_pos<TS == 128 ? kBand128 : kBand64>(lt, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
   const int kbeg = ks * P.kchunk, kend = min(P.K, kbeg + P.kchunk);
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   // waves: 2 along N (32 FN columns each), T / 128 along M (32 rows each)
@@ -674,43 +680,63 @@ __global__ __launch_bounds__(TS * 4) __attribute__((amdgpu_waves_per_eu(SK ? 6 :
   }
 }
 
-hipError_t launch_gemm_dual(const GemmProb* probs, const int* tp, int total_tiles, const int* active,
-                            hipStream_t s, int flags, int bf16, int tile) {
-  if (total_tiles <= 0) return hipSuccess;
-  const int grid = ((total_tiles + 7) / 8) * 8;
-  if (bf16) {
-#define HCC_DUAL16(AK, BN, TS, SK)                                                                      \
-  switch ((flags >> 2) & 3) {                                                                           \
-    case 1: hipLaunchKernelGGL((gemm_dual_bf16<AK, BN, true, false, TS, SK>), dim3(grid), dim3(4 * TS), 0, s, probs, tp, total_tiles, active); break; \
-    case 2: hipLaunchKernelGGL((gemm_dual_bf16<AK, BN, false, true, TS, SK>), dim3(grid), dim3(4 * TS), 0, s, probs, tp, total_tiles, active); break; \
-    case 3: hipLaunchKernelGGL((gemm_dual_bf16<AK, BN, true, true, TS, SK>), dim3(grid), dim3(4 * TS), 0, s, probs, tp, total_tiles, active); break; \
-    default: return hipErrorInvalidValue; /* both operands constant: not a correction product */     \
+// One launch per tile kind runs problems of every layout and operand kind
+// (GemmProb::modes, uniform over a workgroup).
+template <int TS, bool SK>
+__global__ __launch_bounds__(TS * 4) __attribute__((amdgpu_waves_per_eu(SK ? 6 : 4, 8))) void gemm_dual_bf16(
+    const GemmProb* __restrict__ probs, const int* __restrict__ tile_prob, XcdMap xcd,
+    const int* __restrict__ active) {
+  __shared__ __attribute__((aligned(16))) __bf16 A0s[TS * kDualLD];
+  __shared__ __attribute__((aligned(16))) __bf16 dAs[TS * kDualLD];
+  __shared__ __attribute__((aligned(16))) __bf16 dBs[TS * kDualLD];
+  __shared__ __attribute__((aligned(16))) __bf16 Bfs[TS * kDualLD];
+  __shared__ int koffA[kDualKT + kDualBK];
+  __shared__ int koffB[kDualKT + kDualBK];
+  const int x = blockIdx.x & 7, tile = xcd.begin[x] + (int)(blockIdx.x >> 3);
+  if (tile >= xcd.begin[x + 1]) return;
+  const GemmProb P = probs[find_problem(tile_prob, tile)];
+  if (active != nullptr && active[P.mol] == 0) return;
+  const int lt = tile - P.tile_begin;
+#define HCC_DUAL_TILE(AK, BN, HA, HB) \
+  case AK + 2 * BN + 4 * HA + 8 * HB: gemm_dual_tile<AK, BN, HA, HB, TS, SK>(P, lt, A0s, dAs, dBs, Bfs, koffA, koffB); break;
+#define HCC_DUAL_LAYOUTS(HA, HB) \
+  HCC_DUAL_TILE(0, 0, HA, HB) HCC_DUAL_TILE(1, 0, HA, HB) HCC_DUAL_TILE(0, 1, HA, HB) HCC_DUAL_TILE(1, 1, HA, HB)
+  switch (P.modes) {
+    HCC_DUAL_LAYOUTS(1, 0)
+    HCC_DUAL_LAYOUTS(0, 1)
+    HCC_DUAL_LAYOUTS(1, 1)
   }
-#define HCC_DUAL16_T(TS, SK)                           \
-    switch (flags & 3) {                               \
-      case 0: HCC_DUAL16(false, false, TS, SK) break;  \
-      case 1: HCC_DUAL16(true, false, TS, SK) break;   \
-      case 2: HCC_DUAL16(false, true, TS, SK) break;   \
-      default: HCC_DUAL16(true, true, TS, SK) break;   \
-    }
-    // flag 16: every problem of the table has K <= 2 slabs (short-K variant)
-    const bool sk = (flags & 16) != 0;
-    if (tile == 64 && sk) { HCC_DUAL16_T(64, true) }
-    else if (tile == 64) { HCC_DUAL16_T(64, false) }
-    else if (tile == 32 && sk) { HCC_DUAL16_T(32, true) }
-    else if (tile == 32) { HCC_DUAL16_T(32, false) }
-    else if (tile == 256) { HCC_DUAL16_T(128, false) }
-    else return hipErrorInvalidValue;
-#undef HCC_DUAL16_T
-#undef HCC_DUAL16
-  } else {
+#undef HCC_DUAL_LAYOUTS
+#undef HCC_DUAL_TILE
+}
+
+static int longest_run(const XcdMap& xcd) {
+  int longest = 0;
+  for (int x = 0; x < 8; ++x) longest = longest > xcd.begin[x + 1] - xcd.begin[x] ? longest : xcd.begin[x + 1] - xcd.begin[x];
+  return longest;
+}
+
+template <int TS, bool SK>
+static void launch_dual(const GemmProb* probs, const int* tp, const XcdMap& xcd, const int* active, hipStream_t s) {
+  hipLaunchKernelGGL((gemm_dual_bf16<TS, SK>), dim3(8 * longest_run(xcd)), dim3(4 * TS), 0, s, probs, tp, xcd, active);
+}
+
+hipError_t launch_gemm_dual(const GemmProb* probs, const int* tp, const XcdMap& xcd, const int* active, hipStream_t s,
+                            bool bf16, int tile, bool short_k) {
+  if (longest_run(xcd) <= 0) return hipSuccess;
+  if (!bf16) {
     if (tile != 64) return hipErrorInvalidValue;
-    switch (flags & 3) {
-      case 0: hipLaunchKernelGGL((gemm_dual_f64<false, false>), dim3(grid), dim3(256), 0, s, probs, tp, total_tiles, active); break;
-      case 1: hipLaunchKernelGGL((gemm_dual_f64<true, false>), dim3(grid), dim3(256), 0, s, probs, tp, total_tiles, active); break;
-      case 2: hipLaunchKernelGGL((gemm_dual_f64<false, true>), dim3(grid), dim3(256), 0, s, probs, tp, total_tiles, active); break;
-      default: hipLaunchKernelGGL((gemm_dual_f64<true, true>), dim3(grid), dim3(256), 0, s, probs, tp, total_tiles, active); break;
-    }
+    hipLaunchKernelGGL(gemm_dual_f64, dim3(8 * longest_run(xcd)), dim3(256), 0, s, probs, tp, xcd, active);
+  } else if (tile == 64) {
+    if (short_k) launch_dual<64, true>(probs, tp, xcd, active, s);
+    else launch_dual<64, false>(probs, tp, xcd, active, s);
+  } else if (tile == 32) {
+    if (short_k) launch_dual<32, true>(probs, tp, xcd, active, s);
+    else launch_dual<32, false>(probs, tp, xcd, active, s);
+  } else if (tile == 256) {
+    launch_dual<128, false>(probs, tp, xcd, active, s);
+  } else {
+    return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
@@ -806,20 +832,17 @@ void set_f64_modes(GemmProb& p) {
 }
 
 template <int BM, int BN>
-static void launch_f64(const GemmProb* probs, const int* tp, const XcdMap& xcd, int longest, const int* active,
-                       hipStream_t s) {
-  hipLaunchKernelGGL((gemm_f64_kernel<BM, BN>), dim3(8 * longest), dim3(HCC_F64_THREADS(BM, BN)), 0, s, probs, tp, xcd,
+static void launch_f64(const GemmProb* probs, const int* tp, const XcdMap& xcd, const int* active, hipStream_t s) {
+  hipLaunchKernelGGL((gemm_f64_kernel<BM, BN>), dim3(8 * longest_run(xcd)), dim3(HCC_F64_THREADS(BM, BN)), 0, s, probs, tp, xcd,
                      active);
 }
 
 hipError_t launch_gemm_f64(const GemmProb* probs, const int* tile_prob, const XcdMap& xcd, const int* active,
                            hipStream_t s, int tile) {
-  int longest = 0;
-  for (int x = 0; x < 8; ++x) longest = longest > xcd.begin[x + 1] - xcd.begin[x] ? longest : xcd.begin[x + 1] - xcd.begin[x];
-  if (longest <= 0) return hipSuccess;
-  if (tile == 32) launch_f64<32, 32>(probs, tile_prob, xcd, longest, active, s);
-  else if (tile == 128) launch_f64<128, 32>(probs, tile_prob, xcd, longest, active, s);
-  else launch_f64<64, 64>(probs, tile_prob, xcd, longest, active, s);
+  if (longest_run(xcd) <= 0) return hipSuccess;
+  if (tile == 32) launch_f64<32, 32>(probs, tile_prob, xcd, active, s);
+  else if (tile == 128) launch_f64<128, 32>(probs, tile_prob, xcd, active, s);
+  else launch_f64<64, 64>(probs, tile_prob, xcd, active, s);
   return hipGetLastError();
 }
 

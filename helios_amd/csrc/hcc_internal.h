@@ -63,8 +63,9 @@ struct GemmProb {
   int b_nfast;      // 1: B's unit stride runs along N, 0: along K
   int ksplit;       // number of K chunks (1: no split)
   int kchunk;       // K range of one chunk (multiple of the K tile), in kpad's enumeration
-  // FP64 kernel: staging modes of A and B (3 MA + MB, see gemm_f64_kernel), and
-  // the enumeration of K with one padding element behind every run of krun
+  // FP64 kernel: staging modes of A and B (3 MA + MB, see gemm_f64_kernel);
+  // correction kernels: a_kfast | b_nfast << 1 | (dA != 0) << 2 | (dB != 0) << 3.
+  // FP64 kernel: the enumeration of K with one padding element behind every run of krun
   // (0: no such runs), kpad elements long; irun = 1 / (krun + 1)
   int modes;
   int krun, kpad;
@@ -102,8 +103,9 @@ void set_f64_modes(GemmProb& p);
 // correction-form GEMM (see GemmProb::dA/dB); bf16 = 1 rounds the operands to
 // BF16 for V_MFMA_F32_16X16X32_BF16 (FP32 accumulation; tile kinds 32, 64 and
 // 256 = 128x128 output tiles), 0 keeps FP64 (tile kind 64 only)
-hipError_t launch_gemm_dual(const GemmProb* probs, const int* tile_prob, int total_tiles, const int* active,
-                            hipStream_t s, int flags, int bf16, int tile);
+// short_k: no problem has K above 64 (a variant with more waves in flight)
+hipError_t launch_gemm_dual(const GemmProb* probs, const int* tile_prob, const XcdMap& xcd, const int* active,
+                            hipStream_t s, bool bf16, int tile, bool short_k);
 // C = alpha * sum_k ws_k + beta * C for the split problems of a table;
 // prefix: block prefix over the table's problems (256 elements per block),
 // block_prob: problem index of every reduction block

@@ -63,7 +63,7 @@ struct GemmTable {
   int red_blocks = 0;
   int tile = 64;               // output tile edge (64 or 32)
   int alt = -1;                // second part of the same contraction (other tile edge), index in Batch::alt
-  int flags = 3;               // a_kfast | b_nfast << 1 | (dA != 0) << 2 | (dB != 0) << 3 | (K <= 64) << 4
+  bool short_k = false;        // no problem has K (a K chunk) above 64
   // compaction to the molecules still running (compact_tables): per problem
   // its molecule, tiles and split-K reduction blocks; the compacted copies of
   // the problems, the tile and reduction-block maps, and the uploaded lists
@@ -254,7 +254,7 @@ struct Batch {
   std::vector<MolD> hd;   // FP32 corrections (variable buffers) + shared FP64 inputs
   MolD* ddm = nullptr;
   std::vector<std::function<GemmProb(const Mol&)>> ops;
-  std::vector<GemmTable> dit;
+  std::vector<GemmTable> dlv, dit;   // per dependency level, per contraction (as lv and it)
   // (T): undressed integral blocks (xp|yd), (ql|rz), their GEMM tables and the work items
   std::vector<double*> tA, tB;
   std::vector<GemmTable> tpre;
@@ -440,6 +440,11 @@ static void force_split(GemmProb& p, int ks) {
   }
 }
 
+// layouts and changing operands of a correction-form problem
+static void set_dual_modes(GemmProb& p) {
+  p.modes = p.a_kfast | (p.b_nfast << 1) | ((p.dA != nullptr) << 2) | ((p.dB != nullptr) << 3);
+}
+
 // One launchable table from problems that share the tile edge `ts` (their
 // ksplit / kchunk already chosen).
 static GemmTable build_group(Batch& b, std::vector<GemmProb> probs, int ts) {
@@ -452,6 +457,7 @@ static GemmTable build_group(Batch& b, std::vector<GemmProb> probs, int ts) {
     tiles += tm * p.tiles_n * p.ksplit;
     p.a_kfast = unit_cols(p.A) ? 1 : (unit_rows(p.A) ? 0 : 1);
     p.b_nfast = unit_cols(p.B) ? 1 : (unit_rows(p.B) ? 0 : 1);
+    if (p.Cd != nullptr) set_dual_modes(p);
     if (p.ksplit > 1) ws_total += (long)p.ksplit * p.M * p.N;
   }
   GemmTable t;
@@ -466,19 +472,9 @@ static GemmTable build_group(Batch& b, std::vector<GemmProb> probs, int ts) {
     t.hcost.push_back((float)(p.kchunk + 96));
   }
   t.xcd = xcd_runs(t.htiles, t.hcost);
-  if (!probs.empty()) {
-    // the staging layout is a performance choice only (addressing is general):
-    // take the largest problem's unit-stride flags for the whole table
-    size_t big = 0;
-    for (size_t q = 1; q < probs.size(); ++q)
-      if ((double)probs[q].M * probs[q].N * probs[q].K > (double)probs[big].M * probs[big].N * probs[big].K) big = q;
-    t.flags = probs[big].a_kfast | (probs[big].b_nfast << 1) | ((probs[big].dA != nullptr) << 2) |
-              ((probs[big].dB != nullptr) << 3);
-    // short-K variant of the correction GEMM when no problem has more than two 32-deep slabs
-    int kmax = 0;
-    for (const GemmProb& p : probs) kmax = std::max(kmax, p.kchunk);
-    if (kmax <= 64) t.flags |= 16;
-  }
+  // short-K variant of the correction GEMM when no problem has more than two 32-deep slabs
+  t.short_k = true;
+  for (const GemmProb& p : probs) t.short_k = t.short_k && p.kchunk <= 64;
   if (ws_total > 0) {
     double* ws = b.dalloc<double>(ws_total);
     long off = 0;
@@ -1007,7 +1003,8 @@ enum ItOp {
 // molecule: 1600 tiles on 256 CUs, 45-53 TF/s alone).  Solves with one launch
 // per contraction and with levels: octatetraene 6.7 and 4.1 ms, 25 x 14 sites
 // 13.0 and 7.5 ms, 100 sites 287 and 223 ms, 512 ragged molecules 305 and
-// 285 ms.
+// 285 ms; with the correction forms in levels as well, 2048 ragged molecules
+// in mixed precision 863 and 840 ms.
 static const std::vector<std::vector<int>>& gemm_levels() {
   static const std::vector<std::vector<int>> l = {
       {G1_Q, G2A},
@@ -1021,6 +1018,7 @@ static const std::vector<std::vector<int>>& gemm_levels() {
   return l;
 }
 constexpr int kLevelXX = 2;   // Xvv, Xoo and u must be set before this level
+constexpr int kDualTuneOp = 100;   // tuning keys of the correction forms: kDualTuneOp + op
 
 // The molecules of a batch in the order of the level tables: dealt out to the
 // 8 XCDs from the largest down, each XCD's share (a contiguous run of the
@@ -1035,20 +1033,26 @@ static std::vector<int> level_order(const Batch& b) {
   return out;
 }
 
-static void build_levels(Batch& b) {
+static std::vector<GemmTable> level_tables(Batch& b, bool dual, const std::function<GemmProb(int, int)>& build) {
   const std::vector<int> order = level_order(b);
-  b.g1 = make_table(b, [&](int k) { return b.ops[G1_Q](b.hm[k]); }, true, 0, G1_Q);
-  b.lv.clear();
+  const bool exact = dual && !b.mixed_bf16;   // FP64 corrections: 64x64 tiles only
+  std::vector<GemmTable> out;
   for (const auto& level : gemm_levels()) {
     ProbGroups groups;
     for (int k : order)
       for (int op : level) {
-        GemmProb p = b.ops[op](b.hm[k]);
-        const int ts = plan_problem(b, p, k, true, 0, op, 0, false);
+        GemmProb p = build(op, k);
+        const int ts = plan_problem(b, p, k, true, exact ? 64 : 0, exact ? -1 : (dual ? kDualTuneOp : 0) + op, 0, dual);
         groups.add(p, ts);
       }
-    b.lv.push_back(link_groups(b, groups));
+    out.push_back(link_groups(b, groups));
   }
+  return out;
+}
+
+static void build_levels(Batch& b) {
+  b.g1 = make_table(b, [&](int k) { return b.ops[G1_Q](b.hm[k]); }, true, 0, G1_Q);
+  b.lv = level_tables(b, false, [&](int op, int k) { return b.ops[op](b.hm[k]); });
 }
 
 // one table per contraction, for profiled solves and tuning
@@ -1074,13 +1078,14 @@ static GemmProb delta_prob(Batch& b, int op, int k) {
   return p;
 }
 
-// Tuning keys of the correction-form tables: kDualTuneOp + op.
-constexpr int kDualTuneOp = 100;
-
 // correction-form twins of the iteration GEMMs (BF16 tiles chosen per
 // problem, or FP64 64x64 tiles in exact mode)
-static void build_delta_tables(Batch& b) {
+static void build_delta_levels(Batch& b) {
   b.dit.clear();
+  b.dlv = level_tables(b, true, [&](int op, int k) { return delta_prob(b, op, k); });
+}
+static void need_delta_op_tables(Batch& b) {
+  if (!b.dit.empty()) return;
   for (int q = 0; q < (int)b.ops.size(); ++q)
     b.dit.push_back(make_table(b, [&](int k) { return delta_prob(b, q, k); }, true, b.mixed_bf16 ? 0 : 64,
                                b.mixed_bf16 ? kDualTuneOp + q : -1, 0, b.mixed_bf16));
@@ -1230,7 +1235,7 @@ static bool compact_tables(hcc_ctx* c, bool dual, const std::vector<int>& act, i
   Batch& b = *c->batch;
   if (b.arena != nullptr || alive <= 0) return false;   // no-allocation contexts keep full tables
   int& last = dual ? b.dit_live : b.it_live;
-  std::vector<GemmTable>& tabs = dual ? b.dit : (c->prof ? b.it : b.lv);
+  std::vector<GemmTable>& tabs = dual ? (c->prof ? b.dit : b.dlv) : (c->prof ? b.it : b.lv);
   auto each = [&](const std::function<void(GemmTable&)>& f) {
     for (GemmTable& t : tabs)
       for (GemmTable* p = &t; p != nullptr; p = p->alt >= 0 ? &b.alt[p->alt] : nullptr) f(*p);
@@ -1281,7 +1286,7 @@ static bool compact_raggeds(hcc_ctx* c, const std::vector<int>& act, int alive) 
 // full tables and grids again (end of a solve: the energies and other callers
 // run every molecule)
 static void uncompact_tables(Batch& b) {
-  for (auto* v : {&b.it, &b.lv, &b.dit, &b.alt})
+  for (auto* v : {&b.it, &b.lv, &b.dit, &b.dlv, &b.alt})
     for (GemmTable& t : *v) t.ctiles = -1;
   b.it_live = b.dit_live = 0;
   for (Batch::RgComp& r : b.rgc) *r.rg = r.full;
@@ -1425,35 +1430,44 @@ static void run_iteration(hcc_ctx* c, const Params& prm, const int* stop) {
   HCHECK(hipGetLastError());
 }
 
-static void dgemm(hcc_ctx* c, const GemmTable& t, int id) {
-  if (t.nprob == 0) return;
-  if (c->prof) {
-    c->prof_launches += table_parts(c, t);
-    c->prof_op_launches[id] += table_parts(c, t);
-  }
-  prof_open(c, id);
+static void launch_delta_table(hcc_ctx* c, const GemmTable& t) {
   for (const GemmTable* p = &t; p != nullptr; p = p->alt >= 0 ? &c->batch->alt[p->alt] : nullptr) {
+    if (p->nprob == 0) continue;
     const TableView v = view(*p);
-    HCHECK(launch_gemm_dual(v.d, v.tp, v.tiles, c->batch->dact, c->stream, p->flags, c->mixed_bf16, p->tile));
+    HCHECK(launch_gemm_dual(v.d, v.tp, *v.xcd, c->batch->dact, c->stream, c->batch->mixed_bf16, p->tile, p->short_k));
     if (v.red > 0) HCHECK(launch_splitk_reduce(v.d, v.rp, v.rb, v.red, c->batch->dact, c->stream));
   }
+}
+static void dgemm(hcc_ctx* c, const GemmTable& t, int id) {
+  if (t.nprob == 0) return;
+  c->prof_launches += table_parts(c, t);
+  c->prof_op_launches[id] += table_parts(c, t);
+  prof_open(c, id);
+  launch_delta_table(c, t);
   prof_close(c);
 }
 
-// correction residual dOmega at (t0 + dt): every step in correction form
+// correction residual dOmega at (t0 + dt): every step in correction form, in
+// the levels of residual()
 static void residual_delta(hcc_ctx* c) {
   Batch& b = *c->batch;
   hipStream_t s = c->stream;
   prof_open(c, kProfResidualEwMixed);
   mixed_dress(b.dm, b.ddm, b.dst, b.rgNN, b.rgN, b.rgN3, b.nm, s);
   prof_close(c);
-  dgemm(c, b.dit[G1_Q], 32 + G1_Q);
-  dgemm(c, b.dit[G2A], 32 + G2A);
-  dgemm(c, b.dit[G2B], 32 + G2B);
-  prof_open(c, kProfResidualEwMixed);
-  ew_u_xx(b.ddm, b.dst, b.rgT2x, b.rgXX, s);
-  prof_close(c);
-  for (int g = G3; g <= G24; ++g) dgemm(c, b.dit[g], 32 + g);
+  if (c->prof) need_delta_op_tables(b);
+  for (int l = 0; l < (int)b.dlv.size(); ++l) {
+    if (l == kLevelXX) {
+      prof_open(c, kProfResidualEwMixed);
+      ew_u_xx(b.ddm, b.dst, b.rgT2x, b.rgXX, s);
+      prof_close(c);
+    }
+    if (!c->prof) {
+      launch_delta_table(c, b.dlv[l]);
+      continue;
+    }
+    for (int op : gemm_levels()[l]) dgemm(c, b.dit[op], 32 + op);
+  }
   prof_open(c, kProfE2Mixed);
   mixed_e2(b.dm, b.ddm, b.dst, b.rgOcc, b.nm, s);
   prof_close(c);
@@ -1562,7 +1576,7 @@ static void load(hcc_ctx* c, int nmol, const int* n, const int* nocc, const doub
   allocate(*b, keep_mp2);
   build_tables(*b);
   build_levels(*b);
-  if (b->mixed) build_delta_tables(*b);
+  if (b->mixed) build_delta_levels(*b);
   b->flush_uploads();
   // upload, transposing the column-major inputs to row-major: one staging
   // image per arena (molecule blocks at their arena offsets), one copy each;
@@ -1705,7 +1719,7 @@ int hcc_set_mixed(hcc_ctx* ctx, int bf16, double kappa, int max_inner, int max_o
   API_BEGIN
   HCHECK(hipSetDevice(ctx->device));
   ctx->batch->mixed_bf16 = want != 0;
-  build_delta_tables(*ctx->batch);
+  build_delta_levels(*ctx->batch);
   API_END
 }
 
@@ -3011,15 +3025,13 @@ int hcc_gemm_flops_correction(hcc_ctx* ctx, double* per_inner_iteration) {
   API_BEGIN
   Batch& b = *ctx->batch;
   for (int k = 0; k < b.nm; ++k) per_inner_iteration[k] = 0.0;
-  std::vector<GemmProb> h;
-  std::function<void(const GemmTable&)> add = [&](const GemmTable& t) {
-    h.resize(t.nprob);
-    if (t.nprob) HCHECK(hipMemcpy(h.data(), t.d, t.nprob * sizeof(GemmProb), hipMemcpyDeviceToHost));
-    for (const auto& p : h)   // A0 dB and dA (B0 + dB): one product per changing operand
-      per_inner_iteration[p.mol] += 2.0 * p.M * (double)p.N * p.K * ((p.dA != nullptr) + (p.dB != nullptr));
-    if (t.alt >= 0) add(b.alt[t.alt]);
-  };
-  for (const auto& t : b.dit) add(t);
+  if (b.mixed)
+    for (int q = 0; q < (int)b.ops.size(); ++q)
+      for (int k = 0; k < b.nm; ++k) {
+        const GemmProb p = delta_prob(b, q, k);   // A0 dB and dA (B0 + dB): one product per changing operand
+        if (p.M > 0 && p.N > 0)
+          per_inner_iteration[k] += 2.0 * p.M * (double)p.N * p.K * ((p.dA != nullptr) + (p.dB != nullptr));
+      }
   API_END
 }
 
@@ -3078,30 +3090,27 @@ int hcc_tune_gemm(hcc_ctx* ctx, int op, int tile, int ksplit, int reps, double* 
   // the table built below is dropped at the end of the call
   size_t nalloc = b.allocs.size(), nalt = b.alt.size(), nchunk = b.chunks.size(), used = nchunk ? b.chunks.back().used : 0;
   GemmTable t;
-  if (dual)
-    t = tile == 0 ? b.dit[q]
-                  : make_table(b, [&](int k) { return delta_prob(b, q, k); }, true, tile, -1, ksplit > 0 ? ksplit : 1,
-                               true);
-  else if (tile == 0) {
-    need_op_tables(b);
+  auto keep = [&] {
     nalloc = b.allocs.size();
     nalt = b.alt.size();
     nchunk = b.chunks.size();
     used = nchunk ? b.chunks.back().used : 0;
+  };
+  if (dual && tile == 0) {
+    need_delta_op_tables(b);
+    keep();
+    t = b.dit[q];
+  } else if (dual)
+    t = make_table(b, [&](int k) { return delta_prob(b, q, k); }, true, tile, -1, ksplit > 0 ? ksplit : 1, true);
+  else if (tile == 0) {
+    need_op_tables(b);
+    keep();
     t = b.it[q];
   } else
     t = make_table(b, [&](int k) { return b.ops[q](b.hm[k]); }, true, tile, -1, ksplit > 0 ? ksplit : 1);
   auto run = [&]() {
-    if (!dual) {
-      launch_table(ctx, t);
-      return;
-    }
-    for (const GemmTable* p = &t; p != nullptr; p = p->alt >= 0 ? &b.alt[p->alt] : nullptr) {
-      if (p->nprob == 0) continue;
-      HCHECK(launch_gemm_dual(p->d, p->tile_prob, p->tiles, b.dact, ctx->stream, p->flags, true, p->tile));
-      if (p->red_blocks > 0)
-        HCHECK(launch_splitk_reduce(p->d, p->red_prefix, p->red_bprob, p->red_blocks, b.dact, ctx->stream));
-    }
+    if (dual) launch_delta_table(ctx, t);
+    else launch_table(ctx, t);
   };
   reset_state(b.dst, b.dact, b.nm, ctx->stream);   // every molecule active
   hipEvent_t e0, e1;
@@ -3363,12 +3372,13 @@ int hcc_selftest_gemm_correction(int m, int n, int k, int a_kfast, int b_nfast, 
     p.ksplit = 1;
     p.kchunk = k;
     const int tiles = ((m + tile - 1) / tile) * p.tiles_n;
-    const int flags = (a_kfast ? 1 : 0) | (b_nfast ? 2 : 0) | (dA ? 4 : 0) | (dB ? 8 : 0) | (k <= 64 && tile != 128 ? 16 : 0);
+    set_dual_modes(p);
+    const XcdMap xcd = xcd_runs({tiles}, {1.f});
     HCHECK(hipMalloc(&dp, sizeof(GemmProb)));
     HCHECK(hipMemcpy(dp, &p, sizeof(p), hipMemcpyHostToDevice));
     HCHECK(hipMalloc(&dtp, sizeof(int) * tiles));
     HCHECK(hipMemset(dtp, 0, sizeof(int) * tiles));
-    HCHECK(launch_gemm_dual(dp, dtp, tiles, nullptr, nullptr, flags, 1, kind));
+    HCHECK(launch_gemm_dual(dp, dtp, xcd, nullptr, nullptr, true, kind, k <= 64));
     HCHECK(hipDeviceSynchronize());
     HCHECK(hipMemcpy(Cd, cd, sizeof(float) * nc, hipMemcpyDeviceToHost));
     if (ms) *ms = 0.0;
@@ -3376,7 +3386,7 @@ int hcc_selftest_gemm_correction(int m, int n, int k, int a_kfast, int b_nfast, 
       HCHECK(hipEventCreate(&e0));
       HCHECK(hipEventCreate(&e1));
       HCHECK(hipEventRecord(e0, nullptr));
-      for (int r = 0; r < reps; ++r) HCHECK(launch_gemm_dual(dp, dtp, tiles, nullptr, nullptr, flags, 1, kind));
+      for (int r = 0; r < reps; ++r) HCHECK(launch_gemm_dual(dp, dtp, xcd, nullptr, nullptr, true, kind, k <= 64));
       HCHECK(hipEventRecord(e1, nullptr));
       HCHECK(hipEventSynchronize(e1));
       float t = 0.f;

@@ -138,3 +138,37 @@ def test_residual_at_ragged_sizes(o, v):
     print(o, v, np.abs(d1 - r1).max(), np.abs(d2 - r2).max())
     assert np.abs(d1 - r1).max() < 1e-11 * max(1.0, np.abs(r1).max())
     assert np.abs(d2 - r2).max() < 1e-11 * max(1.0, np.abs(r2).max())
+
+
+@pytest.mark.parametrize("m,n,k", [(12 * 64, 64, 17), (12 * 64 + 1, 129, 20), (25 * 64 - 3, 3 * 64, 33), (700, 13 * 64, 16)])
+def test_tile_bands_fp64(m, n, k):
+    """Products whose tile rows fill one band of 12, start the next one and end
+    inside the third: k roundings of a sum of k products, each 2^-53 of the sum
+    of magnitudes."""
+    rng = np.random.default_rng(m + n)
+    A, B, C0 = rng.standard_normal((m, k)), rng.standard_normal((k, n)), rng.standard_normal((m, n))
+    C = capi.selftest_gemm(A, B, C0, alpha=0.5, beta=2.0)
+    bound = 2.0 ** -53 * (k + 4) * (np.abs(A) @ np.abs(B) + 2 * np.abs(C0))
+    assert (np.abs(C - (0.5 * A @ B + 2.0 * C0)) <= bound).all()
+
+
+@pytest.mark.parametrize("tile,m,n,k", [(128, 8 * 128, 130, 40), (128, 8 * 128 + 1, 257, 64), (128, 17 * 128 - 5, 128, 33),
+                                        (64, 12 * 64 + 1, 65, 40), (64, 12 * 64 + 1, 65, 70), (32, 12 * 32 + 1, 33, 40),
+                                        (32, 25 * 32 + 7, 70, 100)])
+@pytest.mark.parametrize("kinds", [(True, True), (True, False), (False, True)])
+@pytest.mark.parametrize("a_kfast,b_nfast", [(True, True), (True, False), (False, True), (False, False)])
+def test_tile_bands_correction(tile, m, n, k, kinds, a_kfast, b_nfast):
+    """The correction GEMM over every layout, either operand constant, at the
+    edges of its bands and on both sides of the short-K rule.  Each of the two
+    products rounds both factors to BF16 (2^-8 relative each, with B0's copy
+    rounded before dB is added: 2^-9 more) and accumulates in FP32."""
+    rng = np.random.default_rng(m * 7 + n)
+    A0, B0 = rng.standard_normal((m, k)), rng.standard_normal((k, n))
+    dA = (1e-3 * rng.standard_normal((m, k))).astype(np.float32) if kinds[0] else None
+    dB = (1e-3 * rng.standard_normal((k, n))).astype(np.float32) if kinds[1] else None
+    C0 = rng.standard_normal((m, n)).astype(np.float32)
+    C, _ = capi.selftest_gemm_correction(A0, dA, B0, dB, C0, alpha=0.5, beta=1.0, a_kfast=a_kfast, b_nfast=b_nfast, tile=tile)
+    a, b = (np.zeros((m, k)) if dA is None else dA.astype(float)), (np.zeros((k, n)) if dB is None else dB.astype(float))
+    ref = 0.5 * (A0 @ b + a @ (B0 + b)) + C0
+    mag = 0.5 * (np.abs(A0) @ np.abs(b) + np.abs(a) @ (np.abs(B0) + np.abs(b)))
+    assert (np.abs(C - ref) <= 2.0 ** -7 * mag + 2.0 ** -23 * (np.abs(C0) + mag)).all()
