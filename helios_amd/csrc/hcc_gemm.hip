@@ -58,6 +58,19 @@ __device__ __forceinline__ int col_off(const Operand& o, int c) {
   const int q = quot(c, o.ic);
   return q * o.sch + (c - q * o.rc) * o.scl;
 }
+// the same for output rows and columns, which may run over pairs
+__device__ __forceinline__ int out_row(const Operand& o, int r) {
+  if (o.rr > 0) return row_off(o, r);
+  int i, j;
+  pair_of(r, -o.rr, i, j);
+  return i * o.srh + j * o.srl;
+}
+__device__ __forceinline__ int out_col(const Operand& o, int c) {
+  if (o.rc > 0) return col_off(o, c);
+  int i, j;
+  pair_of(c, -o.rc, i, j);
+  return i * o.sch + j * o.scl;
+}
 
 // Problem owning global tile `tile`: one load from the table's tile map
 // (a binary search over problems would be a chain of dependent loads).
@@ -172,12 +185,12 @@ __device__ __forceinline__ void gemm_f64_tile(const GemmProb& P, int lt, double*
 #pragma unroll
   for (int i = 0; i < SA::kN; ++i) {
     const int m = m0 + SA::row(t, i);
-    fa[i] = m < P.M ? 8u * (unsigned)row_off(P.A, m) : kPadByte;
+    fa[i] = m < P.M ? 8u * (unsigned)out_row(P.A, m) : kPadByte;
   }
 #pragma unroll
   for (int i = 0; i < SB::kN; ++i) {
     const int n = n0 + SB::row(t, i);
-    fb[i] = n < P.N ? 8u * (unsigned)col_off(P.B, n) : kPadByte;
+    fb[i] = n < P.N ? 8u * (unsigned)out_col(P.B, n) : kPadByte;
   }
   const __amdgpu_buffer_rsrc_t rA = rsrc(P.A.p), rB = rsrc(P.B.p);
   d2 ra[SA::kN], rb[SB::kN];   // mode 2 uses the first element
@@ -281,7 +294,7 @@ __device__ __forceinline__ void gemm_f64_tile(const GemmProb& P, int lt, double*
   for (int j = 0; j < 2; ++j) {
     const int col = n0 + wn + (MB == 0 ? 16 * j + (lane & 15) : 2 * (lane & 15) + j);
     if (col >= P.N) continue;
-    const int co = P.ksplit > 1 ? col : col_off(P.C, col);
+    const int co = P.ksplit > 1 ? col : out_col(P.C, col);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
 #pragma unroll
@@ -292,7 +305,7 @@ __device__ __forceinline__ void gemm_f64_tile(const GemmProb& P, int lt, double*
           W[(long)row * P.N + co] = acc[i][j][r];
           continue;
         }
-        const int o = row_off(P.C, row) + co;
+        const int o = out_row(P.C, row) + co;
         double v = P.alpha * acc[i][j][r];
         if (P.beta != 0.0) v += P.beta * W[o];
         W[o] = v;
@@ -365,10 +378,10 @@ __device__ __forceinline__ void gemm_dual_f64_tile(const GemmProb& P, int lt, do
     const int q = t + i * T;
     const int m = m0 + (AKF ? q / BK : q % BM);
     kqa[i] = AKF ? q % BK : q / BM;
-    fa[i] = m < P.M ? row_off(P.A, m) : -1;
+    fa[i] = m < P.M ? out_row(P.A, m) : -1;
     const int n = n0 + (BNF ? q % BN : q / BK);
     kqb[i] = BNF ? q / BN : q % BK;
-    fb[i] = n < P.N ? col_off(P.B, n) : -1;
+    fb[i] = n < P.N ? out_col(P.B, n) : -1;
   }
   const gdouble* __restrict__ A0 = gptr(P.A.p);
   const float* __restrict__ dA = P.dA;
@@ -453,14 +466,14 @@ __device__ __forceinline__ void gemm_dual_f64_tile(const GemmProb& P, int lt, do
   for (int j = 0; j < 2; ++j) {
     const int col = n0 + wn + 16 * j + (lane & 15);
     if (col >= P.N) continue;
-    const int co = col_off(P.C, col);
+    const int co = out_col(P.C, col);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = m0 + wm + 16 * i + (lane >> 4) + 4 * r;
         if (row >= P.M) continue;
-        const int o = row_off(P.C, row) + co;
+        const int o = out_row(P.C, row) + co;
         double v = P.alpha * acc[i][j][r];
         if (P.beta != 0.0) v += P.beta * Cp[o];
         Cp[o] = v;
@@ -549,8 +562,8 @@ __device__ __forceinline__ void gemm_dual_tile(const GemmProb& P, int lt, __bf16
   int fa[NE], fb[NE];
 #pragma unroll
   for (int j = 0; j < NE; ++j) {
-    fa[j] = m0 + SA::row(t, j) < P.M ? 2 * row_off(P.A, m0 + SA::row(t, j)) : kPad;
-    fb[j] = n0 + SB::row(t, j) < P.N ? 2 * col_off(P.B, n0 + SB::row(t, j)) : kPad;
+    fa[j] = m0 + SA::row(t, j) < P.M ? 2 * out_row(P.A, m0 + SA::row(t, j)) : kPad;
+    fb[j] = n0 + SB::row(t, j) < P.N ? 2 * out_col(P.B, n0 + SB::row(t, j)) : kPad;
   }
   // BF16 resources: byte offset 2e, range 2^28 bytes; FP32: 4e, 2^29 bytes
   // (valid element indices stay below 2^27, checked by the host)
@@ -665,14 +678,14 @@ __device__ __forceinline__ void gemm_dual_tile(const GemmProb& P, int lt, __bf16
   for (int j = 0; j < FN; ++j) {
     const int col = n0 + wn + 16 * j + (lane & 15);
     if (col >= P.N) continue;
-    const int co = col_off(P.C, col);
+    const int co = out_col(P.C, col);
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = m0 + wm + 16 * i + 4 * (lane >> 4) + r;
         if (row >= P.M) continue;
-        const int o = row_off(P.C, row) + co;
+        const int o = out_row(P.C, row) + co;
         double v = P.alpha * (double)acc[i][j][r];
         if (P.beta != 0.0) v += P.beta * Cp[o];
         Cp[o] = v;
@@ -757,7 +770,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmProb* __re
   const int row = e / P.N, col = e % P.N;
   double s = 0.0;
   for (int k = 0; k < P.ksplit; ++k) s += P.ws[k * mn + e];
-  const int o = row_off(P.C, row) + col_off(P.C, col);
+  const int o = out_row(P.C, row) + out_col(P.C, col);
   double v = P.alpha * s;
   if (P.Cd != nullptr) {   // FP32 correction output
     if (P.beta != 0.0) v += P.beta * P.Cd[o];
@@ -815,8 +828,8 @@ hipError_t launch_compact_table(const GemmProb* src, const int* idx, const int* 
 
 void set_f64_modes(GemmProb& p) {
   const int ra = one_run_cols(p.A) ? 0 : p.A.rc, rb = one_run_rows(p.B) ? 0 : p.B.rr;   // runs along K
-  int ma = unit_cols(p.A) ? 0 : (unit_rows(p.A) && (one_run_rows(p.A) || p.A.rr % 2 == 0) ? 1 : 2);
-  int mb = unit_cols(p.B) ? (one_run_cols(p.B) || p.B.rc % 2 == 0 ? 1 : 2) : (unit_rows(p.B) ? 0 : 2);
+  int ma = unit_cols(p.A) ? 0 : (unit_rows(p.A) && (one_run_rows(p.A) || (p.A.rr > 0 && p.A.rr % 2 == 0)) ? 1 : 2);
+  int mb = unit_cols(p.B) ? (one_run_cols(p.B) || (p.B.rc > 0 && p.B.rc % 2 == 0) ? 1 : 2) : (unit_rows(p.B) ? 0 : 2);
   // a padded enumeration for one operand's odd runs shifts the other's pairs
   // against its own runs unless they are the same
   p.krun = 0;

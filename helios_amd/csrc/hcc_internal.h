@@ -41,6 +41,16 @@ struct Operand {
 // lies at least 2^-17 from an integer, the FP64 rounding error is below 2^-25.
 constexpr int kMaxRadix = 1 << 16;
 constexpr int kMaxIndex = 1 << 27;
+// A negative rr (rc) = -o enumerates rows (columns) over the pairs (i, j),
+// i <= j < o, in row-major order instead: offset = i * srh + j * srl.
+__device__ __forceinline__ void pair_of(int r, int o, int& i, int& j) {
+  const int s = o * (o + 1) / 2 - 1 - r;   // counted from the last pair: h full rows of 1 .. h pairs behind it
+  int h = (int)((sqrtf(8.f * (float)s + 1.f) - 1.f) * 0.5f);   // off by at most one (s < 2^27)
+  if (h * (h + 1) / 2 > s) --h;
+  if ((h + 1) * (h + 2) / 2 <= s) ++h;
+  i = o - 1 - h;
+  j = o - 1 - (s - h * (h + 1) / 2);
+}
 inline Operand make_operand(double* p, int rr, int rc, int srh, int srl, int sch, int scl) {
   return Operand{p, rr, rc, srh, srl, sch, scl, 1.0 / rr, 1.0 / rc};
 }

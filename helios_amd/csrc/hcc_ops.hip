@@ -219,11 +219,12 @@ __global__ __launch_bounds__(kEwThreads) void k_u_xx(const MT* __restrict__ mols
 }
 
 // w2 += x + x^T - 1/2 (Z[ai,bj] + Z[bj,ai]) - (Z[aj,bi] + Z[bi,aj]), with
-// Zs[i][j][a][b] = Z[(a,i),(b,j)]
+// Zs[i][j][a][b] = Z[(a,i),(b,j)], at i <= j: Omega2[j][i][b][a] is the mirror
+// image, and whatever reads Omega2 reads that half
 template <class MT>
 __global__ __launch_bounds__(kEwThreads) void k_assemble(const MT* __restrict__ mols, const State* __restrict__ st,
                                                         Ragged rg, int nm) {
-  RAGGED_PROLOGUE((long)mols[mol].o * mols[mol].o * mols[mol].v * mols[mol].v);
+  RAGGED_PROLOGUE((long)mols[mol].o * (mols[mol].o + 1) / 2 * mols[mol].v * mols[mol].v);
   if (!st[mol].active) return;
   using V = std::remove_pointer_t<decltype(M.w2)>;
   const int o = M.o, v = M.v;
@@ -233,24 +234,28 @@ __global__ __launch_bounds__(kEwThreads) void k_assemble(const MT* __restrict__ 
   // kEwItems elements per thread, loads before stores
   double val[kEwItems];
   V w[kEwItems];
+  long at[kEwItems];
 #pragma unroll
   for (int it = 0; it < kEwItems; ++it) {
     const long f = f0 + (long)it * kEwThreads;
-    const long g = f < size_ ? f : 0;
-    int i, j, a, b;
-    ijab_of(g, o, v, i, j, a, b);
+    const unsigned g = f < size_ ? (unsigned)f : 0u;
+    const unsigned q = g / (unsigned)v, p = q / (unsigned)v;
+    int i, j;
+    pair_of((int)p, o, i, j);
+    const int b = (int)(g - q * (unsigned)v), a = (int)(q - p * (unsigned)v);
     const long ij = ((long)i * o + j) * v * v, ji = ((long)j * o + i) * v * v;
     const long ab = (long)a * v + b, ba = (long)b * v + a;
-    double s = (double)x[g] + x[ji + ba];
+    at[it] = ij + ab;
+    double s = (double)x[ij + ab] + x[ji + ba];
     s -= 0.5 * (Z[ij + ab] + Z[ji + ba]);
     s -= Z[ji + ab] + Z[ij + ba];
     val[it] = s;
-    w[it] = w2in[g];
+    w[it] = w2in[ij + ab];
   }
 #pragma unroll
   for (int it = 0; it < kEwItems; ++it) {
     const long f = f0 + (long)it * kEwThreads;
-    if (f < size_) w2[f] = w[it] + val[it];
+    if (f < size_) w2[at[it]] = w[it] + val[it];
   }
 }
 
@@ -1027,7 +1032,10 @@ __global__ __launch_bounds__(kEwThreads) void k_lr_omega(const Mol* __restrict__
   double* o1 = o1p[mol];
   if (o1 == nullptr) return;
   const long n1 = (long)M.o * M.v;
-  const double w2 = M.w2[e];
+  // Omega2 is formed at i <= j
+  int i2, j2, a2, b2;
+  ijab_of(e, M.o, M.v, i2, j2, a2, b2);
+  const double w2 = M.w2[i2 <= j2 ? e : (((long)j2 * M.o + i2) * M.v + b2) * M.v + a2];
   double* q2 = o2p[mol] + e;
   *q2 = minus ? (*q2 - w2) * scale : w2;
   if (e < n1) {
