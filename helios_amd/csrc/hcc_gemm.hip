@@ -328,7 +328,7 @@ __global__ __launch_bounds__(HCC_F64_THREADS(BM, BN)) __attribute__((amdgpu_wave
   if (tile >= xcd.begin[x + 1]) return;
   const GemmProb P = probs[find_problem(tile_prob, tile)];
   if (active != nullptr && active[P.mol] == 0) return;
-  const int lt = tile - P.tile_begin;
+  const int lt = tile - P.tile_begin + P.lt0;
 #define HCC_F64_TILE(MA, MB) \
   case 3 * MA + MB: gemm_f64_tile<BM, BN, MA, MB>(P, lt, As, Bs, koffA, koffB); break;
   switch (P.modes) {   // uniform over the workgroup
@@ -489,7 +489,7 @@ __global__ __launch_bounds__(256) void gemm_dual_f64(const GemmProb* __restrict_
   if (tile >= xcd.begin[x + 1]) return;
   const GemmProb P = probs[find_problem(tile_prob, tile)];
   if (active != nullptr && active[P.mol] == 0) return;
-  const int lt = tile - P.tile_begin;
+  const int lt = tile - P.tile_begin + P.lt0;
   switch (P.modes & 3) {   // uniform over the workgroup
     case 0: gemm_dual_f64_tile<false, false>(P, lt, A0s, dAs, dBs, Bfs); break;
     case 1: gemm_dual_f64_tile<true, false>(P, lt, A0s, dAs, dBs, Bfs); break;
@@ -709,7 +709,7 @@ __global__ __launch_bounds__(TS * 4) __attribute__((amdgpu_waves_per_eu(SK ? 6 :
   if (tile >= xcd.begin[x + 1]) return;
   const GemmProb P = probs[find_problem(tile_prob, tile)];
   if (active != nullptr && active[P.mol] == 0) return;
-  const int lt = tile - P.tile_begin;
+  const int lt = tile - P.tile_begin + P.lt0;
 #define HCC_DUAL_TILE(AK, BN, HA, HB) \
   case AK + 2 * BN + 4 * HA + 8 * HB: gemm_dual_tile<AK, BN, HA, HB, TS, SK>(P, lt, A0s, dAs, dBs, Bfs, koffA, koffB); break;
 #define HCC_DUAL_LAYOUTS(HA, HB) \
@@ -768,8 +768,19 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmProb* __re
   const long mn = (long)P.M * P.N;
   if (e >= mn) return;
   const int row = e / P.N, col = e % P.N;
+  // the adds are a chain; the loads of 16 partials are in flight together (one
+  // load at a time: 53 us for the 211 partials of a 120-site molecule's thin
+  // contractions, 13 us so)
+  const gdouble* __restrict__ W = gptr((const double*)P.ws) + e;
+  constexpr int kBatch = 16;
   double s = 0.0;
-  for (int k = 0; k < P.ksplit; ++k) s += P.ws[k * mn + e];
+  for (int k0 = 0; k0 < P.ksplit; k0 += kBatch) {
+    double part[kBatch];
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) part[k] = k0 + k < P.ksplit ? W[(k0 + k) * mn] : 0.0;
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) s += part[k];
+  }
   const int o = out_row(P.C, row) + out_col(P.C, col);
   double v = P.alpha * s;
   if (P.Cd != nullptr) {   // FP32 correction output

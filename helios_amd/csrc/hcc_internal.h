@@ -67,7 +67,8 @@ struct GemmProb {
   int M, N, K;
   double alpha, beta;
   int tiles_n;      // tiles along N for this problem (for the table's tile size)
-  int tile_begin;   // first global tile of this problem
+  int tile_begin;   // first global tile of this problem (of this part of it)
+  int lt0;          // a problem spread over the XCDs: first tile of this part
   int mol;          // molecule index (for the active mask)
   int a_kfast;      // 1: A's unit stride runs along K, 0: along M
   int b_nfast;      // 1: B's unit stride runs along N, 0: along K

@@ -147,17 +147,23 @@ static int choose_tile_dual(const GemmProb& p) {
   return 2.0 * t32 < t64 ? 32 : 64;
 }
 
-// Split K when a problem has few output tiles and a long K: aim for >= 16
-// work items per problem with K chunks of at least 128.
+// Split K when a problem has few output tiles and a long K: at least 16 work
+// items per problem, chunks of at least 128.  From K = 2048 a single molecule
+// has to fill the chip too, and its thin contractions (K = o v^2, one tile)
+// must not outlast the square ones of their level: up to 256 work items as
+// well, with chunks of at least 1024, or 512 where there are 16 tiles or more
+// (the o v x 1 product).  With 16 chunks of 13500 those of 120 sites ran 600 us
+// on 16 to 48 workgroups, twice an iteration: solves with 16 work items and
+// with this rule 421 and 357 ms (mixed precision), 100 sites 181 and 173 ms.
 static void choose_split(GemmProb& p, int ts) {
   const int tmn = ((p.M + tile_m(ts) - 1) / tile_m(ts)) * ((p.N + tile_n(ts) - 1) / tile_n(ts));
   p.ksplit = 1;
   p.kchunk = p.kpad;
-  if (tmn >= 16 || p.K < 512) return;
-  int want = (16 + tmn - 1) / tmn;
-  int maxs = p.K / 128;
-  int ks = std::min(want, std::max(1, maxs));
-  ks = std::min(ks, 64);
+  if (p.K < 512) return;
+  auto chunks = [&](int items, int least) { return std::min((items + tmn - 1) / tmn, std::max(1, p.K / least)); };
+  int ks = chunks(16, 128);
+  if (p.K >= 2048) ks = std::max(ks, chunks(256, tmn >= 16 ? 512 : 1024));
+  ks = std::min(ks, 256);
   if (ks <= 1) return;
   int chunk = (p.kpad + ks - 1) / ks;
   chunk = (chunk + 31) / 32 * 32;      // multiple of both K tiles (16 for FP64, 32 for BF16)
@@ -267,7 +273,7 @@ struct Batch {
   bool mixed_bf16 = true;   // BF16 correction GEMMs (false: FP64 exact mode, 64x64 tiles only)
   std::vector<MolD> hd;   // FP32 corrections (variable buffers) + shared FP64 inputs
   MolD* ddm = nullptr;
-  std::vector<std::function<GemmProb(const Mol&)>> ops;
+  std::vector<std::function<GemmProb(const Mol&)>> ops, pre_ops;   // of an iteration, of the set-up
   std::vector<GemmTable> dlv, dit;   // per dependency level, per contraction (as lv and it)
   // (T): undressed integral blocks (xp|yd), (ql|rz), their GEMM tables and the work items
   std::vector<double*> tA, tB;
@@ -459,65 +465,113 @@ static void set_dual_modes(GemmProb& p) {
   p.modes = p.a_kfast | (p.b_nfast << 1) | ((p.dA != nullptr) << 2) | ((p.dB != nullptr) << 3);
 }
 
+// Few molecules: every large problem is dealt out to the 8 XCDs in equal
+// parts (its own copy of the problem each, lt0 its first tile), the small ones
+// to the least loaded XCD.  Contiguous runs of equal predicted cost would give
+// an XCD the tiles of one contraction, and those of a level differ in speed
+// (one or two products, layout of the operands): at 120 sites a level of
+// 380 + 557 + 316 us of correction products took 1712 us in such runs, 1246 us
+// in parts (solve 357 and 326 ms).  Fills the parts in launch order and the XCDs' ranges.
+constexpr int kSpreadMols = 16;    // more molecules: each stays on one XCD, in one L2
+constexpr int kSpreadTiles = 64;
+static std::vector<GemmProb> spread_parts(const std::vector<GemmProb>& probs, const std::vector<int>& tiles,
+                                          const std::vector<float>& cost, std::vector<int>& ptiles,
+                                          std::vector<float>& pcost, XcdMap& xcd) {
+  struct Part {
+    int prob, lt0, n;
+  };
+  std::vector<Part> of[8];
+  double load[8] = {0.0};
+  auto put = [&](int x, int q, int lt0, int n) {
+    if (n > 0) of[x].push_back({q, lt0, n});
+    load[x] += (double)n * cost[q];
+  };
+  for (int q = 0; q < (int)probs.size(); ++q)
+    if (tiles[q] >= kSpreadTiles)
+      for (int x = 0; x < 8; ++x) {
+        const int at = (int)((long)tiles[q] * x / 8);
+        put(x, q, at, (int)((long)tiles[q] * (x + 1) / 8) - at);
+      }
+  for (int q = 0; q < (int)probs.size(); ++q)
+    if (tiles[q] < kSpreadTiles) put((int)(std::min_element(load, load + 8) - load), q, 0, tiles[q]);
+  std::vector<GemmProb> parts;
+  int at = 0;
+  for (int x = 0; x < 8; ++x) {
+    xcd.begin[x] = at;
+    for (const Part& w : of[x]) {
+      GemmProb p = probs[w.prob];
+      p.tile_begin = at;
+      p.lt0 = w.lt0;
+      at += w.n;
+      parts.push_back(p);
+      ptiles.push_back(w.n);
+      pcost.push_back(cost[w.prob]);
+    }
+  }
+  xcd.begin[8] = at;
+  return parts;
+}
+
 // One launchable table from problems that share the tile edge `ts` (their
 // ksplit / kchunk already chosen).
 static GemmTable build_group(Batch& b, std::vector<GemmProb> probs, int ts) {
-  int tiles = 0;
+  GemmTable t;
+  t.tile = ts;
+  // short-K variant of the correction GEMM when no problem has more than two 32-deep slabs
+  t.short_k = true;
   long ws_total = 0;
+  bool large = false;
   for (GemmProb& p : probs) {
     p.tiles_n = (p.N + tile_n(ts) - 1) / tile_n(ts);
     const int tm = (p.M + tile_m(ts) - 1) / tile_m(ts);
-    p.tile_begin = tiles;
-    tiles += tm * p.tiles_n * p.ksplit;
+    p.tile_begin = t.tiles;
+    t.htiles.push_back(tm * p.tiles_n * p.ksplit);
+    t.tiles += t.htiles.back();
+    large = large || t.htiles.back() >= kSpreadTiles;
+    // matrix work of a tile plus the equivalent of its set-up, first loads and stores
+    t.hcost.push_back((float)(p.kchunk + 96));
     p.a_kfast = unit_cols(p.A) ? 1 : (unit_rows(p.A) ? 0 : 1);
     p.b_nfast = unit_cols(p.B) ? 1 : (unit_rows(p.B) ? 0 : 1);
     if (p.Cd != nullptr) set_dual_modes(p);
     if (p.ksplit > 1) ws_total += (long)p.ksplit * p.M * p.N;
+    t.short_k = t.short_k && p.kchunk <= 64;
   }
-  GemmTable t;
-  t.nprob = (int)probs.size();
-  t.tiles = tiles;
-  t.tile = ts;
-  for (const GemmProb& p : probs) {
-    t.hmol.push_back(p.mol);
-    t.htiles.push_back(((p.M + tile_m(ts) - 1) / tile_m(ts)) * p.tiles_n * p.ksplit);
-    t.hred.push_back(p.ksplit > 1 ? (int)(((long)p.M * p.N + 255) / 256) : 0);
-    // matrix work of a tile plus the equivalent of its set-up, first loads and stores
-    t.hcost.push_back((float)(p.kchunk + 96));
-  }
-  t.xcd = xcd_runs(t.htiles, t.hcost);
-  // short-K variant of the correction GEMM when no problem has more than two 32-deep slabs
-  t.short_k = true;
-  for (const GemmProb& p : probs) t.short_k = t.short_k && p.kchunk <= 64;
   if (ws_total > 0) {
     double* ws = b.dalloc<double>(ws_total);
-    long off = 0;
-    std::vector<int> pre(probs.size() + 1, 0);
-    for (size_t q = 0; q < probs.size(); ++q) {
-      GemmProb& p = probs[q];
-      int blocks = 0;
-      if (p.ksplit > 1) {
-        p.ws = ws + off;
-        off += (long)p.ksplit * p.M * p.N;
-        blocks = (int)(((long)p.M * p.N + 255) / 256);
-      }
-      pre[q + 1] = pre[q] + blocks;
+    for (GemmProb& p : probs) {
+      if (p.ksplit <= 1) continue;
+      p.ws = ws;
+      ws += (long)p.ksplit * p.M * p.N;
     }
+  }
+  if (large && b.nm < kSpreadMols) {
+    std::vector<int> ptiles;
+    std::vector<float> pcost;
+    probs = spread_parts(probs, t.htiles, t.hcost, ptiles, pcost, t.xcd);
+    t.htiles = ptiles;
+    t.hcost = pcost;
+  } else {
+    t.xcd = xcd_runs(t.htiles, t.hcost);
+  }
+  t.nprob = (int)probs.size();
+  // split-K reduction blocks: one range per problem (with its part at lt0 = 0)
+  std::vector<int> pre(1, 0);
+  for (const GemmProb& p : probs) {
+    t.hmol.push_back(p.mol);
+    t.hred.push_back(p.ksplit > 1 && p.lt0 == 0 ? (int)(((long)p.M * p.N + 255) / 256) : 0);
+    pre.push_back(pre.back() + t.hred.back());
+  }
+  auto expand = [](const std::vector<int>& count) {
+    std::vector<int> of;
+    for (size_t q = 0; q < count.size(); ++q) of.insert(of.end(), count[q], (int)q);
+    return of;
+  };
+  if (pre.back() > 0) {
     t.red_prefix = b.upload(pre);
     t.red_blocks = pre.back();
-    std::vector<int> bp(t.red_blocks);
-    for (size_t q = 0; q < probs.size(); ++q)
-      for (int x = pre[q]; x < pre[q + 1]; ++x) bp[x] = (int)q;
-    t.red_bprob = b.upload(bp);
+    t.red_bprob = b.upload(expand(t.hred));
   }
-  if (tiles > 0) {
-    std::vector<int> tp(tiles);
-    for (size_t q = 0; q < probs.size(); ++q) {
-      const int end = q + 1 < probs.size() ? probs[q + 1].tile_begin : tiles;
-      for (int x = probs[q].tile_begin; x < end; ++x) tp[x] = (int)q;
-    }
-    t.tile_prob = b.upload(tp);
-  }
+  if (t.tiles > 0) t.tile_prob = b.upload(expand(t.htiles));
   if (t.nprob) t.d = b.upload(probs);
   return t;
 }
@@ -829,22 +883,21 @@ static void build_tables(Batch& b) {
   std::vector<Mol>& H = b.hm;
   // --- precompute: Fao = C F C^T, Gklcd = (kc|ld) from undressed P, Q
   b.pre.clear();
-  b.pre.push_back(make_table(b, [&](int k) {   // tmp = C F
-    const Mol& M = H[k];
+  b.pre_ops.clear();
+  b.pre_ops.push_back([](const Mol& M) {   // tmp = C F
     const int N = M.n;
     return prob(rm(M.C, N), rm(M.F, N), rm(M.tmp, N), N, N, N, 1.0, 0.0);
-  }));
-  b.pre.push_back(make_table(b, [&](int k) {   // Fao = tmp C^T
-    const Mol& M = H[k];
+  });
+  b.pre_ops.push_back([](const Mol& M) {   // Fao = tmp C^T
     const int N = M.n;
     return prob(rm(M.tmp, N), trn(M.C, N), rm(M.Fao, N), N, N, N, 1.0, 0.0);
-  }));
-  b.pre.push_back(make_table(b, [&](int k) {   // Gklcd[k][l][c][d] = (kc|ld)
-    const Mol& M = H[k];
+  });
+  b.pre_ops.push_back([](const Mol& M) {   // Gklcd[k][l][c][d] = (kc|ld)
     const int N = M.n, o = M.o, v = M.v, N2 = N * N, ov = o * v;
     return prob(cmp(M.P + o, v, N, 1, 1, N2, 0), cmp(M.Q + o, 1, N2, 0, v, N, 1),
                 cmp(M.Gklcd, v, ov * v, v, v, v * v, 1), ov, ov, N, 1.0, 0.0);
-  }));
+  });
+  for (const auto& op : b.pre_ops) b.pre.push_back(make_table(b, [&](int k) { return op(H[k]); }));
 
   // --- one iteration
   b.it.clear();
@@ -3161,21 +3214,15 @@ int hcc_tune_gemm(hcc_ctx* ctx, int op, int tile, int ksplit, int reps, double* 
 int hcc_gemm_flops(hcc_ctx* ctx, double* per_iteration, double* per_solve_setup) {
   if (ctx == nullptr) return HCC_E_ARG;
   if (int r = need_batch(ctx)) return r;
-  std::vector<GemmProb> h;
   API_BEGIN
   Batch& b = *ctx->batch;
-  std::function<void(const GemmTable&, std::vector<double>&)> table_flops = [&](const GemmTable& t,
-                                                                                std::vector<double>& acc) {
-    h.resize(t.nprob);
-    if (t.nprob)
-      HCHECK(hipMemcpy(h.data(), t.d, t.nprob * sizeof(GemmProb), hipMemcpyDeviceToHost));
-    for (const auto& p : h) acc[p.mol] += 2.0 * p.M * (double)p.N * p.K;
-    if (t.alt >= 0) table_flops(b.alt[t.alt], acc);
-  };
   std::vector<double> it(b.nm, 0.0), pre(b.nm, 0.0);
-  for (const auto& t : b.lv) table_flops(t, it);
-  for (const auto& t : b.pre) table_flops(t, pre);
-  table_flops(b.g1, pre);
+  auto flops = [](const GemmProb& p) { return p.M > 0 && p.N > 0 ? 2.0 * p.M * (double)p.N * p.K : 0.0; };
+  for (int k = 0; k < b.nm; ++k) {
+    for (const auto& op : b.ops) it[k] += flops(op(b.hm[k]));
+    for (const auto& op : b.pre_ops) pre[k] += flops(op(b.hm[k]));
+    pre[k] += flops(b.ops[G1_Q](b.hm[k]));
+  }
   for (int k = 0; k < b.nm; ++k) {
     if (per_iteration) per_iteration[k] = it[k];
     if (per_solve_setup) per_solve_setup[k] = pre[k];
