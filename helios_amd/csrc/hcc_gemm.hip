@@ -117,6 +117,9 @@ constexpr int kBand64 = 12, kBand128 = 8;
 // register bound keeps the accumulators in VGPRs: with a larger budget the
 // compiler moves them to AGPRs and back every slab.
 //
+// A wave in its matrix work has priority over those staging (100 sites: 4.04 and
+// 3.96 ms for an iteration's contractions).
+//
 // Fragments are read from LDS 16 bytes at a time too: mode 0 gives a lane two
 // consecutive K, used by the two halves of an 8-deep step (the K order within
 // a step is free), modes 1 and 2 two consecutive rows, one for each of the
@@ -264,6 +267,7 @@ __device__ __forceinline__ void gemm_f64_tile(const GemmProb& P, int lt, double*
       }
       __syncthreads();
       load(k0 + kBK);   // the last prefetch reads only padding
+      __builtin_amdgcn_s_setprio(1);
 #pragma unroll
       for (int kk = 0; kk < kBK; kk += 8) {
         const int kg = kk + 2 * (lane >> 4), l = lane & 15;
@@ -282,6 +286,7 @@ __device__ __forceinline__ void gemm_f64_tile(const GemmProb& P, int lt, double*
               acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(MA == 0 ? a[i][h] : a[h][i], MB == 0 ? b[j][h] : b[h][j],
                                                                acc[i][j], 0, 0, 0);
       }
+      __builtin_amdgcn_s_setprio(0);
       __syncthreads();
     }
   }
@@ -349,11 +354,9 @@ __global__ __launch_bounds__(HCC_F64_THREADS(BM, BN)) __attribute__((amdgpu_wave
 // Correction-form ("dual") GEMM of the mixed-precision inner iterations:
 //   C = alpha * (A0 dB + dA (B0 + dB)) + beta * C
 // which is the change of A B between the outer point (A0, B0) and the current
-// point (A0 + dA, B0 + dB).  The differences and the full second factor are
-// formed in FP64 before rounding, so with BF16 operands the rounding error is
-// proportional to the size of the correction, not of A B.  64x64 tiles, 256
-// threads; FP64 path: BK 16 and 16x16x4 MFMA; BF16 path: BK 32 and
-// 16x16x32 MFMA with [row][k] LDS staging.
+// point (A0 + dA, B0 + dB), so with BF16 operands the rounding error is
+// proportional to the size of the correction, not of A B.  FP64 form: 64x64
+// tiles, 16-deep slabs; BF16 form below.
 // ---------------------------------------------------------------------------
 constexpr int kDualLds64 = 64 * kPk;   // [row][k] staging; [k][row] takes less
 template <bool AKF, bool BNF>
@@ -501,156 +504,215 @@ __global__ __launch_bounds__(256) void gemm_dual_f64(const GemmProb* __restrict_
 // HA / HB: the operand has a correction (dA / dB non-null for every problem
 // of the table).  A constant A needs only A0 dB, a constant B only dA B0.
 //
-// 64x64 output tiles, 4 waves of 32x32, 32-deep K slabs.  Staging is the
-// bound of this kernel (the matrix cores need 8 instructions per slab and
-// wave), so it is kept to a few instructions per element:
-//  * offsets are formed as row + K-table entry with no compare or select:
-//    a padding row or K carries the sentinel kPad, and any sum that includes
-//    it lands past the end of the 16- and 32-bit resources (which read 0);
-//  * K-contiguous operands are staged one element per lane with the lanes
-//    along K (32 lanes per row), so every load instruction is coalesced;
-//  * row-contiguous operands are staged with the lanes along the rows and two
-//    adjacent K per thread, so one V_CVT_PK_BF16_F32 and one 32-bit LDS store
-//    serve two elements.
-// Both go to LDS as [row][k] with a 40-element pitch and are read back as 8
-// consecutive K per lane.
-constexpr int kPad = 1 << 28;   // 2 x (element index) of a padding row or K
+// Output tiles of 128, 64 or 32 square, 32-deep K slabs.  Staging bounds this
+// kernel (the matrix cores need 16 instructions per slab and wave): LDS stores
+// and fragment reads first, then the return path of the loads, so elements
+// move four at a time:
+//  * an operand that is contiguous along K is loaded in quads of K, 16 bytes
+//    of the FP32 correction and the 12 bytes around 4 BF16 values (which start
+//    at any even byte), lanes along K (KC);
+//  * any other operand is loaded one element per lane, the lanes along its
+//    rows, four consecutive K per thread;
+//  * both store four consecutive K of a row to LDS as 8 bytes.
+// A quad never straddles a run of an operand's composite K: K is enumerated
+// with every run padded to a multiple of four (GemmProb::krun), and the K
+// table's low two bits hold how many of a quad's elements are padding.
+// Offsets are row + K-table entry with no compare or select: a padding row or K
+// carries the sentinel kPad, and any sum that includes it lies past the end of
+// the resources (which read 0).  Measured with single elements (16-bit LDS
+// stores along K) and with quads: a 3600^3 correction with both operands
+// contiguous along K 346 and 285 us for one product, 558 and 520 us for two;
+// 512 ragged molecules' 406 and 336, 439 and 362 us; solves of 2048 ragged
+// molecules 796 and 761 ms, of 120 sites 326 and 318 ms.  What remains is the
+// latency of a slab (two barriers, 16 waves a CU): matrix cores 16 %, load
+// return 70 %, LDS conflicts 20 % of the cycles, none of them full; a
+// conflict-free permuted LDS layout measured equal.
+constexpr unsigned kPad = 1u << 29;   // 4 x (element index) of a padding row or K
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_h(const void* p, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, bytes, 0x00020000);
 }
-// staged element j (0 .. 7) of thread t (of T) in an R-row x BK slab
-// (R * BK = 8 T): K-contiguous operands with the lanes along K,
-// row-contiguous ones with the lanes along the rows and K in adjacent pairs
-template <bool KC, int BK, int R, int T>
-struct Stage {
-  static __device__ __forceinline__ int row(int t, int j) { return KC ? t / BK + (T / BK) * j : t % R; }
-  static __device__ __forceinline__ int k(int t, int j) {
-    return KC ? t % BK : 2 * (t / R) + 2 * (T / R) * (j >> 1) + (j & 1);
-  }
+// staged group i of thread t (of T) in an R-row slab: four consecutive K from
+// k(t, i) of row(t, i)
+template <bool KC, int R, int T>
+struct DualStage {
+  static constexpr int kN = R * 8 / T;
+  static __device__ __forceinline__ int row(int t, int i) { return KC ? t / 8 + (T / 8) * i : t % R; }
+  static __device__ __forceinline__ int k(int t, int i) { return KC ? 4 * (t % 8) : 4 * (t / R) + (4 * T / R) * i; }
 };
 constexpr int kDualBK = 32;   // 64-deep slabs measured slower (K padding of the short contractions, fewer waves)
+constexpr int kDualLD = kDualBK + 8;   // LDS pitch of a staged row
+constexpr int kDualKT = 512;           // K-table chunk
+typedef unsigned u2v __attribute__((ext_vector_type(2)));
+typedef unsigned u3v __attribute__((ext_vector_type(3)));
+typedef unsigned u4v __attribute__((ext_vector_type(4)));
+typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+
+// One operand's staging: X0 (BF16 copy of the outer point, loaded with LX0)
+// and the correction dX (FP32, loaded with LDX)
+template <bool KC, bool LX0, bool LDX, int R, int T>
+struct DualOperand {
+  using S = DualStage<KC, R, T>;
+  static constexpr int N = S::kN;
+  __amdgpu_buffer_rsrc_t r0, rd;
+  unsigned f[KC ? N : 1];   // 4 x row offsets
+  unsigned q0[N][KC ? 3 : 4];
+  f4 qd[N];
+  unsigned pad, sh[KC ? N : 1];   // KC: padding elements of the quad, byte shift of its BF16 values
+  unsigned odd;                   // KC: byte distance of the BF16 block from the dword before it
+  __device__ __forceinline__ void bind(const __bf16* x0, const float* dx) {
+    odd = KC ? (unsigned)(reinterpret_cast<unsigned long>(x0) & 2u) : 0u;
+    r0 = rsrc_h(reinterpret_cast<const char*>(x0) - odd, 1 << 28);
+    rd = rsrc_h(dx, 1 << 29);
+  }
+  __device__ __forceinline__ void load(const unsigned* koff, int kl0, int t) {
+    if (KC) {
+      const unsigned e = koff[kl0 + S::k(t, 0)];
+      pad = e & 3u;
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const unsigned o = f[i] + (e & ~3u);
+        if (LX0) {
+          const unsigned h = (o >> 1) + odd;
+          const u3v w = __builtin_amdgcn_raw_buffer_load_b96(r0, (int)(h & ~3u), 0, 0);
+          q0[i][0] = w[0], q0[i][1] = w[1], q0[i][2] = w[2];
+          sh[i] = h & 2u;
+        }
+        if (LDX) qd[i] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rd, (int)o, 0, 0));
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const u4v e = *reinterpret_cast<const u4v*>(&koff[kl0 + S::k(t, i)]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const unsigned o = f[0] + e[j];
+          if (LX0) q0[i][j] = (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(r0, (int)(o >> 1), 0, 0);
+          if (LDX) qd[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, (int)o, 0, 0));
+        }
+      }
+    }
+  }
+  // 4 BF16 values of X0
+  __device__ __forceinline__ u2v x0(int i) const {
+    if (KC)
+      return u2v{__builtin_amdgcn_alignbyte(q0[i][1], q0[i][0], sh[i]), __builtin_amdgcn_alignbyte(q0[i][2], q0[i][1], sh[i])};
+    return u2v{q0[i][0] | (q0[i][1] << 16), q0[i][2] | (q0[i][3] << 16)};
+  }
+  static __device__ __forceinline__ u2v round(f4 x) { return __builtin_bit_cast(u2v, __builtin_convertvector(x, bf4)); }
+  // X0 + dX (X0 alone for a constant operand), rounded once
+  __device__ __forceinline__ u2v sum(int i) const {
+    const u2v b = x0(i);
+    if (!LDX) return b;
+    f4 x;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const unsigned u = KC ? (j & 1 ? b[j / 2] & 0xffff0000u : b[j / 2] << 16) : q0[i][j] << 16;
+      x[j] = __builtin_bit_cast(float, u) + qd[i][j];
+    }
+    return round(x);
+  }
+  __device__ __forceinline__ void store(__bf16* lds, int t, int i, u2v v) const {
+    if (KC) {
+      v[0] &= pad == 3 ? 0xffffu : ~0u;
+      v[1] &= pad == 0 ? ~0u : (pad == 1 ? 0xffffu : 0u);
+    }
+    *reinterpret_cast<u2v*>(&lds[S::row(t, i) * kDualLD + S::k(t, i)]) = v;
+  }
+};
+
 // TS: output tile edge, 32 (2 waves of 32x16), 64 (4 waves of 32x32) or 128
 // (8 waves of 32x64).  SK (short K, at most two slabs): the next slab is loaded
 // after the current one's matrix-core work instead of during it; the staging
-// registers are then dead during that work, which lets six waves share a SIMD
+// registers are then dead during that work, which lets more waves share a SIMD
 // (a one- or two-slab tile is mostly fixed latency, hidden by more tiles per CU)
-constexpr int kDualLD = kDualBK + 8;   // LDS pitch of a staged row
-constexpr int kDualKT = 512;           // K-table chunk
-template <bool AKF, bool BNF, bool HA, bool HB, int TS, bool SK>
+template <bool KA, bool KB, bool HA, bool HB, int TS, bool SK>
 __device__ __forceinline__ void gemm_dual_tile(const GemmProb& P, int lt, __bf16* A0s, __bf16* dAs, __bf16* dBs,
-                                               __bf16* Bfs, int* koffA, int* koffB) {
-  constexpr int BK = kDualBK, BM = TS, BN = TS, T = TS * 4, LD = kDualLD, NE = 8;
+                                               __bf16* Bfs, unsigned* koffA, unsigned* koffB) {
+  constexpr int BK = kDualBK, BM = TS, BN = TS, T = TS * 4, LD = kDualLD;
   constexpr int FM = 2, FN = TS / 32;   // 16x16 blocks per wave along M and N
   constexpr int KT = kDualKT;
-  constexpr bool KA = AKF, KB = !BNF;   // operand K-contiguous in memory
-  static_assert(BM * BK == NE * T, "staging covers the slab");
-  using SA = Stage<KA, BK, BM, T>;
-  using SB = Stage<KB, BK, BN, T>;
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
   const int tiles_n = (P.N + BN - 1) / BN, tiles_m = (P.M + BM - 1) / BM;
   const int ks = lt / (tiles_m * tiles_n);
   lt -= ks * tiles_m * tiles_n;
   int tm, tn;
   tile_pos<TS == 128 ? kBand128 : kBand64>(lt, tiles_m, tiles_n, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
-  const int kbeg = ks * P.kchunk, kend = min(P.K, kbeg + P.kchunk);
+  const int kbeg = ks * P.kchunk, kend = min(P.kpad, kbeg + P.kchunk);
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   // waves: 2 along N (32 FN columns each), T / 128 along M (32 rows each)
   const int wm = (wave >> 1) * 32, wn = (wave & 1) * (16 * FN);
-  // 2 x row offsets (kPad for rows past the problem)
-  int fa[NE], fb[NE];
+  // A0 dB needs A0 and dB (HB), dA (B0 + dB) needs dA and B0 (HA); BF16
+  // resources of 2^28 bytes, FP32 of 2^29 (valid element indices stay below
+  // 2^27, checked by the host)
+  using OA = DualOperand<KA, HB, HA, BM, T>;
+  using OB = DualOperand<KB, HA, HB, BN, T>;
+  OA A;
+  OB B;
+  A.bind(P.hA, HA ? P.dA : nullptr);
+  B.bind(P.hB, HB ? P.dB : nullptr);
 #pragma unroll
-  for (int j = 0; j < NE; ++j) {
-    fa[j] = m0 + SA::row(t, j) < P.M ? 2 * out_row(P.A, m0 + SA::row(t, j)) : kPad;
-    fb[j] = n0 + SB::row(t, j) < P.N ? 2 * out_col(P.B, n0 + SB::row(t, j)) : kPad;
+  for (int i = 0; i < (KA ? OA::N : 1); ++i) {
+    const int m = m0 + OA::S::row(t, i);
+    A.f[i] = m < P.M ? 4u * (unsigned)out_row(P.A, m) : kPad;
   }
-  // BF16 resources: byte offset 2e, range 2^28 bytes; FP32: 4e, 2^29 bytes
-  // (valid element indices stay below 2^27, checked by the host)
-  const __amdgpu_buffer_rsrc_t rA0 = rsrc_h(P.hA, kPad), rdA = rsrc_h(HA ? P.dA : nullptr, 2 * kPad);
-  const __amdgpu_buffer_rsrc_t rB0 = rsrc_h(P.hB, kPad), rdB = rsrc_h(HB ? P.dB : nullptr, 2 * kPad);
-  // staging registers, converted at the LDS store so that the loads stay in
-  // flight across the current slab's matrix-core work: A0 (BF16 copy) and dB
-  // feed A0 dB (needs HB), dA and B0 (BF16 copy) + dB feed dA (B0 + dB) (needs HA)
-  unsigned short ra0[NE], rb0[NE];
-  float rda[NE], rdb[NE];
+#pragma unroll
+  for (int i = 0; i < (KB ? OB::N : 1); ++i) {
+    const int n = n0 + OB::S::row(t, i);
+    B.f[i] = n < P.N ? 4u * (unsigned)out_col(P.B, n) : kPad;
+  }
   f4 acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+  const int run = P.krun > 0 ? P.krun : P.K, runp = (P.krun + 3) & ~3;   // krun = 0: one run of K
   for (int c0 = kbeg; c0 < kend; c0 += KT) {
     const int clen = min(kend - c0, KT);
     __syncthreads();
-    // 2 x K offsets of the chunk; entries past its end (read by the last,
+    // 4 x K offsets of the chunk; entries past its end (read by the last,
     // partial slab and the final prefetch) carry kPad
     for (int q = t; q < KT + BK; q += T) {
-      koffA[q] = q < clen ? 2 * col_off(P.A, c0 + q) : kPad;
-      koffB[q] = q < clen ? 2 * row_off(P.B, c0 + q) : kPad;
+      const int kp = c0 + q, hi = P.krun > 0 ? quot(kp, P.irun) : 0, lo = kp - hi * runp, k = hi * P.krun + lo;
+      const bool in = q < clen && lo < run && k < P.K;
+      const unsigned pad = (unsigned)max(0, 4 - (run - lo));
+      koffA[q] = in ? 4u * (unsigned)col_off(P.A, k) | (KA ? pad : 0u) : kPad;
+      koffB[q] = in ? 4u * (unsigned)row_off(P.B, k) | (KB ? pad : 0u) : kPad;
     }
     __syncthreads();
     auto load = [&](int kl0) {
-#pragma unroll
-      for (int j = 0; j < NE; ++j) {
-        const int ea = fa[j] + koffA[kl0 + SA::k(t, j)];
-        if (HB) ra0[j] = __builtin_amdgcn_raw_buffer_load_b16(rA0, ea, 0, 0);
-        if (HA) rda[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rdA, 2 * ea, 0, 0));
-        const int eb = fb[j] + koffB[kl0 + SB::k(t, j)];
-        if (HB) rdb[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rdB, 2 * eb, 0, 0));
-        if (HA) rb0[j] = __builtin_amdgcn_raw_buffer_load_b16(rB0, eb, 0, 0);
-      }
-    };
-    // B0 + dB as FP32 (B0 is a BF16 bit pattern)
-    auto bsum = [&](int j) {
-      const float b0 = __builtin_bit_cast(float, (unsigned)rb0[j] << 16);
-      return HB ? b0 + rdb[j] : b0;
+      A.load(koffA, kl0, t);
+      B.load(koffB, kl0, t);
     };
     load(0);
     for (int kl = 0; kl < clen; kl += BK) {
 #pragma unroll
-      for (int j = 0; j < NE; ++j) {
-        // A side
-        if (KA) {
-          const int sa = SA::row(t, j) * LD + SA::k(t, j);
-          if (HB) A0s[sa] = __builtin_bit_cast(__bf16, ra0[j]);
-          if (HA) dAs[sa] = (__bf16)rda[j];
-        } else if ((j & 1) == 0) {
-          const int sa = (SA::row(t, j) * LD + SA::k(t, j)) >> 1;
-          if (HB) reinterpret_cast<unsigned*>(A0s)[sa] = (unsigned)ra0[j] | ((unsigned)ra0[j + 1] << 16);
-          if (HA) reinterpret_cast<bf2*>(dAs)[sa] = __builtin_convertvector((f2{rda[j], rda[j + 1]}), bf2);
-        }
-        // B side
-        if (KB) {
-          const int sb = SB::row(t, j) * LD + SB::k(t, j);
-          if (HB) dBs[sb] = (__bf16)rdb[j];
-          if (HA) Bfs[sb] = (__bf16)bsum(j);
-        } else if ((j & 1) == 0) {
-          const int sb = (SB::row(t, j) * LD + SB::k(t, j)) >> 1;
-          if (HB) reinterpret_cast<bf2*>(dBs)[sb] = __builtin_convertvector((f2{rdb[j], rdb[j + 1]}), bf2);
-          if (HA) reinterpret_cast<bf2*>(Bfs)[sb] = __builtin_convertvector((f2{bsum(j), bsum(j + 1)}), bf2);
-        }
+      for (int i = 0; i < OA::N; ++i) {
+        if (HB) A.store(A0s, t, i, A.x0(i));
+        if (HA) A.store(dAs, t, i, OA::round(A.qd[i]));
+      }
+#pragma unroll
+      for (int i = 0; i < OB::N; ++i) {
+        if (HB) B.store(dBs, t, i, OB::round(B.qd[i]));
+        if (HA) B.store(Bfs, t, i, B.sum(i));
       }
       __syncthreads();
-      if (!SK) load(min(kl + BK, clen));   // the last prefetch reads only padding
+      if (!SK) load(kl + BK);   // the last prefetch reads only padding
+      const int kq = 8 * (lane >> 4);
+      // product with A from Xa, B from Xb (LDS [row][k])
+      auto product = [&](const __bf16* Xa, const __bf16* Xb) {
+        bf8 a[FM], b[FN];
 #pragma unroll
-      for (int kk = 0; kk < BK; kk += 32) {
-        const int kq = kk + 8 * (lane >> 4);
-        // product with A from Xa, B from Xb (LDS [row][k])
-        auto product = [&](const __bf16* Xa, const __bf16* Xb) {
-          bf8 a[FM], b[FN];
+        for (int f = 0; f < FM; ++f) a[f] = *reinterpret_cast<const bf8*>(&Xa[(wm + 16 * f + (lane & 15)) * LD + kq]);
 #pragma unroll
-          for (int f = 0; f < FM; ++f) a[f] = *reinterpret_cast<const bf8*>(&Xa[(wm + 16 * f + (lane & 15)) * LD + kq]);
+        for (int f = 0; f < FN; ++f) b[f] = *reinterpret_cast<const bf8*>(&Xb[(wn + 16 * f + (lane & 15)) * LD + kq]);
 #pragma unroll
-          for (int f = 0; f < FN; ++f) b[f] = *reinterpret_cast<const bf8*>(&Xb[(wn + 16 * f + (lane & 15)) * LD + kq]);
+        for (int i = 0; i < FM; ++i)
 #pragma unroll
-          for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-        };
-        if (HB) product(A0s, dBs);
-        if (HA) product(dAs, Bfs);
-      }
+          for (int j = 0; j < FN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+      };
+      if (HB) product(A0s, dBs);
+      if (HA) product(dAs, Bfs);
       __syncthreads();
       if (SK && kl + BK < clen) load(kl + BK);
     }
@@ -703,15 +765,15 @@ __global__ __launch_bounds__(TS * 4) __attribute__((amdgpu_waves_per_eu(SK ? 6 :
   __shared__ __attribute__((aligned(16))) __bf16 dAs[TS * kDualLD];
   __shared__ __attribute__((aligned(16))) __bf16 dBs[TS * kDualLD];
   __shared__ __attribute__((aligned(16))) __bf16 Bfs[TS * kDualLD];
-  __shared__ int koffA[kDualKT + kDualBK];
-  __shared__ int koffB[kDualKT + kDualBK];
+  __shared__ __attribute__((aligned(16))) unsigned koffA[kDualKT + kDualBK];
+  __shared__ __attribute__((aligned(16))) unsigned koffB[kDualKT + kDualBK];
   const int x = blockIdx.x & 7, tile = xcd.begin[x] + (int)(blockIdx.x >> 3);
   if (tile >= xcd.begin[x + 1]) return;
   const GemmProb P = probs[find_problem(tile_prob, tile)];
   if (active != nullptr && active[P.mol] == 0) return;
   const int lt = tile - P.tile_begin + P.lt0;
 #define HCC_DUAL_TILE(AK, BN, HA, HB) \
-  case AK + 2 * BN + 4 * HA + 8 * HB: gemm_dual_tile<AK, BN, HA, HB, TS, SK>(P, lt, A0s, dAs, dBs, Bfs, koffA, koffB); break;
+  case AK + 2 * BN + 4 * HA + 8 * HB: gemm_dual_tile<AK, !BN, HA, HB, TS, SK>(P, lt, A0s, dAs, dBs, Bfs, koffA, koffB); break;
 #define HCC_DUAL_LAYOUTS(HA, HB) \
   HCC_DUAL_TILE(0, 0, HA, HB) HCC_DUAL_TILE(1, 0, HA, HB) HCC_DUAL_TILE(0, 1, HA, HB) HCC_DUAL_TILE(1, 1, HA, HB)
   switch (P.modes) {
@@ -853,6 +915,30 @@ void set_f64_modes(GemmProb& p) {
   p.modes = 3 * ma + mb;
   p.kpad = p.krun > 0 ? p.K + p.K / p.krun : p.K;
   p.irun = 1.0 / (p.krun + 1);
+}
+
+void set_dual_modes(GemmProb& p, bool bf16) {
+  const bool ka = unit_cols(p.A) || !unit_rows(p.A), kb = !unit_cols(p.B) && unit_rows(p.B);
+  p.krun = 0;
+  p.kpad = p.K;
+  int qa = ka, qb = kb;
+  if (bf16) {
+    // quads along K need unit stride; runs along K (0: one run)
+    const int ra = one_run_cols(p.A) ? 0 : p.A.rc, rb = one_run_rows(p.B) ? 0 : p.B.rr;
+    qa = qa && unit_cols(p.A);
+    // padding one operand's runs shifts the other's quads against its own runs
+    // unless they are the same
+    if (qa && ra % 4 != 0) p.krun = ra;
+    if (qb && rb > 0 && p.krun > 0 && rb != p.krun) qb = 0;
+    if (qb && rb % 4 != 0 && p.krun == 0) {
+      p.krun = rb;
+      if (ra > 0) qa = 0;
+    }
+    const int runp = (p.krun + 3) / 4 * 4;
+    if (p.krun > 0) p.kpad = p.K / p.krun * runp + p.K % p.krun;
+    p.irun = p.krun > 0 ? 1.0 / runp : 0.0;
+  }
+  p.modes = qa | (!qb << 1) | ((p.dA != nullptr) << 2) | ((p.dB != nullptr) << 3);
 }
 
 template <int BM, int BN>

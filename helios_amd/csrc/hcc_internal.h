@@ -70,14 +70,13 @@ struct GemmProb {
   int tile_begin;   // first global tile of this problem (of this part of it)
   int lt0;          // a problem spread over the XCDs: first tile of this part
   int mol;          // molecule index (for the active mask)
-  int a_kfast;      // 1: A's unit stride runs along K, 0: along M
-  int b_nfast;      // 1: B's unit stride runs along N, 0: along K
   int ksplit;       // number of K chunks (1: no split)
   int kchunk;       // K range of one chunk (multiple of the K tile), in kpad's enumeration
-  // FP64 kernel: staging modes of A and B (3 MA + MB, see gemm_f64_kernel);
-  // correction kernels: a_kfast | b_nfast << 1 | (dA != 0) << 2 | (dB != 0) << 3.
-  // FP64 kernel: the enumeration of K with one padding element behind every run of krun
-  // (0: no such runs), kpad elements long; irun = 1 / (krun + 1)
+  // staging modes: FP64 kernel, 3 MA + MB (see gemm_f64_kernel); correction
+  // kernels, A along K | B along its columns << 1 | (dA != 0) << 2 | (dB != 0) << 3.
+  // K is enumerated with padding behind every run of krun (0: no such runs): one
+  // element in the FP64 kernel, up to a multiple of 4 in the BF16 one; kpad
+  // elements long, irun = 1 / (padded run)
   int modes;
   int krun, kpad;
   double irun;
@@ -111,6 +110,8 @@ hipError_t launch_gemm_f64(const GemmProb* probs, const int* tile_prob, const Xc
                            const int* active, hipStream_t s, int tile = 64);
 // staging modes and K enumeration of a problem for the FP64 kernel
 void set_f64_modes(GemmProb& p);
+// the same for a correction-form problem on the BF16 (or the FP64) kernel
+void set_dual_modes(GemmProb& p, bool bf16);
 // correction-form GEMM (see GemmProb::dA/dB); bf16 = 1 rounds the operands to
 // BF16 for V_MFMA_F32_16X16X32_BF16 (FP32 accumulation; tile kinds 32, 64 and
 // 256 = 128x128 output tiles), 0 keeps FP64 (tile kind 64 only)

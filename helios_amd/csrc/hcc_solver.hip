@@ -460,11 +460,6 @@ static void force_split(GemmProb& p, int ks) {
   }
 }
 
-// layouts and changing operands of a correction-form problem
-static void set_dual_modes(GemmProb& p) {
-  p.modes = p.a_kfast | (p.b_nfast << 1) | ((p.dA != nullptr) << 2) | ((p.dB != nullptr) << 3);
-}
-
 // Few molecules: every large problem is dealt out to the 8 XCDs in equal
 // parts (its own copy of the problem each, lt0 its first tile), the small ones
 // to the least loaded XCD.  Contiguous runs of equal predicted cost would give
@@ -530,9 +525,6 @@ static GemmTable build_group(Batch& b, std::vector<GemmProb> probs, int ts) {
     large = large || t.htiles.back() >= kSpreadTiles;
     // matrix work of a tile plus the equivalent of its set-up, first loads and stores
     t.hcost.push_back((float)(p.kchunk + 96));
-    p.a_kfast = unit_cols(p.A) ? 1 : (unit_rows(p.A) ? 0 : 1);
-    p.b_nfast = unit_cols(p.B) ? 1 : (unit_rows(p.B) ? 0 : 1);
-    if (p.Cd != nullptr) set_dual_modes(p);
     if (p.ksplit > 1) ws_total += (long)p.ksplit * p.M * p.N;
     t.short_k = t.short_k && p.kchunk <= 64;
   }
@@ -585,6 +577,7 @@ static int plan_problem(Batch& b, GemmProb& p, int k, bool allow_split, int forc
   if (p.M >= kMaxIndex || p.N >= kMaxIndex || p.K >= kMaxIndex) throw std::string("GEMM dimension out of range");
   p.mol = k;
   if (p.Cd == nullptr) set_f64_modes(p);
+  else set_dual_modes(p, b.mixed_bf16);
   int ts = 0, ks = -1;
   if (force_tile) {
     ts = force_tile;
@@ -806,7 +799,8 @@ static void allocate(Batch& b, bool keep_mp2) {
         off[k] = total;
         total += (f.size(b.n[k], b.o[k], b.v[k]) + 63) / 64 * 64;   // 256-byte aligned blocks
       }
-      float* base = b.dalloc<float>(total);
+      // a quad of the last element's row reads three elements more
+      float* base = b.dalloc<float>(total + 4);
       for (int k = 0; k < b.nm; ++k) b.hd[k].*(f.dmember) = base + off[k];
     }
     b.ddm = b.upload(b.hd);
@@ -815,7 +809,8 @@ static void allocate(Batch& b, bool keep_mp2) {
       const Mol& last = b.hm[b.nm - 1];
       double* base = first.*(f.member);
       const long count = (last.*(f.member) - base) + f.size(last.n, last.o, last.v);
-      Batch::Shadow sh{base, count, b.dalloc<__bf16>(count), variable, false};
+      // the 12 bytes around the last elements' quads reach 5 elements more
+      Batch::Shadow sh{base, count, b.dalloc<__bf16>(count + 8), variable, false};
       for (int k = 0; k < b.nm; ++k) {
         sh.hoff.push_back(b.hm[k].*(f.member) - base);
         sh.hlen.push_back(f.size(b.n[k], b.o[k], b.v[k]));
@@ -3410,18 +3405,18 @@ int hcc_selftest_gemm_correction(int m, int n, int k, int a_kfast, int b_nfast, 
     const long na = (long)m * k, nb = (long)k * n, nc = (long)m * n;
     HCHECK(hipMalloc(&a0, sizeof(double) * na));
     HCHECK(hipMalloc(&b0, sizeof(double) * nb));
-    HCHECK(hipMalloc(&ha, sizeof(__bf16) * na));
-    HCHECK(hipMalloc(&hb, sizeof(__bf16) * nb));
+    HCHECK(hipMalloc(&ha, sizeof(__bf16) * (na + 8)));
+    HCHECK(hipMalloc(&hb, sizeof(__bf16) * (nb + 8)));
     HCHECK(hipMalloc(&cd, sizeof(float) * nc));
     HCHECK(hipMemcpy(a0, A0, sizeof(double) * na, hipMemcpyHostToDevice));
     HCHECK(hipMemcpy(b0, B0, sizeof(double) * nb, hipMemcpyHostToDevice));
     HCHECK(hipMemcpy(cd, Cd, sizeof(float) * nc, hipMemcpyHostToDevice));
     if (dA) {
-      HCHECK(hipMalloc(&da, sizeof(float) * na));
+      HCHECK(hipMalloc(&da, sizeof(float) * (na + 4)));
       HCHECK(hipMemcpy(da, dA, sizeof(float) * na, hipMemcpyHostToDevice));
     }
     if (dB) {
-      HCHECK(hipMalloc(&db, sizeof(float) * nb));
+      HCHECK(hipMalloc(&db, sizeof(float) * (nb + 4)));
       HCHECK(hipMemcpy(db, dB, sizeof(float) * nb, hipMemcpyHostToDevice));
     }
     to_bf16(a0, ha, na, nullptr);
@@ -3437,12 +3432,10 @@ int hcc_selftest_gemm_correction(int m, int n, int k, int a_kfast, int b_nfast, 
     p.hB = hb;
     p.tiles_n = (n + tile - 1) / tile;
     p.tile_begin = 0;
-    p.a_kfast = a_kfast ? 1 : 0;
-    p.b_nfast = b_nfast ? 1 : 0;
+    set_dual_modes(p, true);
     p.ksplit = 1;
-    p.kchunk = k;
+    p.kchunk = p.kpad;
     const int tiles = ((m + tile - 1) / tile) * p.tiles_n;
-    set_dual_modes(p);
     const XcdMap xcd = xcd_runs({tiles}, {1.f});
     HCHECK(hipMalloc(&dp, sizeof(GemmProb)));
     HCHECK(hipMemcpy(dp, &p, sizeof(p), hipMemcpyHostToDevice));

@@ -172,3 +172,26 @@ def test_tile_bands_correction(tile, m, n, k, kinds, a_kfast, b_nfast):
     ref = 0.5 * (A0 @ b + a @ (B0 + b)) + C0
     mag = 0.5 * (np.abs(A0) @ np.abs(b) + np.abs(a) @ (np.abs(B0) + np.abs(b)))
     assert (np.abs(C - ref) <= 2.0 ** -7 * mag + 2.0 ** -23 * (np.abs(C0) + mag)).all()
+
+
+def test_correction_residual_at_every_run_length():
+    """BF16 corrections over composite K of every run length modulo 4 (n_occ =
+    n_virt = 5 .. 23) against the FP64 corrections.  Each outer step of the
+    exact form contracts the residual by kappa = 0.05; BF16 rounding (2^-8 per
+    factor, a few factors deep) adds about 0.02, so from 1 to 1e-8 the
+    ln(1e8) / ln(1/0.05) = 6.1 outer steps become ln(1e8) / ln(1/0.07) = 6.9: at
+    most two more in whole steps.  A product missing or repeating elements is
+    off by an order of its own size and needs several times as many."""
+    mols = [ppp.prepare(M.random_fragment(2 * o, seed=o)) for o in (5, 6, 7, 8, 9, 10, 11, 14, 17, 23)]
+    outer = {}
+    for bf16 in (False, True):
+        ctx = capi.Context(0, capi.HCC_MIXED, 8)
+        ctx.set_mixed(bf16=bf16, kappa=0.05, max_inner=60, max_outer=40)
+        ctx.batch_load(mols)
+        ctx.batch_solve(capi.GUESS_MP2, 4000, 1e-8)
+        _, _, st = ctx.batch_results()
+        outer[bf16], inner = ctx.batch_statistics()
+        ctx.close()
+        print("bf16", bf16, "outer", outer[bf16], "inner", inner)
+        assert (st == 1).all()
+    assert (outer[True] <= outer[False] + 2).all()
