@@ -436,7 +436,7 @@ def main():
         rooflines["roofline_update"] = {
             "bound": "hbm", "achieved": upd_b / (upd_ms * 1e-3) / 1e9, "peak": PEAK_HBM / 1e9, "unit": "GB/s",
             "frac": upd_b / (upd_ms * 1e-3) / PEAK_HBM, "kernel_ms": upd_ms,
-            "kernel": "k_update1 + k_update2 (FP64 solver)", "work": "24 o^2 v^2 bytes per molecule-iteration"}
+            "kernel": "k_update (FP64 solver)", "work": "24 o^2 v^2 bytes per molecule-iteration"}
         diis_ms = float(ms[65])
         dbytes = float(diis_bytes(o, v, its, args.diis).sum())
         rooflines["roofline_diis"] = {

@@ -7,14 +7,15 @@ namespace hcc {
 constexpr int kEwThreads = 256;
 constexpr int kDotItems = 8;   // elements per thread of a DIIS dot-product workgroup
 constexpr int kPItems = 4;     // elements per thread of the P / PT builders (table rgN3)
-// elements per thread of k_u, k_assemble, k_update2, k_update2_mixed (table rgT2x, whose
+// elements per thread of k_u_xx, k_assemble, k_update, k_update_mixed (table rgT2x, whose
 // block prefix also indexes their max|d| partials) and k_zero_delta, k_commit_delta (rgT2Sx)
 constexpr int kEwItems = 4;
 constexpr int kMaxDiis = 32;
 
 void ew_dress(const Mol* mols, const State* st, Ragged rgNN, int nm, hipStream_t s);
-void ew_fock_m(const Mol* mols, const State* st, Ragged rgN, Ragged rgNN, int nm, hipStream_t s);
-void ew_pouter(const Mol* mols, const State* st, Ragged rgN3, int nm, hipStream_t s);
+// P, PT and dvec from Xf and Yf; then M (reads dvec)
+void ew_pouter(const Mol* mols, const State* st, Ragged rgN3, Ragged rgN, hipStream_t s);
+void ew_fock_m(const Mol* mols, const State* st, Ragged rgNN, int nm, hipStream_t s);
 // u = 2 t2 - t2(a<->b) and the Fock parts of the E2 intermediates
 void ew_u_xx(const Mol* mols, const State* st, Ragged rgT2, Ragged rgXX, hipStream_t s);
 void ew_u_xx(const MolD* mols, const State* st, Ragged rgT2, Ragged rgXX, hipStream_t s);

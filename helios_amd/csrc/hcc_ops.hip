@@ -107,9 +107,9 @@ __device__ __forceinline__ double dressed_density(const Mol& M, int mu, int nu) 
 }
 
 // dvec[mu] = dD[mu][mu]
-__global__ __launch_bounds__(kEwThreads) void k_fock_diag(const Mol* __restrict__ mols, const State* __restrict__ st,
-                                                         Ragged rg, int nm) {
-  RAGGED_PROLOGUE((long)mols[mol].n);
+__device__ __forceinline__ void fock_diag_block(const Mol* __restrict__ mols, const State* __restrict__ st, const Ragged& rg,
+                                                int block) {
+  RAGGED_PROLOGUE_OF(block, (long)mols[mol].n);
   if (e >= size_ || !st[mol].active) return;
   M.dvec[e] = dressed_density(M, (int)e, (int)e);
 }
@@ -132,9 +132,9 @@ __global__ __launch_bounds__(kEwThreads) void k_fock_m(const Mol* __restrict__ m
 // P[mu][p*N+q] = Xf[mu][p] * Yf[mu][q] and its transpose PT[mu][p*N+q] = P[mu][q*N+p];
 // kPItems elements per thread (the ragged table of these kernels counts
 // kEwThreads * kPItems elements per workgroup)
-__global__ __launch_bounds__(kEwThreads) void k_pouter(const Mol* __restrict__ mols, const State* __restrict__ st,
-                                                      Ragged rg, int nm) {
-  RAGGED_PROLOGUE((long)mols[mol].n * mols[mol].n * mols[mol].n);
+__device__ __forceinline__ void pouter_block(const Mol* __restrict__ mols, const State* __restrict__ st, const Ragged& rg,
+                                             int block) {
+  RAGGED_PROLOGUE_OF(block, (long)mols[mol].n * mols[mol].n * mols[mol].n);
   if (!st[mol].active) return;
   const int N = M.n, N2 = N * N;
   const gptr<double> X = global_view(M.Xf), Y = global_view(M.Yf);
@@ -162,6 +162,12 @@ __global__ __launch_bounds__(kEwThreads) void k_pouter(const Mol* __restrict__ m
       PT[f] = xq[it] * yp[it];
     }
   }
+}
+// P, PT and, in the last workgroups, dvec: all that needs only Xf and Yf
+__global__ __launch_bounds__(kEwThreads) void k_pouter(const Mol* __restrict__ mols, const State* __restrict__ st,
+                                                      Ragged rgN3, Ragged rgN) {
+  if ((int)blockIdx.x < rgN3.nblocks) pouter_block(mols, st, rgN3, blockIdx.x);
+  else fock_diag_block(mols, st, rgN, blockIdx.x - rgN3.nblocks);
 }
 
 // u = 2 t2 - t2(a<->b); kEwItems elements per thread, loads before stores
@@ -350,10 +356,9 @@ __device__ __forceinline__ double diis_combine(const State& S, const T* x, long 
 }
 
 // Singles: d1 = w1 + Ft_ai; t1 += s1 d1 / (F_ii - F_aa).  size o*v
-__global__ __launch_bounds__(kEwThreads) void k_update1(const Mol* __restrict__ mols, const State* __restrict__ st,
-                                                       Ragged rg, int nm, Params prm, double* __restrict__ part) {
-  __shared__ double sh[kEwThreads / 64];
-  RAGGED_PROLOGUE((long)mols[mol].o * mols[mol].v);
+__device__ __forceinline__ void update1_block(const Mol* __restrict__ mols, const State* __restrict__ st, const Ragged& rg,
+                                              int block, const Params& prm, double* __restrict__ part, double* sh) {
+  RAGGED_PROLOGUE_OF(block, (long)mols[mol].o * mols[mol].v);
   if (!st[mol].active) return;
   double amax = 0.0;
   if (e < size_) {
@@ -372,7 +377,7 @@ __global__ __launch_bounds__(kEwThreads) void k_update1(const Mol* __restrict__ 
     }
   }
   const double r = block_max(amax, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = r;
+  if (threadIdx.x == 0) part[block] = r;
 }
 
 // Index set of element g of an o x o x v x v array for the pair updates: the
@@ -405,10 +410,9 @@ __device__ __forceinline__ PairIx pair_ix(long g, int o, int v) {
 // kEwItems elements per thread (table rgT2x), loads before stores.  The
 // representative of each pair updates both of its elements and contributes the
 // pair's max|d|; a non-representative element reads nothing.
-__global__ __launch_bounds__(kEwThreads) void k_update2(const Mol* __restrict__ mols, const State* __restrict__ st,
-                                                       Ragged rg, int nm, Params prm, double* __restrict__ part) {
-  __shared__ double sh[kEwThreads / 64];
-  RAGGED_PROLOGUE((long)mols[mol].o * mols[mol].o * mols[mol].v * mols[mol].v);
+__device__ __forceinline__ void update2_block(const Mol* __restrict__ mols, const State* __restrict__ st, const Ragged& rg,
+                                              int block, const Params& prm, double* __restrict__ part, double* sh) {
+  RAGGED_PROLOGUE_OF(block, (long)mols[mol].o * mols[mol].o * mols[mol].v * mols[mol].v);
   if (!st[mol].active) return;
   const int N = M.n, o = M.o, v = M.v;
   const gptr<double> w2 = global_view(M.w2), F = global_view(M.F), t2in = global_view(M.t2);
@@ -451,11 +455,21 @@ __global__ __launch_bounds__(kEwThreads) void k_update2(const Mol* __restrict__ 
     }
   }
   const double rr = block_max(amax, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = rr;
+  if (threadIdx.x == 0) part[block] = rr;
+}
+
+// the FP64 step in one launch: doubles, then singles (nothing of one is read
+// by the other; a launch more costs 4.4 us, 5 % of a small molecule's iteration)
+__global__ __launch_bounds__(kEwThreads) void k_update(const Mol* __restrict__ mols, const State* __restrict__ st,
+                                                      Ragged rgOV, Ragged rgT2, Params prm, double* __restrict__ part1,
+                                                      double* __restrict__ part2) {
+  __shared__ double sh[kEwThreads / 64];
+  if ((int)blockIdx.x < rgT2.nblocks) update2_block(mols, st, rgT2, blockIdx.x, prm, part2, sh);
+  else update1_block(mols, st, rgOV, blockIdx.x - rgT2.nblocks, prm, part1, sh);
 }
 
 // Reference-form residuals for the parity interface: d1 (already final in w1
-// after k_update1 is NOT assumed; computed here from Omega) and
+// after k_update is NOT assumed; computed here from Omega) and
 // d2 = 2 Omega_sym - Omega_sym(a<->b), both in row-major [i][a] / [i][j][a][b].
 __global__ __launch_bounds__(kEwThreads) void k_contravariant(const Mol* __restrict__ mols, Ragged rg, int nm,
                                                              double* __restrict__ d1, double* __restrict__ d2,
@@ -908,12 +922,12 @@ __global__ void k_activate(State* __restrict__ st, int* __restrict__ act, int nm
 void ew_dress(const Mol* mols, const State* st, Ragged rgNN, int nm, hipStream_t s) {
   RAGGED_LAUNCH(k_dress, rgNN, mols, st, rgNN, nm);
 }
-void ew_fock_m(const Mol* mols, const State* st, Ragged rgN, Ragged rgNN, int nm, hipStream_t s) {
-  RAGGED_LAUNCH(k_fock_diag, rgN, mols, st, rgN, nm);
-  RAGGED_LAUNCH(k_fock_m, rgNN, mols, st, rgNN, nm);
+void ew_pouter(const Mol* mols, const State* st, Ragged rgN3, Ragged rgN, hipStream_t s) {
+  const int blocks = rgN3.nblocks + rgN.nblocks;
+  if (blocks > 0) hipLaunchKernelGGL(k_pouter, dim3(blocks), dim3(kEwThreads), 0, s, mols, st, rgN3, rgN);
 }
-void ew_pouter(const Mol* mols, const State* st, Ragged rgN3, int nm, hipStream_t s) {
-  RAGGED_LAUNCH(k_pouter, rgN3, mols, st, rgN3, nm);
+void ew_fock_m(const Mol* mols, const State* st, Ragged rgNN, int nm, hipStream_t s) {
+  RAGGED_LAUNCH(k_fock_m, rgNN, mols, st, rgNN, nm);
 }
 template <class MT>
 static void ew_u_xx_t(const MT* mols, const State* st, Ragged rgT2, Ragged rgXX, hipStream_t s) {
@@ -938,8 +952,8 @@ void ew_assemble(const MolD* mols, const State* st, Ragged rgT2, int nm, hipStre
 }
 void ew_update(const Mol* mols, const State* st, Ragged rgOV, Ragged rgT2, int nm, const Params& prm,
                double* part1, double* part2, hipStream_t s) {
-  RAGGED_LAUNCH(k_update1, rgOV, mols, st, rgOV, nm, prm, part1);
-  RAGGED_LAUNCH(k_update2, rgT2, mols, st, rgT2, nm, prm, part2);
+  const int blocks = rgT2.nblocks + rgOV.nblocks;
+  if (blocks > 0) hipLaunchKernelGGL(k_update, dim3(blocks), dim3(kEwThreads), 0, s, mols, st, rgOV, rgT2, prm, part1, part2);
 }
 void ew_contravariant(const Mol* mols, Ragged rgT2S, int nm, double* d1, double* d2, hipStream_t s) {
   RAGGED_LAUNCH(k_contravariant, rgT2S, mols, rgT2S, nm, d1, d2, 0L, 0L);
@@ -1411,11 +1425,10 @@ void mixed_e2(const Mol* m0, const MolD* md, const State* st, Ragged rgOcc, int 
 }
 
 // mixed update, singles: Omega1 = (w1_0 incl. F~_ai) + dw1 + dF~_ai; T = t1_0 + dt1
-__global__ __launch_bounds__(kEwThreads) void k_update1_mixed(const Mol* __restrict__ mols, const MolD* __restrict__ dmols,
-                                                             const State* __restrict__ st, Ragged rg, int nm, Params prm,
-                                                             double* __restrict__ part) {
-  __shared__ double sh[kEwThreads / 64];
-  RAGGED_PROLOGUE((long)mols[mol].o * mols[mol].v);
+__device__ __forceinline__ void update1_mixed_block(const Mol* __restrict__ mols, const MolD* __restrict__ dmols,
+                                                    const State* __restrict__ st, const Ragged& rg, int block,
+                                                    const Params& prm, double* __restrict__ part, double* sh) {
+  RAGGED_PROLOGUE_OF(block, (long)mols[mol].o * mols[mol].v);
   if (!st[mol].active) return;
   double amax = 0.0;
   if (e < size_) {
@@ -1437,15 +1450,14 @@ __global__ __launch_bounds__(kEwThreads) void k_update1_mixed(const Mol* __restr
     }
   }
   const double r = block_max(amax, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = r;
+  if (threadIdx.x == 0) part[block] = r;
 }
 
-// mixed update, doubles (pair representatives as in k_update2); DIIS stores corrections
-__global__ __launch_bounds__(kEwThreads) void k_update2_mixed(const Mol* __restrict__ mols, const MolD* __restrict__ dmols,
-                                                             const State* __restrict__ st, Ragged rg, int nm, Params prm,
-                                                             double* __restrict__ part) {
-  __shared__ double sh[kEwThreads / 64];
-  RAGGED_PROLOGUE((long)mols[mol].o * mols[mol].o * mols[mol].v * mols[mol].v);
+// mixed update, doubles (pair representatives as in update2_block); DIIS stores corrections
+__device__ __forceinline__ void update2_mixed_block(const Mol* __restrict__ mols, const MolD* __restrict__ dmols,
+                                                    const State* __restrict__ st, const Ragged& rg, int block,
+                                                    const Params& prm, double* __restrict__ part, double* sh) {
+  RAGGED_PROLOGUE_OF(block, (long)mols[mol].o * mols[mol].o * mols[mol].v * mols[mol].v);
   if (!st[mol].active) return;
   const MolD& Dm = dmols[mol];
   const int N = M.n, o = M.o, v = M.v;
@@ -1453,7 +1465,7 @@ __global__ __launch_bounds__(kEwThreads) void k_update2_mixed(const Mol* __restr
   const gptr<float> dw2 = global_view(Dm.w2), dt2in = global_view(Dm.t2);
   const gwptr<float> dt2 = global_out(Dm.t2), sd = global_out(Dm.sd), stv = global_out(Dm.st);
   const long f0 = (long)lb * kEwItems * kEwThreads + threadIdx.x;
-  // kEwItems elements per thread, loads before stores (as in k_update2)
+  // kEwItems elements per thread, loads before stores (as in update2_block)
   PairIx q[kEwItems];
   double om[kEwItems], omx[kEwItems], dd[kEwItems], t0[kEwItems];
   float dw[kEwItems], dwx[kEwItems], dt[kEwItems];
@@ -1500,7 +1512,17 @@ __global__ __launch_bounds__(kEwThreads) void k_update2_mixed(const Mol* __restr
     }
   }
   const double rr = block_max(amax, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = rr;
+  if (threadIdx.x == 0) part[block] = rr;
+}
+
+// the inner step in one launch (as k_update)
+__global__ __launch_bounds__(kEwThreads) void k_update_mixed(const Mol* __restrict__ mols, const MolD* __restrict__ dmols,
+                                                            const State* __restrict__ st, Ragged rgOV, Ragged rgT2,
+                                                            Params prm, double* __restrict__ part1,
+                                                            double* __restrict__ part2) {
+  __shared__ double sh[kEwThreads / 64];
+  if ((int)blockIdx.x < rgT2.nblocks) update2_mixed_block(mols, dmols, st, rgT2, blockIdx.x, prm, part2, sh);
+  else update1_mixed_block(mols, dmols, st, rgOV, blockIdx.x - rgT2.nblocks, prm, part1, sh);
 }
 
 // after the FP64 residual at the outer point: acc0, convergence, inner set-up
@@ -1648,8 +1670,9 @@ void mixed_commit(const Mol* m0, const MolD* md, const State* st, Ragged rgT2S, 
 }
 void mixed_update(const Mol* m0, const MolD* md, const State* st, Ragged rgOV, Ragged rgT2, int nm, const Params& prm,
                   double* part1, double* part2, hipStream_t s) {
-  RAGGED_LAUNCH(k_update1_mixed, rgOV, m0, md, st, rgOV, nm, prm, part1);
-  RAGGED_LAUNCH(k_update2_mixed, rgT2, m0, md, st, rgT2, nm, prm, part2);
+  const int blocks = rgT2.nblocks + rgOV.nblocks;
+  if (blocks > 0)
+    hipLaunchKernelGGL(k_update_mixed, dim3(blocks), dim3(kEwThreads), 0, s, m0, md, st, rgOV, rgT2, prm, part1, part2);
 }
 void mixed_outer_control(const Mol* mols, State* st, int* act, int nm, const Params& prm, int max_outer, Ragged rgOV,
                          const double* part1, Ragged rgT2, const double* part2, hipStream_t s) {

@@ -1171,9 +1171,9 @@ using namespace hcc;
 constexpr int kProfSlots = 96;
 static_assert(kProfSlots == 96, "profile slot arrays are sized 96");
 enum ProfGroup {
-  kProfUpdate = 64,        // k_update1 + k_update2 (FP64 step, DIIS push fused)
+  kProfUpdate = 64,        // k_update (FP64 step, DIIS push fused)
   kProfDiis = 65,          // k_diis_dot + k_diis_solve + k_diis_extrap (FP64)
-  kProfUpdateMixed = 66,   // k_update1_mixed + k_update2_mixed (inner step)
+  kProfUpdateMixed = 66,   // k_update_mixed (inner step)
   kProfDiisMixed = 67,     // DIIS over the FP32 corrections (inner)
   kProfE2 = 68,            // k_e2 (FP64)
   kProfE2Mixed = 69,       // k_e2_d (correction form)
@@ -1455,8 +1455,8 @@ static void residual(hcc_ctx* c) {
   hipStream_t s = c->stream;
   prof_open(c, kProfResidualEw);
   ew_dress(b.dm, b.dst, b.rgNN, b.nm, s);
-  ew_fock_m(b.dm, b.dst, b.rgN, b.rgNN, b.nm, s);
-  ew_pouter(b.dm, b.dst, b.rgN3, b.nm, s);
+  ew_pouter(b.dm, b.dst, b.rgN3, b.rgN, s);
+  ew_fock_m(b.dm, b.dst, b.rgNN, b.nm, s);
   prof_close(c);
   if (c->prof) need_op_tables(b);
   for (int l = 0; l < (int)b.lv.size(); ++l) {
@@ -1561,7 +1561,7 @@ static void precompute(hcc_ctx* c) {
   gemm(c, b.pre[1], 61);
   prof_open(c, kProfPrecomputeEw);
   ew_dress(b.dm, b.dst, b.rgNN, b.nm, s);
-  ew_pouter(b.dm, b.dst, b.rgN3, b.nm, s);
+  ew_pouter(b.dm, b.dst, b.rgN3, Ragged{}, s);
   prof_close(c);
   gemm(c, b.g1, 62);
   gemm(c, b.pre[2], 63);
@@ -1980,7 +1980,7 @@ int hcc_batch_triples(hcc_ctx* ctx, double* energies, double* e_t) {
   arm_all(b.dst, b.dact, b.dtsave, b.nm, false, s);
   zero_t1(b.dm, b.rgOV, b.nm, s);
   ew_dress(b.dm, b.dst, b.rgNN, b.nm, s);
-  ew_pouter(b.dm, b.dst, b.rgN3, b.nm, s);
+  ew_pouter(b.dm, b.dst, b.rgN3, Ragged{}, s);
   prof_close(ctx);
   gemm(ctx, b.g1, 62);
   gemm(ctx, b.tpre[0], 58);
