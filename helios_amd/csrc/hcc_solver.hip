@@ -2034,12 +2034,18 @@ static void setup_lr(Batch& b) {
   b.lr_n2 = n2;
   b.lr_span1 = (long)(last.t1 - first.t1) + (long)last.o * last.v;
   b.lr_span2 = (long)(last.t2 - first.t2) + (long)last.o * last.o * last.v * last.v;
-  b.dlr_r1 = b.dalloc<double>(n1);
-  b.dlr_r2 = b.dalloc<double>(n2);
-  b.dlr_s1 = b.dalloc<double>(n1);
-  b.dlr_s2 = b.dalloc<double>(n2);
-  b.dlr_t1b = b.dalloc<double>(b.lr_span1);
-  b.dlr_t2b = b.dalloc<double>(b.lr_span2);
+  // one block for all six (256-byte aligned parts): the first product of a
+  // batch pays for these allocations
+  const long part[6] = {n1, n2, n1, n2, b.lr_span1, b.lr_span2};
+  double** const at[6] = {&b.dlr_r1, &b.dlr_r2, &b.dlr_s1, &b.dlr_s2, &b.dlr_t1b, &b.dlr_t2b};
+  auto up = [](long x) { return (x + 31) / 32 * 32; };
+  long total = 0;
+  for (long x : part) total += up(x);
+  double* p = b.dalloc<double>(total);
+  for (int q = 0; q < 6; ++q) {
+    *at[q] = p;
+    p += up(part[q]);
+  }
   long a1 = 0, a2 = 0;
   for (int k = 0; k < nm; ++k) {
     pc[k] = b.dlr_r1 + a1;
