@@ -107,7 +107,7 @@ def triples_leg(ctx, o, v):
     fl = float(f_triples(o, v).sum())
     out = {"bound": "mfma", "achieved": fl / (kms * 1e-3) / 1e12, "peak": PEAK_FP64 / 1e12, "unit": "TFLOP/s",
            "frac": fl / (kms * 1e-3) / PEAK_FP64,
-           "kernel": "k_triples_mfma (FP64 matrix cores, W in LDS; k_triples for v > 24)", "kernel_ms": kms,
+           "kernel": "k_triples_mfma, k_triples_blocked (FP64 matrix cores, W in LDS; k_triples for v > 32)", "kernel_ms": kms,
            "integral_gemm_ms": float(ops[58] + ops[59] + ops[62]), "setup_ew_ms": float(ops[79]),
            "wall_ms_incl_readback": wall * 1e3, "molecules": int(len(o)),
            "mean_e_t_eV": float(et.sum(1).mean()),

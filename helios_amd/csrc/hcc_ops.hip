@@ -215,7 +215,7 @@ __device__ __forceinline__ void init_xx_block(const MT* __restrict__ mols, const
   }
 }
 
-// k_u and k_init_xx in one launch (both precede the contractions that read u,
+// u and the initial Xvv, Xoo in one launch (both precede the contractions that read u,
 // Xvv and Xoo): workgroups past the first table's are the second's
 template <class MT>
 __global__ __launch_bounds__(kEwThreads) void k_u_xx(const MT* __restrict__ mols, const State* __restrict__ st, Ragged rgT2,

@@ -288,7 +288,7 @@ int hcc_gemm_flops_correction(hcc_ctx* ctx, double* per_inner_iteration);
  * of the iteration (0..24 in launch order), 32+k for its correction form
  * (mixed solver), 60..63 for the set-up GEMMs, 58 and 59 for the (T)
  * integral blocks; then elementwise groups:
- * 64 FP64 update (k_update1/2 with the DIIS push), 65 FP64 DIIS (dots, solve,
+ * 64 FP64 update (k_update with the DIIS push), 65 FP64 DIIS (dots, solve,
  * extrapolation), 66 mixed inner update, 67 mixed inner DIIS, 68 E2 pass,
  * 69 its correction form, 70 residual elementwise (dressing, Fock, P/PT, u,
  * assembly), 71 its correction form, 72 outer-point residual norms, 73 commit
