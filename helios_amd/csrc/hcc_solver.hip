@@ -1126,11 +1126,43 @@ static void build_levels(Batch& b) {
   b.lv = level_tables(b, false, [&](int op, int k) { return b.ops[op](b.hm[k]); });
 }
 
+// How far a loaded batch's memory and table list reach: drop() gives back what
+// was built since, which nothing may refer to any more.
+struct TableMark {
+  Batch& b;
+  const size_t nalloc, nalt, nchunk, used, arena_used;
+  explicit TableMark(Batch& batch)
+      : b(batch), nalloc(b.allocs.size()), nalt(b.alt.size()), nchunk(b.chunks.size()),
+        used(nchunk ? b.chunks.back().used : 0), arena_used(b.arena_used) {}
+  void drop() {
+    for (size_t q = nalloc; q < b.allocs.size(); ++q) (void)hipFree(b.allocs[q].p);
+    b.allocs.resize(nalloc);
+    b.chunks.resize(nchunk);
+    if (nchunk) b.chunks.back().used = used;
+    b.alt.resize(nalt);
+    b.arena_used = arena_used;
+  }
+};
+// all the tables of `build`, or none of them
+static std::vector<GemmTable> whole_tables(Batch& b, const std::function<std::vector<GemmTable>()>& build) {
+  TableMark mark(b);
+  try {
+    return build();
+  } catch (...) {
+    mark.drop();
+    throw;
+  }
+}
+
 // one table per contraction, for profiled solves and tuning
 static void need_op_tables(Batch& b) {
   if (!b.it.empty()) return;
-  for (int q = 0; q < (int)b.ops.size(); ++q)
-    b.it.push_back(make_table(b, [&](int k) { return b.ops[q](b.hm[k]); }, true, 0, q));
+  b.it = whole_tables(b, [&] {
+    std::vector<GemmTable> t;
+    for (int q = 0; q < (int)b.ops.size(); ++q)
+      t.push_back(make_table(b, [&](int k) { return b.ops[q](b.hm[k]); }, true, 0, q));
+    return t;
+  });
 }
 
 // Correction-form twin of iteration GEMM `op` for molecule k: the FP64
@@ -1157,9 +1189,13 @@ static void build_delta_levels(Batch& b) {
 }
 static void need_delta_op_tables(Batch& b) {
   if (!b.dit.empty()) return;
-  for (int q = 0; q < (int)b.ops.size(); ++q)
-    b.dit.push_back(make_table(b, [&](int k) { return delta_prob(b, q, k); }, true, b.mixed_bf16 ? 0 : 64,
-                               b.mixed_bf16 ? kDualTuneOp + q : -1, 0, b.mixed_bf16));
+  b.dit = whole_tables(b, [&] {
+    std::vector<GemmTable> t;
+    for (int q = 0; q < (int)b.ops.size(); ++q)
+      t.push_back(make_table(b, [&](int k) { return delta_prob(b, q, k); }, true, b.mixed_bf16 ? 0 : 64,
+                             b.mixed_bf16 ? kDualTuneOp + q : -1, 0, b.mixed_bf16));
+    return t;
+  });
 }
 
 }  // namespace hcc
@@ -3164,27 +3200,16 @@ int hcc_tune_gemm(hcc_ctx* ctx, int op, int tile, int ksplit, int reps, double* 
   }
   API_BEGIN
   HCHECK(hipSetDevice(ctx->device));
-  // the table built below is dropped at the end of the call
-  size_t nalloc = b.allocs.size(), nalt = b.alt.size(), nchunk = b.chunks.size(), used = nchunk ? b.chunks.back().used : 0;
-  GemmTable t;
-  auto keep = [&] {
-    nalloc = b.allocs.size();
-    nalt = b.alt.size();
-    nchunk = b.chunks.size();
-    used = nchunk ? b.chunks.back().used : 0;
-  };
-  if (dual && tile == 0) {
-    need_delta_op_tables(b);
-    keep();
-    t = b.dit[q];
-  } else if (dual)
-    t = make_table(b, [&](int k) { return delta_prob(b, q, k); }, true, tile, -1, ksplit > 0 ? ksplit : 1, true);
-  else if (tile == 0) {
-    need_op_tables(b);
-    keep();
-    t = b.it[q];
-  } else
-    t = make_table(b, [&](int k) { return b.ops[q](b.hm[k]); }, true, tile, -1, ksplit > 0 ? ksplit : 1);
+  if (tile == 0 && dual) need_delta_op_tables(b);
+  else if (tile == 0) need_op_tables(b);
+  TableMark mark(b);   // a table built below is dropped at the end of the call
+  const GemmTable t =
+      tile == 0 ? (dual ? b.dit[q] : b.it[q])
+                : whole_tables(b, [&] {
+                    return std::vector<GemmTable>{make_table(
+                        b, [&](int k) { return dual ? delta_prob(b, q, k) : b.ops[q](b.hm[k]); }, true, tile, -1,
+                        ksplit > 0 ? ksplit : 1, dual)};
+                  })[0];
   auto run = [&]() {
     if (dual) launch_delta_table(ctx, t);
     else launch_table(ctx, t);
@@ -3203,11 +3228,7 @@ int hcc_tune_gemm(hcc_ctx* ctx, int op, int tile, int ksplit, int reps, double* 
   *ms = el / reps;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  for (size_t q = nalloc; q < b.allocs.size(); ++q) HCHECK(hipFree(b.allocs[q].p));
-  b.allocs.resize(nalloc);
-  b.chunks.resize(nchunk);
-  if (nchunk) b.chunks.back().used = used;
-  b.alt.resize(nalt);
+  mark.drop();
   ctx->have_guess = false;
   API_END
 }

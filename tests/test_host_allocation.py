@@ -1,0 +1,47 @@
+"""What the library's host code does when device memory runs out, and how much
+of it a load holds: run on the CPU with the HIP runtime replaced (_hoststub)."""
+import pytest
+
+from helios_amd import capi
+from tests import _hoststub
+from tests._hoststub import molecule
+
+
+@pytest.fixture(scope="module")
+def stub_lib(tmp_path_factory):
+    return _hoststub.build(tmp_path_factory.mktemp("hoststub"))
+
+
+def _batch(precision, mols):
+    ctx = capi.Context(0, precision, 8)
+    ctx.set_graphs(False)
+    ctx.batch_load(mols)
+    return ctx
+
+
+# enough molecules that the tables of all contractions outgrow the block the load left
+MANY = [molecule(6, 3)] * 700
+
+
+def _profiled_solve(ctx):
+    ctx.profile(True)
+    ctx.batch_solve(capi.GUESS_MP2, 8, 1e-8)
+
+
+def profiled_solve(stub):
+    stub.each_failure(lambda: _batch(capi.HCC_FP64, MANY), _profiled_solve)
+
+
+def tune_correction_tables(stub):
+    stub.each_failure(lambda: _batch(capi.HCC_MIXED, MANY), lambda ctx: [ctx.tune_gemm(100 + q, 0, 0, 1) for q in range(25)])
+
+
+def tune_own_tables(stub):
+    stub.each_failure(lambda: _batch(capi.HCC_FP64, MANY), lambda ctx: [ctx.tune_gemm(q, 0, 0, 1) for q in range(25)])
+
+
+@pytest.mark.parametrize("function", [profiled_solve, tune_own_tables, tune_correction_tables], ids=lambda f: f.__name__)
+def test_tables_per_contraction_after_a_failed_build(stub_lib, function):
+    """A profiled solve and a tuning call build tables of their own; when that
+    fails half-way, the next one builds them again."""
+    _hoststub.check(stub_lib, function)
