@@ -1182,10 +1182,18 @@ static GemmProb delta_prob(Batch& b, int op, int k) {
 }
 
 // correction-form twins of the iteration GEMMs (BF16 tiles chosen per
-// problem, or FP64 64x64 tiles in exact mode)
-static void build_delta_levels(Batch& b) {
+// problem, or FP64 64x64 tiles in exact mode); the batch keeps its form and
+// tables when those of the other one cannot be built
+static void build_delta_levels(Batch& b, bool bf16) {
+  const bool before = b.mixed_bf16;
+  b.mixed_bf16 = bf16;
+  try {
+    b.dlv = whole_tables(b, [&] { return level_tables(b, true, [&](int op, int k) { return delta_prob(b, op, k); }); });
+  } catch (...) {
+    b.mixed_bf16 = before;
+    throw;
+  }
   b.dit.clear();
-  b.dlv = level_tables(b, true, [&](int op, int k) { return delta_prob(b, op, k); });
 }
 static void need_delta_op_tables(Batch& b) {
   if (!b.dit.empty()) return;
@@ -1663,7 +1671,6 @@ static void load(hcc_ctx* c, int nmol, const int* n, const int* nocc, const doub
   b->m = c->diis_steps;
   b->inner_m = c->mixed_diis > 0 ? std::min(c->mixed_diis, c->diis_steps) : c->diis_steps;
   b->mixed = c->precision == HCC_MIXED;
-  b->mixed_bf16 = c->mixed_bf16 != 0;
   b->tuning = c->tuning.empty() ? nullptr : &c->tuning;
   for (int k = 0; k < nmol; ++k) {
     if (n[k] < 2 || nocc[k] < 1 || nocc[k] >= n[k]) throw std::string("invalid molecule dimensions");
@@ -1683,7 +1690,7 @@ static void load(hcc_ctx* c, int nmol, const int* n, const int* nocc, const doub
   allocate(*b, keep_mp2);
   build_tables(*b);
   build_levels(*b);
-  if (b->mixed) build_delta_levels(*b);
+  if (b->mixed) build_delta_levels(*b, c->mixed_bf16 != 0);
   b->flush_uploads();
   // upload, transposing the column-major inputs to row-major: one staging
   // image per arena (molecule blocks at their arena offsets), one copy each;
@@ -1815,18 +1822,17 @@ int hcc_set_mixed(hcc_ctx* ctx, int bf16, double kappa, int max_inner, int max_o
     ctx->err = "invalid mixed-precision options";
     return HCC_E_ARG;
   }
+  const int want = bf16 ? 1 : 0;
+  API_BEGIN
+  // a loaded batch's correction tables depend on the choice (tile kinds)
+  if (want != ctx->mixed_bf16 && ctx->batch != nullptr && ctx->batch->mixed) {
+    HCHECK(hipSetDevice(ctx->device));
+    build_delta_levels(*ctx->batch, want != 0);
+  }
+  ctx->mixed_bf16 = want;
   ctx->kappa = kappa;
   ctx->max_inner = max_inner;
   ctx->max_outer = max_outer;
-  const int want = bf16 ? 1 : 0;
-  if (want == ctx->mixed_bf16) return HCC_OK;
-  ctx->mixed_bf16 = want;
-  // a loaded batch's correction tables depend on the choice (tile kinds)
-  if (ctx->batch == nullptr || !ctx->batch->mixed) return HCC_OK;
-  API_BEGIN
-  HCHECK(hipSetDevice(ctx->device));
-  ctx->batch->mixed_bf16 = want != 0;
-  build_delta_levels(*ctx->batch);
   API_END
 }
 

@@ -1,8 +1,9 @@
 // Host stand-in for the HIP runtime calls of libhelios_ccsd, so that a test
 // without a device can follow what the library's host code asks for: device
-// memory is host memory, a launch runs nothing and is written down (kernel,
-// grid, and which of its pointer arguments are null), and an allocation can be
-// made to fail.  Loaded with RTLD_GLOBAL before the library, whose undefined
+// memory is host memory, a launch is written down (kernel, grid, and which of
+// its pointer arguments are null) and runs nothing, except that the first
+// stub_running() molecules stay active in a solve, and an allocation can be made
+// to fail.  Loaded with RTLD_GLOBAL before the library, whose undefined
 // runtime symbols then resolve here first.
 #include <cxxabi.h>
 
@@ -24,6 +25,7 @@ std::map<const void*, Kernel> kernels;
 std::map<void*, size_t> blocks;
 size_t held = 0, peak = 0;
 long allocations = 0, fail_at = 0;
+int running = 0;   // molecules that a solve's reset kernel leaves active
 std::string launches;
 thread_local Dim3 call_grid, call_block;
 thread_local size_t call_shared;
@@ -63,6 +65,7 @@ extern "C" {
 // test controls: the n-th allocation from now fails (0: none)
 void stub_fail_at(long n) { fail_at = n; }
 long stub_allocations() { return allocations; }
+void stub_running(int n) { running = n; }
 size_t stub_held() { return held; }
 size_t stub_peak(int reset) {
   if (reset) peak = held;
@@ -94,6 +97,10 @@ int hipLaunchKernel(const void* host, Dim3 grid, Dim3 block, void** args, size_t
   for (size_t q = 0; q < k.pointer.size(); ++q)
     if (k.pointer[q]) launches += *static_cast<void**>(args[q]) == nullptr ? '0' : '1';
   launches += '\n';
+  if (k.name.find("k_reset_state") != std::string::npos) {   // (State*, int* active, int molecules)
+    int* const active = *static_cast<int**>(args[1]);
+    for (int q = 0, n = *static_cast<int*>(args[2]); q < n; ++q) active[q] = q < running;
+  }
   return 0;
 }
 

@@ -45,3 +45,32 @@ def test_tables_per_contraction_after_a_failed_build(stub_lib, function):
     """A profiled solve and a tuning call build tables of their own; when that
     fails half-way, the next one builds them again."""
     _hoststub.check(stub_lib, function)
+
+
+def _exact(ctx):
+    ctx.set_mixed(bf16=False, max_inner=3, max_outer=1)
+
+
+def switch_corrections(stub):
+    def make():
+        ctx = _batch(capi.HCC_MIXED, MANY)
+        ctx.set_mixed(bf16=True, max_inner=3, max_outer=1)
+        return ctx
+
+    def solve(ctx):
+        ctx.batch_solve(capi.GUESS_MP2, 8, 1e-8)
+
+    def again(ctx):
+        _exact(ctx)
+        solve(ctx)
+
+    stub.lib.stub_running(len(MANY))
+    assert stub.launches(lambda: again(make())) != stub.launches(lambda: solve(make()))
+    stub.each_failure(make, _exact, solve)
+    stub.each_failure(make, _exact, again)
+
+
+def test_correction_form_after_a_failed_switch(stub_lib):
+    """When the tables of the other correction form cannot be built, the solves
+    that follow run the form that was set before, and the switch can be repeated."""
+    _hoststub.check(stub_lib, switch_corrections)
