@@ -649,17 +649,18 @@ void dalloc(T** p, size_t count) {
 // gradient sums to reduce (65000 samples: 1016 sums of 21 KB instead of 254).
 int samples_per_block(long nb) { return nb <= 16384 ? 64 : 256; }
 
-void ensure_part(hcc_mlp* net, int blocks) {
-  if (blocks <= net->pcap) return;
-  dalloc(&net->part, (size_t)blocks * kMlpParams);
-  net->pcap = blocks;
+// a buffer of `count` times `each` elements; a failed growth leaves none (capacity 0)
+template <class T, class N>
+void grow(T** p, N* cap, N count, size_t each) {
+  if (count <= *cap) return;
+  *cap = 0;
+  dalloc(p, (size_t)count * each);
+  *cap = count;
 }
 
-void ensure_loss(hcc_mlp* net, long blocks) {
-  if (blocks <= net->lcap) return;
-  dalloc(&net->lossp, (size_t)blocks);
-  net->lcap = blocks;
-}
+void ensure_part(hcc_mlp* net, int blocks) { grow(&net->part, &net->pcap, blocks, kMlpParams); }
+
+void ensure_loss(hcc_mlp* net, long blocks) { grow(&net->lossp, &net->lcap, blocks, 1); }
 
 // one mini-batch of nb samples on `blocks` workgroups (those past nb add
 // zero): loss and gradient; update = Adam step

@@ -1,5 +1,6 @@
 """What the library's host code does when device memory runs out, and how much
 of it a load holds: run on the CPU with the HIP runtime replaced (_hoststub)."""
+import numpy as np
 import pytest
 
 from helios_amd import capi
@@ -74,3 +75,23 @@ def test_correction_form_after_a_failed_switch(stub_lib):
     """When the tables of the other correction form cannot be built, the solves
     that follow run the form that was set before, and the switch can be repeated."""
     _hoststub.check(stub_lib, switch_corrections)
+
+
+def _trainer(rows):
+    tr = capi.Trainer(rows)
+    tr.write_samples(np.zeros((rows, capi.MLP_ROW), dtype=np.float32))
+    return tr
+
+
+def trainer_buffers(stub):
+    """Calls on all samples that need larger buffers than the trainer has, and
+    after a failed one a call on a few, which needs no more than it has."""
+    few = lambda tr: tr.gradient(0, 100)
+    stub.each_failure(lambda: _trainer(100000), lambda tr: tr.gradient(), few)
+    stub.each_failure(lambda: _trainer(100000), lambda tr: tr.evaluate(), few)
+    stub.each_failure(lambda: _trainer(100000), lambda tr: tr.train(epochs=1, batch=90000), few)
+    stub.each_failure(lambda: _trainer(100000), lambda tr: tr.gradient())
+
+
+def test_trainer_buffers_after_a_failed_growth(stub_lib):
+    _hoststub.check(stub_lib, trainer_buffers)
