@@ -1303,10 +1303,10 @@ static void compact_table(Batch& b, GemmTable& t, const std::vector<int>& act, h
   if (t.nprob == 0) return;
   const int np = t.nprob;
   if (t.cd == nullptr) {
-    t.cd = b.dalloc<GemmProb>(np);
     t.ctp = b.dalloc<int>(std::max(1, t.tiles));
     t.cbp = b.dalloc<int>(std::max(1, t.red_blocks));
     t.cbuf = b.dalloc<int>(3 * (size_t)np + 2);
+    t.cd = b.dalloc<GemmProb>(np);   // last: all four are there
   }
   // the previous upload from hbuf has completed: a compaction follows a
   // synchronisation of the stream
@@ -1378,8 +1378,8 @@ static bool compact_raggeds(hcc_ctx* c, const std::vector<int>& act, int alive) 
   if (alive > kCompactFrac * (b.rg_live > 0 ? b.rg_live : b.nm)) return false;
   for (Batch::RgComp& r : b.rgc) {
     if (r.cpre == nullptr) {
-      r.cpre = b.dalloc<int>(b.nm + 1);
       r.cbm = b.dalloc<int>(std::max(1, r.full.nblocks));
+      r.cpre = b.dalloc<int>(b.nm + 1);   // last: both are there
     }
     // the previous upload from hbuf has completed (a compaction follows a
     // synchronisation of the stream)
@@ -1987,12 +1987,12 @@ static void setup_triples(Batch& b, int device) {
     tm[k] = TripMol{M.n, M.o, M.v, 0, b.tA[k], b.tB[k], M.Gklcd, M.t1, M.t2, M.F};
   }
   HCHECK(hipDeviceGetAttribute(&b.tcus, hipDeviceAttributeMultiprocessorCount, device));
-  b.dtm = b.upload(tm);
   b.dtrange = b.upload(range);
   b.dtri = b.upload(items);
   b.dtpart = b.dalloc<double>(2 * items.size());
   b.dtout = b.dalloc<double>(2 * (long)nm);
-  b.dtsave = b.dalloc<int>(nm);
+  if (b.dtsave == nullptr) b.dtsave = b.dalloc<int>(nm);
+  b.dtm = b.upload(tm);   // last: marks the set-up as done
 }
 
 int hcc_batch_triples(hcc_ctx* ctx, double* energies, double* e_t) {
@@ -2097,10 +2097,9 @@ static void setup_lr(Batch& b) {
     a1 += (long)b.o[k] * b.v[k];
     a2 += (long)b.o[k] * b.o[k] * b.v[k] * b.v[k];
   }
-  b.dlr_pc = b.dalloc<double*>(pc.size());
-  b.dlr_ps = b.dalloc<double*>(pc.size());
-  HCHECK(hipMemcpy(b.dlr_pc, pc.data(), pc.size() * sizeof(double*), hipMemcpyHostToDevice));
   if (b.dtsave == nullptr) b.dtsave = b.dalloc<int>(nm);
+  b.dlr_ps = b.dalloc<double*>(pc.size());
+  b.dlr_pc = b.upload(pc);   // last: marks the set-up as done
 }
 
 static int lr_ready(hcc_ctx* ctx) {
@@ -2184,8 +2183,8 @@ static int lr_space_impl(hcc_ctx* ctx, const std::vector<int>& counts) {
   HCHECK(hipMalloc(&b.dlr_space, (size_t)std::max<long>(total, 32) * sizeof(double)));
   HCHECK(hipMemsetAsync(b.dlr_space, 0, (size_t)std::max<long>(total, 32) * sizeof(double), ctx->stream));
   if (b.dlr_len == nullptr) {
-    b.dlr_len = b.dalloc<long>(nm);
     b.dlr_base = b.dalloc<long>(nm);
+    b.dlr_len = b.dalloc<long>(nm);   // last: both are there
   }
   HCHECK(hipMemcpy(b.dlr_len, b.lr_len.data(), nm * sizeof(long), hipMemcpyHostToDevice));
   HCHECK(hipMemcpy(b.dlr_base, b.lr_base.data(), nm * sizeof(long), hipMemcpyHostToDevice));
@@ -2232,9 +2231,10 @@ static bool lr_slot_ok(const Batch& b, int mol, int slot) {
 // staging region of at least `bytes` (grown by doubling; contents not kept)
 static char* lr_stage(Batch& b, size_t bytes) {
   if (bytes > b.lr_stage_cap) {
+    const size_t cap = std::max<size_t>(bytes, 2 * b.lr_stage_cap);
+    b.lr_stage_cap = 0;   // until the new region is there
     if (b.dlr_stage) HCHECK(hipFree(b.dlr_stage));
     b.dlr_stage = nullptr;
-    size_t cap = std::max<size_t>(bytes, 2 * b.lr_stage_cap);
     HCHECK(hipMalloc(&b.dlr_stage, cap));
     b.lr_stage_cap = cap;
   }
@@ -2756,8 +2756,8 @@ int hcc_residual(hcc_ctx* ctx, double* d1, double* d2) {
   const int o = b.o[0], v = b.v[0];
   const size_t n1 = (size_t)o * v, n2 = (size_t)o * o * v * v;
   if (b.d1out == nullptr) {
-    b.d1out = b.dalloc<double>(n1);
     b.d2out = b.dalloc<double>(n2);
+    b.d1out = b.dalloc<double>(n1);   // last: both are there
   }
   ew_contravariant(b.dm, b.rgT2S, b.nm, b.d1out, b.d2out, ctx->stream);
   std::vector<double> h1(n1), h2(n2);

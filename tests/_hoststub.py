@@ -51,7 +51,8 @@ class Stub:
         call(obj)
         count = self.lib.stub_allocations() - first
         assert count > 0, "no allocation in the call"
-        want = self.launches(lambda: then(make() if then is not call else obj))
+        fresh = obj if then is call else make()
+        want = self.launches(lambda: then(fresh))
         for k in range(1, count + 1):
             obj = make()
             assert self.fails(lambda: call(obj), k), f"allocation {k} of {count}: failure not reported"

@@ -95,3 +95,62 @@ def trainer_buffers(stub):
 
 def test_trainer_buffers_after_a_failed_growth(stub_lib):
     _hoststub.check(stub_lib, trainer_buffers)
+
+
+def _solved(mols):
+    ctx = _batch(capi.HCC_FP64, mols)
+    ctx.batch_solve(capi.GUESS_MP2, 4, 1e-8)
+    return ctx
+
+
+def triples_setup(stub):
+    # 12 x 5984 work items: their partial sums are an allocation of their own
+    stub.each_failure(lambda: _solved([molecule(34, 32)] * 12), lambda ctx: ctx.batch_triples())
+
+
+def response_setup(stub):
+    # 33000 molecules: each of the pointer lists is an allocation of its own
+    mols = [molecule(2, 1)] * 33000
+    r1, r2 = np.zeros(len(mols)), np.zeros(len(mols))
+    stub.each_failure(lambda: _solved(mols), lambda ctx: ctx.batch_lr_sigma(r1, r2))
+
+
+def response_staging(stub):
+    def make():
+        ctx = _solved([molecule(8, 4)] * 4)
+        ctx.lr_space(4)
+        ctx.lr_gram([[0, 1, 1, 0, 0]], [0])
+        return ctx
+
+    jobs = [[m, 4, 4, 0, 0] for m in range(4)] * 8
+    few = lambda ctx: ctx.lr_gram([[0, 1, 1, 0, 0]], [0])
+    stub.each_failure(make, lambda ctx: ctx.lr_gram(jobs, range(4)), few)
+
+
+def residual_outputs(stub):
+    def make():
+        ctx = capi.Context(0, capi.HCC_FP64, 8)
+        m = molecule(80, 40)
+        ctx.set_molecule(m["C"], m["F"], m["G"], m["nocc"], 0.0)
+        ctx.guess()
+        return ctx
+
+    stub.each_failure(make, lambda ctx: ctx.residual())
+
+
+def compaction(stub):
+    stub.lib.stub_running(100)
+    for precision in (capi.HCC_FP64, capi.HCC_MIXED):
+        def make():
+            ctx = _batch(precision, MANY)
+            ctx.set_mixed(max_inner=3, max_outer=1)
+            return ctx
+        stub.each_failure(make, lambda ctx: ctx.batch_solve(capi.GUESS_MP2, 8, 1e-8))
+
+
+@pytest.mark.parametrize("function", [triples_setup, response_setup, response_staging, residual_outputs, compaction],
+                         ids=lambda f: f.__name__)
+def test_set_up_on_first_use_after_a_failure(stub_lib, function):
+    """What a batch allocates when a call first needs it counts as there only
+    when all of it is."""
+    _hoststub.check(stub_lib, function)
