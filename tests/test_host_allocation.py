@@ -154,3 +154,31 @@ def test_set_up_on_first_use_after_a_failure(stub_lib, function):
     """What a batch allocates when a call first needs it counts as there only
     when all of it is."""
     _hoststub.check(stub_lib, function)
+
+
+def load_peak(stub):
+    """Memory held while a batch replaces another: never more than the larger of the two."""
+    def mols(sizes):
+        return [molecule(n, n // 2) for n in sizes]
+
+    shapes = [mols([20] * 40), mols([26] * 25), mols([8] * 300), mols(range(10, 40, 2)), mols([40])]
+    alone = []
+    for m in shapes:
+        ctx = _batch(capi.HCC_FP64, m)
+        alone.append(stub.lib.stub_held())
+        ctx.close()
+        assert stub.lib.stub_held() == 0
+    ctx = capi.Context(0, capi.HCC_FP64, 8)
+    for first in range(len(shapes)):
+        for second in range(len(shapes)):
+            ctx.batch_load(shapes[first])
+            stub.lib.stub_peak(1)
+            ctx.batch_load(shapes[second])
+            peak, held = stub.lib.stub_peak(0), stub.lib.stub_held()
+            # a block taken again may exceed the request by an eighth and 64 KiB
+            assert held <= 1.125 * alone[second] + (64 << 16), (first, second, held, alone[second])
+            assert peak <= 1.125 * max(alone[first], alone[second]) + (64 << 16), (first, second, peak, alone)
+
+
+def test_load_holds_no_more_than_the_larger_batch(stub_lib):
+    _hoststub.check(stub_lib, load_peak)
