@@ -1910,6 +1910,16 @@ int hcc_batch_load_scf(hcc_ctx* ctx, int nmol, const int* n, const int* n_occ, c
         std::to_string(lds_max) + " bytes per workgroup)";
   std::vector<double> zero_eref(nmol, 0.0);
   load(ctx, nmol, n, n_occ, nullptr, nullptr, gamma, zero_eref.data(), false);
+  // no orbitals yet: a failure from here on leaves no batch, as one in load() does
+  struct Unload {
+    hcc_ctx* c;
+    ~Unload() {
+      if (c == nullptr) return;
+      delete c->batch;
+      c->batch = nullptr;
+      c->pool.trim();
+    }
+  } unload{ctx};
   Batch& b = *ctx->batch;
   // core and Hueckel matrices (row-major; column-major inputs transposed) and work blocks
   long total = 0;
@@ -1943,6 +1953,7 @@ int hcc_batch_load_scf(hcc_ctx* ctx, int nmol, const int* n, const int* n_occ, c
     if (scf_iterations) scf_iterations[k] = res[k].iterations;
     if (scf_status) scf_status[k] = res[k].status;
   }
+  unload.c = nullptr;
   API_END
 }
 

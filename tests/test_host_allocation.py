@@ -182,3 +182,24 @@ def load_peak(stub):
 
 def test_load_holds_no_more_than_the_larger_batch(stub_lib):
     _hoststub.check(stub_lib, load_peak)
+
+
+def scf_load(stub):
+    n = 48   # the three matrices of the molecules are allocations of their own
+    mols = [dict(core=np.eye(n), G=np.eye(n), huckel=np.eye(n), nocc=n // 2)] * 60
+
+    def load(ctx):
+        ctx.batch_load_scf(mols)
+
+    ctx = capi.Context(0, capi.HCC_FP64, 8)
+    first = stub.lib.stub_allocations()
+    load(ctx)
+    count = stub.lib.stub_allocations() - first
+    for k in range(1, count + 1):
+        ctx = capi.Context(0, capi.HCC_FP64, 8)
+        assert stub.fails(lambda: load(ctx), k), k
+        assert stub.fails(lambda: ctx.batch_solve(), 0), f"allocation {k} of {count} failed, yet there is a batch"
+
+
+def test_no_batch_after_a_failed_scf_load(stub_lib):
+    _hoststub.check(stub_lib, scf_load)
