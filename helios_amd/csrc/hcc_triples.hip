@@ -39,6 +39,15 @@ __device__ __forceinline__ double trip_load(__amdgpu_buffer_rsrc_t r, bool in, i
   return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, in ? element * 8 : kTripPad, 0, 0));
 }
 
+// Orders the wave's LDS accesses before this point with those after it, of all
+// its lanes.  LDS serves a wave in program order, so this costs no instruction;
+// it keeps the compiler from moving an access across.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // permutation s of three positions: position k of the permuted triple takes entry kPerm[s][k]
 __constant__ int kPerm[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
 
@@ -256,6 +265,7 @@ k_triples_mfma(const TripMol* __restrict__ mols, const int2* __restrict__ items,
           for (int e = 0; e < 4; ++e)
             if (e < nr) W[rx[e] * sx + ry[e] * sy + z * sz] += acc[ct][e];
         }
+        wave_lds_order();   // other lanes' elements are updated next
         // permutation 2h + 1: columns v + z of the same tiles at x sx + y sz + z sy
 #pragma unroll
         for (int ct = 0; ct < kCt; ++ct) {
@@ -265,6 +275,7 @@ k_triples_mfma(const TripMol* __restrict__ mols, const int2* __restrict__ items,
           for (int e = 0; e < 4; ++e)
             if (e < nr) W[rx[e] * sx + ry[e] * sz + z * sy] += acc[ct][e];
         }
+        wave_lds_order();   // and the next tile's rows share x with this one's
       }
     }
     // energy of the item: L slices (jb|kc), (ia|kc), (ia|jb) (in the B-operand
@@ -504,6 +515,7 @@ __global__ __launch_bounds__(kTbThreads) __attribute__((amdgpu_waves_per_eu(2)))
               *w = h == 0 ? a0[e] : *w + a0[e];
             }
           }
+          wave_lds_order();   // other lanes' elements of the x slab are updated next
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int y = kq + 4 * e;
