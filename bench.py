@@ -31,13 +31,14 @@ PEAK_FP64 = 78.6e12      # MI355X dense FP64 (matrix) FLOP/s
 PEAK_BF16 = 2.5e15
 PEAK_HBM = 8.0e12        # HBM3E bytes/s
 # HBM bytes per dispatch of the dominant kernels on the default 4096-molecule batch
-# with the default solver settings: FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 (factors from a
-# 1 GiB copy), two rocprofv3 --pmc passes of "bench.py --workers 0 --no-cpu --no-lr
-# --skip-reference --steps 1 --warmup 0 --no-profile" summarised in
-# profiles/hbm_traffic_batch4096.md.  A counter pass cannot run inside this process, so
-# other workloads report null.
-GEMM_TRAFFIC_BATCH4096 = 3.285e9        # gemm_f64_kernel, FP64 solve
-DUAL_GEMM_TRAFFIC_BATCH4096 = 1.468e9   # gemm_dual_bf16, mixed solve
+# with the default solver settings, in the profiled solves that the rooflines time (one
+# launch per contraction; the timed solves launch a dependency level at once):
+# FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 (factors from a 1 GiB copy), two rocprofv3 --pmc
+# passes of "bench.py --workers 0 --no-cpu --no-lr --skip-reference --steps 1 --warmup 0"
+# summarised in profiles/hbm_traffic_batch4096.md.  A counter pass cannot run inside this
+# process, so other workloads report null.
+GEMM_TRAFFIC_BATCH4096 = 3.598e9        # gemm_f64_kernel, FP64 solve
+DUAL_GEMM_TRAFFIC_BATCH4096 = 1.336e9   # gemm_dual_bf16, mixed solve
 
 
 def _prep(k):
@@ -107,7 +108,7 @@ def triples_leg(ctx, o, v):
     fl = float(f_triples(o, v).sum())
     out = {"bound": "mfma", "achieved": fl / (kms * 1e-3) / 1e12, "peak": PEAK_FP64 / 1e12, "unit": "TFLOP/s",
            "frac": fl / (kms * 1e-3) / PEAK_FP64,
-           "kernel": "k_triples_mfma, k_triples_blocked (FP64 matrix cores, W in LDS; k_triples for v > 32)", "kernel_ms": kms,
+           "kernel": "k_triples_mfma, k_triples_blocked (FP64 matrix cores, W in LDS; up to 32 virtual orbitals)", "kernel_ms": kms,
            "integral_gemm_ms": float(ops[58] + ops[59] + ops[62]), "setup_ew_ms": float(ops[79]),
            "wall_ms_incl_readback": wall * 1e3, "molecules": int(len(o)),
            "mean_e_t_eV": float(et.sum(1).mean()),
@@ -418,7 +419,7 @@ def main():
                  "unit": "TFLOP/s", "frac": falg64 / (gemm_ms * 1e-3) / PEAK_FP64,
                  "executed_tflops": gemm_exec / (gemm_ms * 1e-3) / 1e12,
                  "traffic": GEMM_TRAFFIC_BATCH4096 if default_workload else None,
-                 "kernel": "gemm_f64_kernel (FP64 solver, all contractions)", "launches": int(r64["launches"]),
+                 "kernel": "gemm_f64_kernel (FP64 solver, all contractions, one launch each)", "launches": int(r64["launches"]),
                  "kernel_ms": gemm_ms, "avg_launch_ms": gemm_ms / max(1, int(r64["launches"])),
                  "work": "F_iter = 2o^2v^4 + 4o^4v^2 + 12o^3v^3 per molecule-iteration"}
         rooflines["roofline_fp64_solver"] = rfp64
@@ -457,7 +458,7 @@ def main():
                         "unit": "TFLOP/s", "frac": falg / (corr_ms * 1e-3) / PEAK_BF16,
                         "executed_tflops": fexec / (corr_ms * 1e-3) / 1e12,
                         "traffic": DUAL_GEMM_TRAFFIC_BATCH4096 if default_workload else None,
-                        "kernel": "gemm_dual_bf16 (mixed solver, correction contractions of the inner iterations)",
+                        "kernel": "gemm_dual_bf16 (mixed solver, correction contractions of the inner iterations, one launch each)",
                         "kernel_ms": corr_ms, "launches": int(rmx["ops_n"][32:57].sum()),
                         "avg_launch_ms": corr_ms / max(1, int(rmx["ops_n"][32:57].sum())),
                         "work": "F_iter = 2o^2v^4 + 4o^4v^2 + 12o^3v^3 per correction evaluation"}

@@ -101,9 +101,11 @@ constexpr int kBand64 = 12, kBand128 = 8;
 //
 // What bounds it: the matrix cores, and next to them the return path of the
 // vector loads -- a 64-lane 8-byte load occupies it for 16 cycles, as long as
-// a 16-byte one (31 and 62 bytes a cycle).  So an
-// operand is staged in 16-byte pairs along its unit-stride dimension wherever
-// pairs exist (GemmProb::modes):
+// a 16-byte one (31 and 62 bytes a cycle).  In a 100-site solve the matrix cores
+// are busy 72 % of the kernel's cycles and the return path 64 % (with 8-byte
+// loads and one launch per contraction 44 to 53 % and 41 to 62 %), over 512 ragged
+// molecules 64 and 78 %.  So an operand is staged in 16-byte pairs along its
+// unit-stride dimension wherever pairs exist (GemmProb::modes):
 //   mode 0  pairs along K, staged [row][k];
 //   mode 1  pairs along the rows (columns of B), staged [k][row];
 //   mode 2  single elements, staged [k][row]: any strides.
@@ -123,7 +125,7 @@ constexpr int kBand64 = 12, kBand128 = 8;
 // Fragments are read from LDS 16 bytes at a time too: mode 0 gives a lane two
 // consecutive K, used by the two halves of an 8-deep step (the K order within
 // a step is free), modes 1 and 2 two consecutive rows, one for each of the
-// wave's two 16-row blocks.  Both layouts are free of bank conflicts.
+// wave's two 16-row blocks (bank conflicts 5 to 7 % of the cycles).
 // ---------------------------------------------------------------------------
 constexpr int kPk = kBK + 2;   // pitch of the [row][k] staging layout (16-byte aligned rows)
 
@@ -524,9 +526,9 @@ __global__ __launch_bounds__(256) void gemm_dual_f64(const GemmProb* __restrict_
 // contiguous along K 346 and 285 us for one product, 558 and 520 us for two;
 // 512 ragged molecules' 406 and 336, 439 and 362 us; solves of 2048 ragged
 // molecules 796 and 761 ms, of 120 sites 326 and 318 ms.  What remains is the
-// latency of a slab (two barriers, 16 waves a CU): matrix cores 16 %, load
-// return 70 %, LDS conflicts 20 % of the cycles, none of them full; a
-// conflict-free permuted LDS layout measured equal.
+// latency of a slab (two barriers, 12 to 16 waves a CU): of the 128 x 128 tiles'
+// cycles in a 120-site solve, matrix cores 15 %, load return 80 %, LDS conflicts
+// 18 %; a conflict-free permuted LDS layout measured equal.
 constexpr unsigned kPad = 1u << 29;   // 4 x (element index) of a padding row or K
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_h(const void* p, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, bytes, 0x00020000);

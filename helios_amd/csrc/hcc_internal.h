@@ -66,7 +66,6 @@ struct GemmProb {
   Operand A, B, C;  // A: M x K, B: K x N, C: M x N
   int M, N, K;
   double alpha, beta;
-  int tiles_n;      // tiles along N for this problem (for the table's tile size)
   int tile_begin;   // first global tile of this problem (of this part of it)
   int lt0;          // a problem spread over the XCDs: first tile of this part
   int mol;          // molecule index (for the active mask)

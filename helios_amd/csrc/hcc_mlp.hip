@@ -730,8 +730,9 @@ int hcc_mlp_create(hcc_mlp** out, int device, long capacity) {
     HCHECK(hipMemset(net->m2, 0, kMlpParams * sizeof(float)));
     dalloc(&net->rows, (size_t)capacity * kMlpRow);
     dalloc(&net->where, (size_t)capacity * 2);
-    // gradient sums of up to 16384 samples, with the trainer's other arrays: the
-    // 5 MB cost the first gradient call 0.35 ms (larger calls grow them)
+    // 256 workgroups' gradient sums, with the trainer's other arrays: enough for
+    // 16384 samples at 64 a workgroup and for 65536 at 256.  Allocated by the first
+    // gradient call, the 5 MB cost it 0.35 ms (larger calls grow them)
     const int blocks = (int)std::min<long>(256, (capacity + 63) / 64);
     ensure_part(net, blocks);
     ensure_loss(net, blocks);

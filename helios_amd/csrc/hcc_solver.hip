@@ -155,6 +155,10 @@ static int choose_tile_dual(const GemmProb& p) {
 // (the o v x 1 product).  With 16 chunks of 13500 those of 120 sites ran 600 us
 // on 16 to 48 workgroups, twice an iteration: solves with 16 work items and
 // with this rule 421 and 357 ms (mixed precision), 100 sites 181 and 173 ms.
+// The line at K = 2048 against lines at 512 and 8192 and none (twelve FP64
+// iterations): 72 sites 11.4, 11.8, 11.4 and 12.9 ms, 4 x 72 sites 33.1, 33.9,
+// 33.3 and 35.9, 100 sites 48.6, 48.6, 50.3 and 59.9; up to 40 sites, and batches of
+// 40 and 200 molecules, equal within 1 %.
 static void choose_split(GemmProb& p, int ts) {
   const int tmn = ((p.M + tile_m(ts) - 1) / tile_m(ts)) * ((p.N + tile_n(ts) - 1) / tile_n(ts));
   p.ksplit = 1;
@@ -185,12 +189,13 @@ struct DevBuf {
 // device memory of a context
 // ---------------------------------------------------------------------------
 // Blocks that a replaced batch leaves for the next one: a load of the same
-// shapes then allocates nothing (the device SCF of 1024 molecules 152 -> 52 ms;
-// what hipMalloc and hipFree of its arenas cost varies by more than that gain
-// with what else the process holds).  A load of other shapes frees blocks of at least a new block's size before it
-// allocates that one, so no more is held at any time than the larger of the two
-// batches.  The blocks not taken by the time a load ends are freed, so a context
-// holds its batch and nothing else between calls.
+// shapes then allocates nothing.  (The device SCF of 1024 molecules takes 52 to
+// 61 ms; with an allocation per arena and load it took 152 to 990 ms from run to
+// run, by what hipMalloc and hipFree cost in that process.)  A load of other
+// shapes frees blocks of at least a new block's size before it allocates that
+// one, so no more is held at any time than the larger of the two batches.  The
+// blocks not taken by the time a load ends are freed, so a context holds its
+// batch and nothing else between calls.
 struct DevBlock {
   void* p;
   size_t bytes;
@@ -480,7 +485,20 @@ static void force_split(GemmProb& p, int ks) {
 // (one or two products, layout of the operands): at 120 sites a level of
 // 380 + 557 + 316 us of correction products took 1712 us in such runs, 1246 us
 // in parts (solve 357 and 326 ms).  Fills the parts in launch order and the XCDs' ranges.
-constexpr int kSpreadMols = 16;    // more molecules: each stays on one XCD, in one L2
+//
+// Both sides of the lines, twelve iterations in ms without and with parts:
+//   mixed, 1 / 2 / 3 / 4 of 120 sites   72.3 64.5   136 128   200 193   257 259
+//   mixed, 1 / 2 / 3 / 4 of 100 sites   37.0 34.6  67.6 65.0  100 95.7  130 127
+//   mixed, 1 / 4 / 8 / 15 of 72 sites   7.80 8.14  18.7 19.7 32.0 33.5  57.0 58.4
+//   FP64, 1 / 2 / 4 of 100 sites        50.7 50.2   101 100   200 199
+//   FP64, 1 / 4 / 8 / 15 of 72 sites    10.6 11.3  32.8 33.6 56.7 57.1   102 104
+//   FP64, 2 / 5 / 8 / 15 of 48 sites    5.19 5.60  7.16 7.48 9.89 9.82  14.2 14.6
+// so parts gain for up to three molecules of 100 sites and more, and cost up to
+// 8 % of some of the smaller ones below the line; above it they lose 2 to 5 %
+// (16 and 24 molecules of 48 and 72 sites), where each molecule stays on one XCD,
+// in one L2.  With parts from 16 tiles on the same solves take 0.93 to 1.08
+// times the time, without a trend; from 256 on, 72 sites take 16.5 instead of 11.3 ms.
+constexpr int kSpreadMols = 16;
 constexpr int kSpreadTiles = 64;
 static std::vector<GemmProb> spread_parts(const std::vector<GemmProb>& probs, const std::vector<int>& tiles,
                                           const std::vector<float>& cost, std::vector<int>& ptiles,
@@ -530,10 +548,9 @@ static GemmTable build_group(Batch& b, std::vector<GemmProb> probs, int ts) {
   long ws_total = 0;
   bool large = false;
   for (GemmProb& p : probs) {
-    p.tiles_n = (p.N + tile_n(ts) - 1) / tile_n(ts);
-    const int tm = (p.M + tile_m(ts) - 1) / tile_m(ts);
+    const int tm = (p.M + tile_m(ts) - 1) / tile_m(ts), tn = (p.N + tile_n(ts) - 1) / tile_n(ts);
     p.tile_begin = t.tiles;
-    t.htiles.push_back(tm * p.tiles_n * p.ksplit);
+    t.htiles.push_back(tm * tn * p.ksplit);
     t.tiles += t.htiles.back();
     large = large || t.htiles.back() >= kSpreadTiles;
     // matrix work of a tile plus the equivalent of its set-up, first loads and stores
@@ -1692,7 +1709,7 @@ static void load(hcc_ctx* c, int nmol, const int* n, const int* nocc, const doub
     const long nn = n[k], oo = nocc[k], vv = n[k] - nocc[k];
     const long largest = std::max({vv * vv * vv * vv, oo * oo * oo * oo, nn * nn * nn, oo * oo * vv * vv, oo * vv * vv * vv});
     if (largest >= (1L << 28)) throw std::string("molecule too large: a per-molecule array exceeds 2^28 elements");
-    // the correction GEMM forms 2 x (element index) in 29 bits
+    // the correction GEMM forms 4 x (element index) below its sentinel 2^29
     if (b->mixed && largest >= (1L << 27))
       throw std::string("molecule too large for the mixed solver: a per-molecule array exceeds 2^27 elements");
     b->n.push_back(n[k]);
@@ -2100,8 +2117,8 @@ static void setup_lr(Batch& b) {
   b.lr_n2 = n2;
   b.lr_span1 = (long)(last.t1 - first.t1) + (long)last.o * last.v;
   b.lr_span2 = (long)(last.t2 - first.t2) + (long)last.o * last.o * last.v * last.v;
-  // one block for all six (256-byte aligned parts): the first product of a
-  // batch pays for these allocations
+  // one block for all six (256-byte aligned parts), allocated by the first call
+  // of a batch that needs them: hcc_lr_space, or a product without a vector space
   const long part[6] = {n1, n2, n1, n2, b.lr_span1, b.lr_span2};
   double** const at[6] = {&b.dlr_r1, &b.dlr_r2, &b.dlr_s1, &b.dlr_s2, &b.dlr_t1b, &b.dlr_t2b};
   auto up = [](long x) { return (x + 31) / 32 * 32; };
@@ -3421,12 +3438,11 @@ int hcc_selftest_gemm(int m, int n, int k, const double* A, const double* B, dou
     HCHECK(hipMemcpy(dB, B, sizeof(double) * k * n, hipMemcpyHostToDevice));
     HCHECK(hipMemcpy(dC, C, sizeof(double) * m * n, hipMemcpyHostToDevice));
     GemmProb p = prob(rm(dA, k), rm(dB, n), rm(dC, n), m, n, k, alpha, beta);
-    p.tiles_n = (n + kBN - 1) / kBN;
     p.tile_begin = 0;
     p.ksplit = 1;
     set_f64_modes(p);
     p.kchunk = p.kpad;
-    const int tiles = ((m + kBM - 1) / kBM) * p.tiles_n;
+    const int tiles = ((m + kBM - 1) / kBM) * ((n + kBN - 1) / kBN);
     HCHECK(hipMemcpy(dp, &p, sizeof(p), hipMemcpyHostToDevice));
     HCHECK(hipMalloc(&dtp, sizeof(int) * tiles));
     HCHECK(hipMemset(dtp, 0, sizeof(int) * tiles));
@@ -3487,12 +3503,11 @@ int hcc_selftest_gemm_correction(int m, int n, int k, int a_kfast, int b_nfast, 
     p.Cd = cd;
     p.hA = ha;
     p.hB = hb;
-    p.tiles_n = (n + tile - 1) / tile;
     p.tile_begin = 0;
     set_dual_modes(p, true);
     p.ksplit = 1;
     p.kchunk = p.kpad;
-    const int tiles = ((m + tile - 1) / tile) * p.tiles_n;
+    const int tiles = ((m + tile - 1) / tile) * ((n + tile - 1) / tile);
     const XcdMap xcd = xcd_runs({tiles}, {1.f});
     HCHECK(hipMalloc(&dp, sizeof(GemmProb)));
     HCHECK(hipMemcpy(dp, &p, sizeof(p), hipMemcpyHostToDevice));

@@ -77,10 +77,10 @@ __device__ double trip_block_sum(double v, double* red) {
 // orders its own read-modify-writes and the workgroup meets only between
 // pairs.  (With row tiles dealt out to all waves, each tile needed a barrier
 // between the two permutations, 30 an item at v = 24, and the matrix cores
-// were busy a third of the time: 512 ragged molecules of 10 to 48 sites took
-// 116 ms, now 90.)  v <= 16 has its own instance of 4 waves
-// whose 51 KB of LDS let three items share a CU; a single one leaves the CU
-// idle while it stages.
+// were busy 23 % of the cycles: 512 ragged molecules of 10 to 48 sites took
+// 116 ms.  Now they take 90, the matrix cores busy 34 % at v <= 24 and 28 % at
+// v <= 16.)  v <= 16 has its own instance of 4 waves whose 51 KB of LDS let three
+// items share a CU; a single one leaves the CU idle while it stages.
 typedef double trip_d4 __attribute__((ext_vector_type(4)));
 constexpr int kTripKL = kTripMaxOV / 4;        // K steps over l
 // W[a][b][c] at a S2 + b S1 + c with S1 = v + 1 and S2 = v S1 + 1 (both odd):
@@ -363,9 +363,10 @@ k_triples_mfma(const TripMol* __restrict__ mols, const int2* __restrict__ items,
 // streams from the caches straight into registers (the next x's are loaded
 // meanwhile), B operands sit in LDS.  Bound by the matrix cores in principle
 // (3072 instructions per wave and item at v = o = 32) and by those operand
-// loads: one 512-byte read per matrix instruction.  Six molecules of 54 to 64
-// sites take 19.9 ms (18 TF/s); a kernel of vector FMAs with W in global
-// memory took 275 ms.
+// loads: one 512-byte read per matrix instruction (matrix cores busy 36 % of the
+// cycles, the return path of the loads 77 %).  Six molecules of 54 to 64 sites
+// take 19.9 ms (18 TF/s); a kernel of vector FMAs with W in global memory took
+// 275 ms.
 constexpr int kTbThreads = 512;
 constexpr int kTbS1 = 17, kTbS2 = 16 * kTbS1 + 1, kTbBlk = 16 * kTbS2;   // strides and size of a 16^3 block (odd strides)
 constexpr int kTbP = 33;                                                   // pitch of the 32 x 32 operand matrices
